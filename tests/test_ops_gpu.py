@@ -89,6 +89,21 @@ def test_edge_ramp_bit_exact(n):
     assert torch.equal(gx, edge_ramp(g))
 
 
+@pytest.mark.parametrize("rows, n", [(34, 85473), (32, 64000), (34, 85489)])
+def test_edge_ramp_is_the_same_every_time(rows, n):
+    """Rows of many workgroups: 40 launches, each equal to the exact product
+    (x k/16 in float32), the tail of every row included."""
+
+    x = torch.randn(rows, n, device="cuda")
+    weight = torch.ones(n, device="cuda")
+    ramp = torch.arange(1, 16, device="cuda") / 16
+    weight[:15] *= ramp
+    weight[-15:] *= ramp.flip(0)
+    want = x * weight
+    for _ in range(40):
+        assert torch.equal(edge_ramp(x), want)
+
+
 def test_edge_ramp_needs_15_samples():
     with pytest.raises(RuntimeError):
         edge_ramp(torch.randn(2, 14, device="cuda"))

@@ -87,9 +87,14 @@ __global__ void __launch_bounds__(kEwThreads)
     const int64_t b = blockIdx.x / blocks_per_row;
     const int64_t blk = blockIdx.x - b * blocks_per_row;
     for (int64_t i = blk * kEwSpan + threadIdx.x; i < (blk + 1) * kEwSpan && i < n; i += kEwThreads) {
-        // (x * head) * tail in float32; k/16 and j k/256 are exact
-        const float head = i < 15 ? static_cast<float>(i + 1) / 16.0f : 1.0f;
-        const float tail = i >= n - 15 ? static_cast<float>(n - i) / 16.0f : 1.0f;
+        // (x * head) * tail in float32; k/16 and j k/256 are exact.  The small
+        // counts are converted as 32-bit integers: the conversion of a 64-bit
+        // one is a 64-bit shift by a vector register, whose shift count the
+        // compiler had placed in the last register allocated to the wavefront;
+        // gfx950 then took wrong counts now and then (tail weights of 1/16 or
+        // 2^16 times the right one in some launches).
+        const float head = i < 15 ? static_cast<float>(static_cast<int>(i) + 1) / 16.0f : 1.0f;
+        const float tail = i >= n - 15 ? static_cast<float>(static_cast<int>(n - i)) / 16.0f : 1.0f;
         y[b * n + i] = (x[b * n + i] * head) * tail;
     }
 }
