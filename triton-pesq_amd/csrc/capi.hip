@@ -56,25 +56,17 @@ static int fill_sections(IirTable &t, int first, const pesq_iir_sections &s, dou
         t.a1[q] = s.a1[k];
         t.a2[q] = s.a2[k];
         // chunk transfer powers: level 0 = A^kChunk, level j = A^(kChunk 2^j)
-        const double a[4] = {-s.a1[k], 1.0, -s.a2[k], 0.0};
+        const double a[4] = {-s.a1[k], -s.a2[k], 1.0, 0.0};
         double p[4] = {1.0, 0.0, 0.0, 1.0};
         for (int i = 0; i < kChunk; ++i) mat_mul(a, p, p);
         for (int level = 0; level < kLevels; ++level) {
             std::memcpy(t.pw[level][q], p, sizeof(p));
             mat_mul(p, p, p);
         }
-        // chunk end state weights: fir[i] = A^(kChunk - 1 - i) beta, beta the
-        // state increment per unit input (y = b0 x + z1 feeds back through a1, a2)
-        {
-            double g[2] = {t.b1[q] - s.a1[k] * t.b0[q], t.b2[q] - s.a2[k] * t.b0[q]};
-            for (int m = 0; m < kChunk; ++m) {
-                t.fir[q][kChunk - 1 - m][0] = g[0];
-                t.fir[q][kChunk - 1 - m][1] = g[1];
-                const double g0 = a[0] * g[0] + a[1] * g[1];
-                const double g1 = a[2] * g[0] + a[3] * g[1];
-                g[0] = g0;
-                g[1] = g1;
-            }
+        // chunk end state weights: the impulse response of 1 / (1 + a1 z^-1 + a2 z^-2)
+        for (int m = 0; m < kChunk; ++m) {
+            t.fir[q][m] = (m == 0 ? 1.0 : -s.a1[k] * t.fir[q][m - 1]) -
+                          (m >= 2 ? s.a2[k] * t.fir[q][m - 2] : 0.0);
         }
         // block pair powers M^(2 i), M = A^kSpan (level kLevelBlock)
         {

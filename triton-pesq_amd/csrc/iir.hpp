@@ -1,15 +1,17 @@
 // Chunked parallel scan of a bank of parallel second order sections, fp64 state.
 //
 // A filter is realised in parallel form, y = c0 x + sum_k y_k, where section k
-// is a direct form II transposed biquad with b2 = 0 (the form partial
-// fractions give; the table packing folds any b2 into the direct term)
-//     y_k  = b0 x + z1
-//     z1'  = b1 x - a1 y_k + z2
-//     z2'  = - a2 y_k
-// i.e. the state z = (z1, z2) evolves as z' = A_k z + beta_k x with
-// A_k = [[-a1, 1], [-a2, 0]].  Because every A_k is 2x2 and the sections are
+// is a direct form II biquad with b2 = 0 (the form partial fractions give; the
+// table packing folds any b2 into the direct term)
+//     w    = x - a1 z1 - a2 z2
+//     y_k  = b0 w + b1 z1
+//     z1', z2' = w, z1
+// i.e. the state z = (z1, z2) evolves as z' = A_k z + (x, 0) with
+// A_k = [[-a1, -a2], [1, 0]].  Because every A_k is 2x2 and the sections are
 // independent, the chunk transfer matrices are block diagonal (4 numbers per
-// section) and the scan combine costs 4 FMAs per section.
+// section) and the scan combine costs 4 FMAs per section.  A sample costs 4
+// FMAs per section, of which one (w from z1) is on the serial chain; the
+// transposed form, run before, took 5 operations with two on the chain.
 //
 // Geometry.  A lane runs the recursion of all sections over a chunk of kChunk
 // consecutive samples (the sections are independent chains, so the lane has
@@ -72,6 +74,9 @@ constexpr bool kSplitOutput = PESQ_SPLIT_OUTPUT != 0;
 #define PESQ_OUTPUT_WAVES 2
 #endif
 constexpr int kOutputWaves = PESQ_OUTPUT_WAVES;
+#ifndef PESQ_SEGMENT_MIN
+#define PESQ_SEGMENT_MIN 2
+#endif
 constexpr int kMaxSections = PESQ_IIR_MAX_SECTIONS;
 // power levels: A^(kChunk 2^j); j = 0..5 in-wave, 6 = one block, 6..11 the
 // block level scan over 64 blocks
@@ -88,10 +93,10 @@ struct IirTable {
     double a1[kMaxSections], a2[kMaxSections];
     double pw[kLevels][kMaxSections][4];     // A_k^(kChunk 2^j), row major 2x2
     double lane_pw[kMaxSections][kWave][4];  // A_k^(kChunk lane), lane start powers
-    // A_k^(kChunk - 1 - i) beta_k: the weight of the chunk's sample i in the
-    // section's state after the chunk, from a zero state (beta_k: the state
-    // increment per unit input, (b1 - a1 b0, b2 - a2 b0))
-    double fir[kMaxSections][kChunk][2];
+    // h_m, m < kChunk: the impulse response of 1 / (1 + a1 z^-1 + a2 z^-2),
+    // the weight of the sample m before the last one in z1 after the chunk
+    // from a zero state (z2 is z1 one sample earlier)
+    double fir[kMaxSections][kChunk];
     // M^(2 i), M = A_k^kSpan the block transfer: the weight of the block pair
     // (M e_j + e_j+1) 2 i + 2 blocks before a block (block_start_reduce)
     double blk_pw2[kWave][kMaxSections][4];
@@ -150,6 +155,41 @@ __host__ __device__ __forceinline__ ScanPlan scan_plan(int64_t rows, int64_t nbl
     return {lanes, lanes && nblk <= kFusedPrefixBlocks};
 }
 
+// Segments (grids that do not keep lane states, filters that decay within the
+// window).  A wavefront of the output pass runs `blocks` consecutive segment
+// blocks (64 kSegmentChunk samples, two aggregate blocks) of a row one after
+// the other, the state carried from block to block, so that only a segment's
+// first block needs a start state from before: the aggregate pass runs on the
+// two blocks before each segment instead of on every block, and the prefix
+// pass combines each pair (iir_prefix_kernel).  The count of segments per row
+// is the one whose rounds of wavefronts are shortest: `slots` wavefronts are
+// resident at a time (Mode::kSegmentSlots), and a wavefront takes its blocks
+// plus about one more for its start.
+struct SegmentPlan {
+    int count;   // segments per row (0: the scan is not segmented)
+    int blocks;  // segment blocks per segment
+};
+constexpr int kSegmentChunk = 32;                               // samples per lane
+constexpr int kSegmentSpan = kWave * kSegmentChunk;             // samples per segment block
+constexpr int kSegmentRatio = kSegmentSpan / kSpan;             // aggregate blocks in it
+static_assert(kSegmentRatio * kSpan == kSegmentSpan, "whole aggregate blocks");
+constexpr int kSegmentMin = PESQ_SEGMENT_MIN;  // blocks of a segment at least
+__host__ inline SegmentPlan segment_plan(int64_t rows, int64_t nblk, int64_t slots) {
+    if (rows <= 0 || scan_plan(rows, nblk).lane_states) return {0, 0};
+    const int64_t span = cdiv(nblk, kSegmentRatio);
+    SegmentPlan best{1, static_cast<int>(span)};
+    int64_t least = 0;
+    for (int64_t n = 1; n <= 256 && (n == 1 || n * kSegmentMin <= span); ++n) {
+        const int64_t blocks = cdiv(span, n), count = cdiv(span, blocks);
+        const int64_t cost = cdiv(rows * count, slots) * (blocks + (count > 1 ? 1 : 0));
+        if (n == 1 || cost < least) {
+            least = cost;
+            best = {static_cast<int>(count), static_cast<int>(blocks)};
+        }
+    }
+    return best;
+}
+
 // Scan workspace of `rows` rows of nblk blocks and `ns` sections: the block
 // aggregates [row][section][block][2], then, when the plan stores them, the
 // lane states [row][block][section][lane][2].
@@ -177,6 +217,10 @@ struct Bank {
     }
 };
 
+// doubles of the constant address space: uniform reads are scalar loads, also
+// after barriers and stores
+using ConstDoubles = const __attribute__((address_space(4))) double *;
+
 // Coefficients of NS sections starting at section S0.  With kB2 the sections
 // are full biquads (z2' = b2 x - a2 y_k, the cascade passes); without it b2 is
 // 0 (the parallel form, whose table packing folds b2 into the direct term).
@@ -198,27 +242,49 @@ struct Coeffs {
         c0 = direct;
     }
 
+    __device__ __forceinline__ void load_scalar(const IirTable &t, const double &direct) {
+        const ConstDoubles tb0 = (ConstDoubles)t.b0, tb1 = (ConstDoubles)t.b1;
+        const ConstDoubles ta1 = (ConstDoubles)t.a1, ta2 = (ConstDoubles)t.a2;
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            b0[k] = tb0[S0 + k];
+            b1[k] = tb1[S0 + k];
+            b2[k] = 0.0;
+            a1[k] = ta1[S0 + k];
+            a2[k] = ta2[S0 + k];
+        }
+        c0 = *(ConstDoubles)&direct;
+    }
+    // one section's step: its output added to y
+    __device__ __forceinline__ double section(int k, Bank<NS> &s, double x, double y) const {
+        const double w = fma(-a1[k], s.u[k], fma(-a2[k], s.v[k], x));
+        double out = fma(b1[k], s.u[k], y);
+        if constexpr (kB2) out = fma(b2[k], s.v[k], out);
+        out = fma(b0[k], w, out);
+        s.v[k] = s.u[k];
+        s.u[k] = w;
+        return out;
+    }
     // one time step: consumes x, advances the state, returns c0 x + sum_k y_k
     __device__ __forceinline__ double step(Bank<NS> &s, double x) const {
         double y = c0 * x;
 #pragma unroll
-        for (int k = 0; k < NS; ++k) {
-            const double yk = fma(b0[k], x, s.u[k]);
-            s.u[k] = fma(-a1[k], yk, fma(b1[k], x, s.v[k]));
-            s.v[k] = kB2 ? fma(b2[k], x, -a2[k] * yk) : -a2[k] * yk;
-            y += yk;
-        }
+        for (int k = 0; k < NS; ++k) y = section(k, s, x, y);
         return y;
     }
     // the same step, each section's output kept apart (y[k] = y_k)
     __device__ __forceinline__ void step_parts(Bank<NS> &s, double x,
                                                double (&y)[NS > 0 ? NS : 1]) const {
 #pragma unroll
+        for (int k = 0; k < NS; ++k) y[k] = section(k, s, x, 0.0);
+    }
+    // the states alone
+    __device__ __forceinline__ void advance(Bank<NS> &s, double x) const {
+#pragma unroll
         for (int k = 0; k < NS; ++k) {
-            const double yk = fma(b0[k], x, s.u[k]);
-            s.u[k] = fma(-a1[k], yk, fma(b1[k], x, s.v[k]));
-            s.v[k] = kB2 ? fma(b2[k], x, -a2[k] * yk) : -a2[k] * yk;
-            y[k] = yk;
+            const double w = fma(-a1[k], s.u[k], fma(-a2[k], s.v[k], x));
+            s.v[k] = s.u[k];
+            s.u[k] = w;
         }
     }
 };
@@ -462,6 +528,8 @@ struct BankPair {
 //   Mode::kB2                     full biquad sections (b2 read from the table)
 //   Mode::kReverse                process the time axis back to front
 //   Mode::kAccumulates            the output pass reduces a per block sum
+//   Mode::kSegments               large grids may run segmented (SegmentPlan),
+//                                 Mode::kSegmentSlots wavefronts at a time
 //   Mode::kRamp                   the Mode uses the edge ramp weight w of the
 //                                 sample (edge_weight(n, len)); otherwise the
 //                                 kernels pass w = 1
@@ -478,9 +546,8 @@ struct BankPair {
 // constants are applied by compute.
 //
 // Memory access: a lane reads and writes its kChunk consecutive samples as
-// 16-byte vectors when the row's alignment allows it (the whole wavefront
-// then covers kSpan contiguous samples per instruction group), else element
-// by element; the last chunk of a row is handled element by element.
+// 16-byte vectors (the whole wavefront covers kSpan contiguous samples per
+// instruction group); the last chunk of a row is handled element by element.
 // --------------------------------------------------------------------------
 
 // physical index of the first sample of a full chunk starting at time j0
@@ -489,29 +556,24 @@ __device__ __forceinline__ int64_t chunk_lo(int64_t j0, int64_t len) {
     return kRev ? len - j0 - kChunk : j0;
 }
 
-// 16-byte vector moves of float (4 per vector) and double (2 per vector)
-__device__ __forceinline__ void load16(const float *p, float *dst) {
-    const float4 w = *reinterpret_cast<const float4 *>(p);
-    dst[0] = w.x;
-    dst[1] = w.y;
-    dst[2] = w.z;
-    dst[3] = w.w;
+// 16-byte vector moves of float (4 per vector) and double (2 per vector), at
+// the alignment of the element (global_load/store_dwordx4 need no more than 4
+// bytes): rows of odd lengths start at any element, and an element by element
+// chunk is 16 loads or stores that touch 64 cache lines each (48 rows of 84754
+// samples: forward scans 59 -> 35 us, backward output pass 30 -> 22 us; 8 biquads
+// over 24 rows of 160001 samples, forward and adjoint, 568 -> 445 us)
+template <typename T>
+__device__ __forceinline__ void load16(const T *p, T *dst) {
+    __builtin_memcpy(dst, p, 16);
 }
-__device__ __forceinline__ void load16(const double *p, double *dst) {
-    const double2 w = *reinterpret_cast<const double2 *>(p);
-    dst[0] = w.x;
-    dst[1] = w.y;
-}
-__device__ __forceinline__ void store16(float *p, const float *src) {
-    *reinterpret_cast<float4 *>(p) = make_float4(src[0], src[1], src[2], src[3]);
-}
-__device__ __forceinline__ void store16(double *p, const double *src) {
-    *reinterpret_cast<double2 *>(p) = make_double2(src[0], src[1]);
+template <typename T>
+__device__ __forceinline__ void store16(T *p, const T *src) {
+    __builtin_memcpy(p, src, 16);
 }
 
-// One path for all inputs (16-byte vectors when every input's chunk is full
-// and aligned, else elements), so that the loads of all inputs are issued
-// before the first wait for one of them.
+// One path for all inputs (16-byte vectors when the chunk is full, else
+// elements), so that the loads of all inputs are issued before the first wait
+// for one of them.
 template <class Mode>
 __device__ __forceinline__ void load_chunk(const Mode &m, int row, int64_t j0, int64_t len,
                                            typename Mode::In (&in)[kChunk][Mode::kInputs]) {
@@ -519,12 +581,7 @@ __device__ __forceinline__ void load_chunk(const Mode &m, int row, int64_t j0, i
     constexpr int kVec = 16 / sizeof(T);
     const bool full = j0 + kChunk <= len;
     const int64_t lo = chunk_lo<Mode::kReverse>(j0, len);
-    bool vec = full;
-#pragma unroll
-    for (int q = 0; q < Mode::kInputs; ++q) {
-        vec = vec && (reinterpret_cast<uintptr_t>(m.src(row, q) + lo) & 15) == 0;
-    }
-    if (vec) {
+    if (full) {
         T buf[Mode::kInputs][kChunk];
 #pragma unroll
         for (int q = 0; q < Mode::kInputs; ++q) {
@@ -559,7 +616,7 @@ __device__ __forceinline__ void store_chunk(T *base, const T (&out)[kChunk], boo
     constexpr int kVec = 16 / sizeof(T);
     const bool full = j0 + kChunk <= len;
     const int64_t lo = kRev ? len - j0 - kChunk : j0;
-    if (full && (reinterpret_cast<uintptr_t>(base + lo) & 15) == 0) {
+    if (full) {
         T e[kChunk];
 #pragma unroll
         for (int i = 0; i < kChunk; ++i) e[i] = out[kRev ? kChunk - 1 - i : i];
@@ -598,19 +655,21 @@ __device__ __forceinline__ void element_inputs(const Mode &m,
 }
 
 // state of NS sections from S0 after the chunk, from a zero state, as the
-// weighted sums of the chunk's inputs x[0 .. kChunk - 1]: kChunk independent
-// fused multiply-adds per state component instead of the recursion's chain
+// weighted sums of the chunk's inputs x[0 .. kChunk - 1]: independent fused
+// multiply-adds instead of the recursion's chain (z2 has the weights of z1 one
+// sample later; the weight of the last sample, h_0, is 1)
 template <int S0, int NS>
 __device__ __forceinline__ void chunk_end_state(const IirTable &t, const double (&x)[kChunk],
                                                 Bank<NS> &s) {
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
-        double u = t.fir[S0 + k][0][0] * x[0];
-        double v = t.fir[S0 + k][0][1] * x[0];
+        double u = x[kChunk - 1];
+        double v = x[kChunk - 2];
 #pragma unroll
-        for (int i = 1; i < kChunk; ++i) {
-            u = fma(t.fir[S0 + k][i][0], x[i], u);
-            v = fma(t.fir[S0 + k][i][1], x[i], v);
+        for (int m = 1; m < kChunk; ++m) {
+            const double h = t.fir[S0 + k][m];
+            u = fma(h, x[kChunk - 1 - m], u);
+            if (m < kChunk - 1) v = fma(h, x[kChunk - 2 - m], v);
         }
         s.u[k] = u;
         s.v[k] = v;
@@ -636,8 +695,8 @@ __device__ __forceinline__ void zero_run(const Mode &m, const IirTable &t,
         for (int i = 0; i < kChunk; ++i) {
             double w, xa, xb;
             element_inputs<kGeneral>(m, in[i], j0 + i, len, w, xa, xb);
-            if constexpr (NA > 0) ca.step(s.a, xa);
-            if constexpr (NB > 0) cb.step(s.b, xb);
+            if constexpr (NA > 0) ca.advance(s.a, xa);
+            if constexpr (NB > 0) cb.advance(s.b, xb);
         }
     } else {
         double xa[kChunk], xb[kChunk];
@@ -758,11 +817,19 @@ __device__ __forceinline__ void aggregate_block(const Mode &m, const IirTable &t
 template <int NA, int NB, class Mode, bool kLaneStates, int kBase = 0, int kLayout = NA + NB>
 __global__ void __launch_bounds__(kWave)
     iir_aggregate_kernel(Mode m, const IirTable *__restrict__ table, double *__restrict__ aggr,
-                         double *__restrict__ lanes, int64_t len, int nblk) {
+                         double *__restrict__ lanes, int64_t len, int nblk, SegmentPlan seg) {
     const IirTable &t = *table;
-    const int row = blockIdx.x / nblk;
-    const int blk = blockIdx.x - row * nblk;
     const int lane = threadIdx.x;
+    // segmented scans: the two blocks before segments 1 .. count - 1 of a row,
+    // their aggregates at 2 segment and 2 segment + 1 of 2 count
+    const int per_row = seg.count > 0 ? kWarmBlocks * (seg.count - 1) : nblk;
+    const int slots = seg.count > 0 ? kWarmBlocks * seg.count : nblk;
+    const int row = blockIdx.x / per_row;
+    const int idx = blockIdx.x - row * per_row;
+    const int slot = seg.count > 0 ? idx + kWarmBlocks : idx;
+    const int blk = seg.count > 0 ? (idx / kWarmBlocks + 1) * seg.blocks * kSegmentRatio - kWarmBlocks +
+                                      idx % kWarmBlocks
+                                : idx;
     if constexpr (kLaneStates) {
         aggregate_block<NA, NB, kBase, kLayout>(m, t, aggr, lanes, len, nblk, row, blk, lane);
     } else {
@@ -782,7 +849,7 @@ __global__ void __launch_bounds__(kWave)
         } else {
             zero_run<false, true>(m, t, ca, cb, in, j0, len, s);
         }
-        block_end_state<NS>(t, s, aggr + (int64_t(row) * NS * nblk + blk) * 2, nblk, lane);
+        block_end_state<NS>(t, s, aggr + (int64_t(row) * NS * slots + slot) * 2, slots, lane);
     }
 }
 
@@ -847,7 +914,7 @@ __device__ __forceinline__ Mat2 mat2_mul(const Mat2 &x, const Mat2 &y) {
 template <int NS>
 __global__ void __launch_bounds__(kWave *kPrefixWaves)
     iir_prefix_kernel(const IirTable *__restrict__ table, double *__restrict__ aggr, int nblk,
-                      int64_t nseq) {
+                      int64_t nseq, SegmentPlan seg) {
     const IirTable &t = *table;
     const int64_t seq = int64_t(blockIdx.x) * kPrefixWaves +
                         __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
@@ -857,6 +924,20 @@ __global__ void __launch_bounds__(kWave *kPrefixWaves)
     double2 *agg = reinterpret_cast<double2 *>(aggr + seq * nblk * 2);
     const double *pm = t.pw[kLevelBlock][k];
     const Mat2 m{pm[0], pm[1], pm[2], pm[3]};
+    if (seg.count > 0) {
+        // windowed segment starts: e_(b-1) + M e_(b-2) over the pair's first entry
+        agg = reinterpret_cast<double2 *>(aggr) + seq * seg.count * kWarmBlocks;
+        for (int i = lane; i < seg.count; i += kWave) {
+            double2 start = make_double2(0.0, 0.0);
+            if (i > 0) {
+                const double2 e0 = agg[kWarmBlocks * i], e1 = agg[kWarmBlocks * i + 1];
+                start.x = fma(m.a, e0.x, fma(m.b, e0.y, e1.x));
+                start.y = fma(m.c, e0.x, fma(m.d, e0.y, e1.y));
+            }
+            agg[kWarmBlocks * i] = start;
+        }
+        return;
+    }
     const int per = (nblk + kWave - 1) / kWave;
     const int j0 = lane * per;
     const int j1 = j0 + per < nblk ? j0 + per : nblk;
@@ -928,12 +1009,374 @@ __global__ void __launch_bounds__(kWave *kPrefixWaves)
     }
 }
 
+// --------------------------------------------------------------------------
+// A segment of the output pass by one wavefront (SegmentPlan).
+//
+// A lane runs kChunk consecutive samples, so its own 16-byte loads and stores
+// are 64 bytes apart and each instruction touches 64 cache lines: with the per
+// lane powers of the scan and of the block start, read through the same path,
+// the address processing of a CU cost as much as its arithmetic.  Here a block
+// moves between memory and LDS in rows of 1 KB (16 bytes per lane,
+// contiguous), the next block's loads going out before this one runs, and the
+// lanes read their samples from padded chunks in LDS (kStageChunk: the lanes
+// of an LDS cycle on distinct banks), four at a time, and leave their outputs
+// there; so few registers are live that three wavefronts fit on a SIMD.  The
+// powers of the scan's row carries come from LDS too, staged once per
+// workgroup; the block's start state enters the scan through lane 0, so that
+// no per lane power is applied to it, and the state of the last lane is the
+// next block's start.  The chunk end states come from the recursion, 2 FMAs
+// per section and sample, and not as weighted sums, whose weights would be
+// read from memory for every block.
+//
+// Issue bound: 1040 VALU instructions per 1024 samples and filter pair (1310
+// with 16 samples per lane, whose scan is half as long per sample; the
+// unsegmented passes, aggregate and output, took about 1700), 80 % of the
+// kernel's time forward with three wavefronts per SIMD, 58 % backward with the
+// two that its LDS allows (16 samples per lane and three wavefronts were no
+// faster).  512 rows of 64000 samples: forward scans 173 -> 115 us, backward
+// 117 -> 83 us, the training step at 256 x 4 s, 48 kHz 706 -> 633 us; 74 rows of
+// 116961: 57 -> 51 us.
+// --------------------------------------------------------------------------
+constexpr int kSegmentWaves = 4;             // wavefronts (segments) per workgroup
+constexpr int kStageChunk = kSegmentChunk + 4;  // floats between the staged chunks of two lanes
+constexpr int kStageFloats = kWave * kStageChunk;
+constexpr int kCarryPowers = kWave / 2 + 1;  // A^(kSegmentChunk m), m <= 32
+template <int NS>
+constexpr int carry_stride() { return 4 * NS + 2; }  // doubles between two powers m
+
+// first sample of block blk in memory, and whether the row holds all of it
+template <bool kRev>
+__device__ __forceinline__ int64_t segment_lo(int blk, int64_t len) {
+    return kRev ? len - int64_t(blk + 1) * kSegmentSpan : int64_t(blk) * kSegmentSpan;
+}
+__device__ __forceinline__ bool segment_full(int64_t lo, int64_t len) {
+    return lo >= 0 && lo + kSegmentSpan <= len;
+}
+// word of the stage that holds sample i (memory order) of a block
+__device__ __forceinline__ int stage_word(int i) {
+    return i / kSegmentChunk * kStageChunk + i % kSegmentChunk;
+}
+
+// four floats, in LDS (16-byte aligned) and in a row (at any element)
+using Vec4 = float __attribute__((ext_vector_type(4)));
+using Vec4Row = float __attribute__((ext_vector_type(4), aligned(4)));
+
+// a full block of one raw input in memory order, 16 bytes per lane and r
+__device__ __forceinline__ void segment_load(const float *src, int lane, Vec4 (&v)[kSegmentChunk / 4]) {
+#pragma unroll
+    for (int r = 0; r < kSegmentChunk / 4; ++r) {
+        v[r] = *reinterpret_cast<const Vec4Row *>(src + 4 * (lane + kWave * r));
+    }
+}
+// a block into the stage: from the registers a full one was loaded into, else
+// from the row itself, zero outside it
+__device__ __forceinline__ void stage_in(float *stage, const Vec4 (&v)[kSegmentChunk / 4],
+                                         const float *base, int64_t lo, int64_t len, int lane) {
+    if (segment_full(lo, len)) {
+#pragma unroll
+        for (int r = 0; r < kSegmentChunk / 4; ++r) {
+            *reinterpret_cast<Vec4 *>(stage + stage_word(4 * (lane + kWave * r))) = v[r];
+        }
+    } else {
+#pragma unroll 1
+        for (int i = lane; i < kSegmentSpan; i += kWave) {
+            const int64_t n = lo + i;
+            const float w = base[n < 0 ? 0 : (n < len ? n : len - 1)];
+            stage[stage_word(i)] = n >= 0 && n < len ? w : 0.0f;
+        }
+    }
+}
+__device__ __forceinline__ void stage_out(float *base, const float *stage, int64_t lo, int64_t len,
+                                          int lane) {
+    if (segment_full(lo, len)) {
+        float *dst = base + lo;
+#pragma unroll
+        for (int r = 0; r < kSegmentChunk / 4; ++r) {
+            const int i = 4 * (lane + kWave * r);
+            *reinterpret_cast<Vec4Row *>(dst + i) =
+                *reinterpret_cast<const Vec4 *>(stage + stage_word(i));
+        }
+    } else {
+#pragma unroll 1
+        for (int i = lane; i < kSegmentSpan; i += kWave) {
+            const int64_t n = lo + i;
+            if (n >= 0 && n < len) base[n] = stage[stage_word(i)];
+        }
+    }
+}
+
+// samples 4 g .. 4 g + 3 (time order) of a lane's staged chunk
+template <bool kRev>
+__device__ __forceinline__ void chunk_read(const float *own, int g, float (&x)[4]) {
+    const float4 w = *reinterpret_cast<const float4 *>(own + (kRev ? kSegmentChunk - 4 - 4 * g : 4 * g));
+    x[kRev ? 3 : 0] = w.x;
+    x[kRev ? 2 : 1] = w.y;
+    x[kRev ? 1 : 2] = w.z;
+    x[kRev ? 0 : 3] = w.w;
+}
+template <bool kRev>
+__device__ __forceinline__ void chunk_write(float *own, int g, const float (&y)[4]) {
+    *reinterpret_cast<float4 *>(own + (kRev ? kSegmentChunk - 4 - 4 * g : 4 * g)) =
+        make_float4(y[kRev ? 3 : 0], y[kRev ? 2 : 1], y[kRev ? 1 : 2], y[kRev ? 0 : 3]);
+}
+
+// A^(kSegmentChunk 2^level)
+static_assert(kSegmentChunk == 2 * kChunk, "one level above the aggregate pass's chunks");
+__device__ __forceinline__ ConstDoubles scan_powers(ConstDoubles pw, int level, int k) {
+    return pw + ((level + 1) * kMaxSections + k) * 4;
+}
+
+// One block of a segment: own[q] the lane's staged chunk of buffer q (raw
+// input q, replaced by output q), p the block's start state (in lane 0),
+// replaced by the next block's.  before / after: samples of the row before
+// the lane's chunk and from its first sample to the row's end, at most 64
+// (ramp weights).  kEdge: the block holds samples with a ramp weight, or the
+// row's end.
+template <bool kEdge, int NA, int NB, class Mode>
+__device__ __forceinline__ void segment_block(const Mode &m, ConstDoubles pw,
+                                              const Coeffs<0, NA> &ca, const Coeffs<NA, NB> &cb,
+                                              const double *carry, float *own, float *second,
+                                              int before, int after, const double *sh, int lane,
+                                              Bank<NA + NB> &p, double &acc) {
+    constexpr int NS = NA + NB;
+    constexpr bool kRev = Mode::kReverse;
+    auto weight = [&](int j) -> double {  // edge_weight of chunk sample j
+        if constexpr (!kEdge || !Mode::kRamp) return 1.0;
+        const int head = before + j + 1 < 16 ? before + j + 1 : 16;
+        const int tail = after - j < 16 ? (after - j > 0 ? after - j : 0) : 16;
+        const int first = kRev ? tail : head, last = kRev ? head : tail;
+        return static_cast<double>(first) * 0.0625 * (static_cast<double>(last) * 0.0625);
+    };
+    auto group = [&](int g, float (&x)[Mode::kInputs][4]) {
+#pragma unroll
+        for (int q = 0; q < Mode::kInputs; ++q) chunk_read<kRev>(own + q * kStageFloats, g, x[q]);
+    };
+    // chunk end states from a zero state
+    BankPair<NA, NB> z;
+    z.zero();
+#pragma unroll 1
+    for (int g = 0; g < kSegmentChunk / 4; ++g) {
+        float x[Mode::kInputs][4];
+        group(g, x);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float in[Mode::kInputs];
+            double xa, xb;
+#pragma unroll
+            for (int q = 0; q < Mode::kInputs; ++q) in[q] = x[q][i];
+            m.inputs(weight(4 * g + i), in, xa, xb);
+            ca.advance(z.a, xa);
+            cb.advance(z.b, xb);
+        }
+    }
+    // the block's start state enters lane 0's chunk, then an inclusive scan
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const double fu = lane == 0 ? p.u[k] : 0.0, fv = lane == 0 ? p.v[k] : 0.0;
+        const ConstDoubles q = scan_powers(pw, 0, k);
+        z.u(k) = fma(q[0], fu, fma(q[1], fv, z.u(k)));
+        z.v(k) = fma(q[2], fu, fma(q[3], fv, z.v(k)));
+    }
+    using std::integral_constant;
+    auto level = [&](auto ctrl, int j) {
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            const ConstDoubles q = scan_powers(pw, j, k);
+            const double ou = dpp_move<decltype(ctrl)::value, 0xF>(z.u(k));
+            const double ov = dpp_move<decltype(ctrl)::value, 0xF>(z.v(k));
+            z.u(k) = fma(q[0], ou, fma(q[1], ov, z.u(k)));
+            z.v(k) = fma(q[2], ou, fma(q[3], ov, z.v(k)));
+        }
+    };
+    level(integral_constant<int, 0x111>{}, 0);
+    level(integral_constant<int, 0x112>{}, 1);
+    level(integral_constant<int, 0x114>{}, 2);
+    level(integral_constant<int, 0x118>{}, 3);
+    auto carry_level = [&](auto ctrl, auto mask, int power) {
+        int at = power * carry_stride<NS>();
+        asm volatile("" : "+v"(at));  // one address, immediate offsets from it
+        const double *c = carry + at;
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            const double2 q0 = *reinterpret_cast<const double2 *>(c + 4 * k);
+            const double2 q1 = *reinterpret_cast<const double2 *>(c + 4 * k + 2);
+            const double ou = dpp_move<decltype(ctrl)::value, decltype(mask)::value>(z.u(k));
+            const double ov = dpp_move<decltype(ctrl)::value, decltype(mask)::value>(z.v(k));
+            z.u(k) = fma(q0.x, ou, fma(q0.y, ov, z.u(k)));
+            z.v(k) = fma(q1.x, ou, fma(q1.y, ov, z.v(k)));
+        }
+    };
+    carry_level(integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{}, (lane & 15) + 1);
+    carry_level(integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{},
+                lane >= 32 ? lane - 31 : 0);
+    // every lane's start state: the lane before it (rotated: lane 0 receives
+    // lane 63, the next block's start), lane 0's the block's start
+    BankPair<NA, NB> s;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const double ru = dpp_move<0x13C, 0xF>(z.u(k)), rv = dpp_move<0x13C, 0xF>(z.v(k));
+        s.u(k) = lane == 0 ? p.u[k] : ru;
+        s.v(k) = lane == 0 ? p.v[k] : rv;
+        p.u[k] = ru;
+        p.v[k] = rv;
+    }
+#pragma unroll 1
+    for (int g = 0; g < kSegmentChunk / 4; ++g) {
+        float x[Mode::kInputs][4], y[Mode::kOutputs][4];
+        group(g, x);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const double w = weight(4 * g + i);
+            float in[Mode::kInputs], o[Mode::kOutputs];
+            double xa, xb;
+#pragma unroll
+            for (int q = 0; q < Mode::kInputs; ++q) in[q] = x[q][i];
+            m.inputs(w, in, xa, xb);
+            const double ya = ca.step(s.a, xa), yb = cb.step(s.b, xb);
+            const double was = acc;
+            m.compute(w, ya, yb, acc, sh, o);
+            if constexpr (kEdge) {
+                if (4 * g + i >= after) acc = was;  // past the end of the row
+            }
+#pragma unroll
+            for (int q = 0; q < Mode::kOutputs; ++q) y[q][i] = o[q];
+        }
+        chunk_write<kRev>(own, g, y[0]);
+        if constexpr (Mode::kOutputs > 1) {
+            if (second != nullptr) {
+                if constexpr (!kEdge) {
+                    const Vec4 v = {y[1][0], y[1][1], y[1][2], y[1][3]};
+                    *reinterpret_cast<Vec4Row *>(second + 4 * g) = v;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        if (4 * g + i < after) second[4 * g + i] = y[1][i];
+                    }
+                }
+            }
+        }
+    }
+}
+
+template <int NA, int NB, class Mode>
+__device__ __forceinline__ void output_segment(const Mode &m, const IirTable &t,
+                                               const double *aggr, int64_t len, int nblk,
+                                               const SegmentPlan &seg, int64_t nseg) {
+    constexpr int NS = NA + NB;
+    constexpr bool kRev = Mode::kReverse;
+    static_assert(!Mode::kB2 && std::is_same<typename Mode::In, float>::value &&
+                      std::is_same<typename Mode::Out, float>::value,
+                  "float rows, parallel form");
+    __shared__ __attribute__((aligned(16))) float stages[kSegmentWaves][Mode::kInputs * kStageFloats];
+    __shared__ __attribute__((aligned(16))) double carry[kCarryPowers * carry_stride<NS>()];
+    const int wave = wave_index();
+    const int lane = static_cast<int>(threadIdx.x) % kWave;
+    const int64_t id = int64_t(blockIdx.x) * kSegmentWaves + wave;
+    const bool live = id < nseg;  // (the last workgroup: whole wavefronts past the end)
+    const int row = live ? static_cast<int>(id / seg.count) : 0;
+    const int index = live ? static_cast<int>(id - int64_t(row) * seg.count) : 0;
+    const int b0 = index * seg.blocks;
+    const int span = (nblk + kSegmentRatio - 1) / kSegmentRatio;
+    const int b1 = b0 + seg.blocks < span ? b0 + seg.blocks : span;
+    float *stage = stages[wave];
+    float *own = stage + (kRev ? kWave - 1 - lane : lane) * kStageChunk;
+    Vec4 next[Mode::kInputs][kSegmentChunk / 4];
+    auto request = [&](int blk) {
+        const int64_t lo = segment_lo<kRev>(blk, len);
+        if (segment_full(lo, len)) {
+#pragma unroll
+            for (int q = 0; q < Mode::kInputs; ++q) segment_load(m.src(row, q) + lo, lane, next[q]);
+        }
+    };
+    request(b0);
+    Bank<NS> p;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const double *src =
+            aggr + ((int64_t(row) * NS + k) * seg.count + index) * (2 * kWarmBlocks);
+        p.u[k] = index > 0 ? src[0] : 0.0;
+        p.v[k] = index > 0 ? src[1] : 0.0;
+    }
+    // the scan's uniform powers, read by scalar loads for every block: into the L2
+    {
+        const double2 touch = *reinterpret_cast<const double2 *>(&t.pw[1][0][0] + 2 * lane);
+        static_assert(4 * kMaxSections * 4 >= 2 * kWave, "levels 1 .. 4");
+        asm volatile("" ::"v"(touch.x), "v"(touch.y));
+    }
+    for (int i = threadIdx.x; i < kCarryPowers * NS; i += kSegmentWaves * kWave) {
+        const int power = i / NS, k = i - power * NS;
+        double *dst = carry + power * carry_stride<NS>() + 4 * k;
+        // A^(kSegmentChunk power), power 32 = one aggregate block
+        const double *src = power < kWave / 2 ? t.lane_pw[k][2 * power] : t.pw[kLevelBlock][k];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dst[e] = src[e];
+    }
+    __syncthreads();
+    if (!live) return;
+    double sh[4];
+    if constexpr (HasPre<Mode>::value) {
+        typename Mode::Pre pre;
+        m.prefetch(row, lane, pre);
+        m.setup(row, sh, lane, pre);
+    } else {
+        m.setup(row, sh, lane);
+    }
+    static_assert(Mode::kOutputs == 1 || !kRev, "a second output is written in time order");
+    float *second = Mode::kOutputs > 1 ? m.dst(row, Mode::kOutputs - 1) : nullptr;
+    Coeffs<0, NA> ca;
+    Coeffs<NA, NB> cb;
+    ca.load_scalar(t, t.c0a);
+    cb.load_scalar(t, t.c0b);
+#pragma unroll 1
+    for (int blk = b0; blk < b1; ++blk) {
+        const int64_t lo = segment_lo<kRev>(blk, len);
+#pragma unroll
+        for (int q = 0; q < Mode::kInputs; ++q) {
+            stage_in(stage + q * kStageFloats, next[q], m.src(row, q), lo, len, lane);
+        }
+        wave_lds_fence();
+        if (blk + 1 < b1) request(blk + 1);
+        // the scan's uniform powers are read again for every block (scalar loads):
+        // hoisted out of the loop they would fill the vector registers
+        ConstDoubles pw = (ConstDoubles)(&t.pw[0][0][0]);
+        asm volatile("" : "+s"(pw));
+        double acc = 0.0;
+        const int64_t j0 = int64_t(blk) * kSegmentSpan + int64_t(lane) * kSegmentChunk;
+        float *out2 = second != nullptr ? second + j0 : nullptr;
+        // uniform: ramp weights and row ends only in a row's first and last blocks
+        if (blk == 0 || int64_t(blk + 1) * kSegmentSpan + kEdge > len) {
+            const int before = static_cast<int>(j0 < kWave ? j0 : kWave);
+            const int64_t rest = len - j0;
+            const int after = static_cast<int>(rest < 0 ? 0 : (rest < kWave ? rest : kWave));
+            segment_block<true, NA, NB>(m, pw, ca, cb, carry, own, out2, before, after, sh, lane,
+                                        p, acc);
+        } else {
+            segment_block<false, NA, NB>(m, pw, ca, cb, carry, own, out2, 0, 0, sh, lane, p, acc);
+        }
+        wave_lds_fence();
+        stage_out(m.dst(row, 0), stage, lo, len, lane);
+        wave_lds_fence();
+        if constexpr (Mode::kAccumulates) {
+            acc = wave_sum(acc);
+            // (one sum per segment block: in its first aggregate block's place)
+            if (lane < kSegmentRatio && blk * kSegmentRatio + lane < nblk) {
+                m.finish(row, blk * kSegmentRatio + lane, lane == 0 ? acc : 0.0);
+            }
+        }
+    }
+}
+
 template <int NA, int NB, class Mode, bool kLaneStates, int kPrefix, bool kWarmB = false>
-__global__ void __launch_bounds__(kWave)
+__global__ void __launch_bounds__(Mode::kSegments && !kLaneStates ? kSegmentWaves *kWave : kWave,
+                                  Mode::kSegments && !kLaneStates ? 3 : 1)
     iir_output_kernel(Mode m, const IirTable *__restrict__ table,
                       const double *__restrict__ aggr, const double *__restrict__ lanes,
-                      int64_t len, int nblk) {
+                      int64_t len, int nblk, SegmentPlan seg, int64_t rows) {
     constexpr int NS = NA + NB;
+    if constexpr (Mode::kSegments && !kLaneStates) {
+        output_segment<NA, NB>(m, *table, aggr, len, nblk, seg, rows * seg.count);
+        return;
+    }
     static_assert(kLaneStates || kPrefix == kStoredStarts,
                   "grids that recompute the lane states take stored block starts");
     static_assert(!kWarmB || (kLaneStates && kPrefix != kStoredStarts && NB == 1),
@@ -1422,6 +1865,10 @@ int launch_scan(const Mode &m, const IirTable *table, double *ws, int64_t rows, 
     if (grid == 0) return PESQ_OK;
     const ScanPlan plan = scan_plan(rows, nblk);
     const bool lane_states = plan.lane_states;
+    SegmentPlan seg{0, 0};
+    if constexpr (Mode::kSegments) {
+        if (window) seg = segment_plan(rows, nblk, Mode::kSegmentSlots);
+    }
     const bool windowed = window && lane_states;
     const bool fused = !windowed && plan.fused_prefix;
     PESQ_CHECK_ARG(!warm_b || (NB == 1 && Mode::kInputs == 2 && (windowed || fused)),
@@ -1439,19 +1886,22 @@ int launch_scan(const Mode &m, const IirTable *table, double *ws, int64_t rows, 
         if (launched) {
         } else if (lane_states) {
             hipLaunchKernelGGL((iir_aggregate_kernel<NA, NB, Mode, true>), dim3(grid), dim3(kWave),
-                               0, stream, m, table, aggr, lanes, len, static_cast<int>(nblk));
-        } else {
-            hipLaunchKernelGGL((iir_aggregate_kernel<NA, NB, Mode, false>), dim3(grid),
+                               0, stream, m, table, aggr, lanes, len, static_cast<int>(nblk), seg);
+        } else if (seg.count != 1) {
+            // (a row of one segment starts from zero: nothing to aggregate)
+            const unsigned blocks =
+                seg.count > 0 ? static_cast<unsigned>(rows * kWarmBlocks * (seg.count - 1)) : grid;
+            hipLaunchKernelGGL((iir_aggregate_kernel<NA, NB, Mode, false>), dim3(blocks),
                                dim3(kWave), 0, stream, m, table, aggr, lanes, len,
-                               static_cast<int>(nblk));
+                               static_cast<int>(nblk), seg);
         }
         PESQ_CHECK_LAUNCH("iir aggregate");
-        if (!fused && !windowed) {
+        if (!fused && !windowed && seg.count != 1) {
             const int64_t nseq = rows * NS;
             hipLaunchKernelGGL(iir_prefix_kernel<NS>,
                                dim3(static_cast<unsigned>(cdiv(nseq, kPrefixWaves))),
                                dim3(kWave * kPrefixWaves), 0, stream, table, aggr,
-                               static_cast<int>(nblk), nseq);
+                               static_cast<int>(nblk), nseq, seg);
             PESQ_CHECK_LAUNCH("iir prefix");
         }
     }
@@ -1474,27 +1924,30 @@ int launch_scan(const Mode &m, const IirTable *table, double *ws, int64_t rows, 
             if (launched) {
             } else if (windowed && warm_b) {
                 hipLaunchKernelGGL((iir_output_kernel<NA, NB, Mode, true, kWindowStarts, true>),
-                                   dim3(grid), dim3(kWave), 0, stream, m, table, ca, cl, len, nb);
+                                   dim3(grid), dim3(kWave), 0, stream, m, table, ca, cl, len, nb, seg, rows);
                 launched = true;
             } else if (fused && warm_b) {
                 hipLaunchKernelGGL((iir_output_kernel<NA, NB, Mode, true, kFusedSums, true>),
-                                   dim3(grid), dim3(kWave), 0, stream, m, table, ca, cl, len, nb);
+                                   dim3(grid), dim3(kWave), 0, stream, m, table, ca, cl, len, nb, seg, rows);
                 launched = true;
             }
         }
         if (launched) {
         } else if (windowed) {
             hipLaunchKernelGGL((iir_output_kernel<NA, NB, Mode, true, kWindowStarts>),
-                               dim3(grid), dim3(kWave), 0, stream, m, table, ca, cl, len, nb);
+                               dim3(grid), dim3(kWave), 0, stream, m, table, ca, cl, len, nb, seg, rows);
         } else if (fused) {
             hipLaunchKernelGGL((iir_output_kernel<NA, NB, Mode, true, kFusedSums>), dim3(grid),
-                               dim3(kWave), 0, stream, m, table, ca, cl, len, nb);
+                               dim3(kWave), 0, stream, m, table, ca, cl, len, nb, seg, rows);
         } else if (lane_states) {
             hipLaunchKernelGGL((iir_output_kernel<NA, NB, Mode, true, kStoredStarts>),
-                               dim3(grid), dim3(kWave), 0, stream, m, table, ca, cl, len, nb);
+                               dim3(grid), dim3(kWave), 0, stream, m, table, ca, cl, len, nb, seg, rows);
         } else {
+            const unsigned groups =
+                seg.count > 0 ? static_cast<unsigned>(cdiv(rows * seg.count, kSegmentWaves)) : grid;
             hipLaunchKernelGGL((iir_output_kernel<NA, NB, Mode, false, kStoredStarts>),
-                               dim3(grid), dim3(kWave), 0, stream, m, table, ca, cl, len, nb);
+                               dim3(groups), dim3(seg.count > 0 ? kSegmentWaves * kWave : kWave), 0,
+                               stream, m, table, ca, cl, len, nb, seg, rows);
         }
         PESQ_CHECK_LAUNCH("iir output");
     }

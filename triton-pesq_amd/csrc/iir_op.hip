@@ -12,6 +12,7 @@ struct SingleMode {
     static constexpr bool kRamp = false;
     static constexpr bool kReverse = kRev;
     static constexpr bool kAccumulates = false;
+    static constexpr bool kSegments = false;
     static constexpr bool kB2 = false;
     using In = float;
     using Out = float;
@@ -69,6 +70,7 @@ struct CascadeMode {
     static constexpr bool kRamp = false;
     static constexpr bool kReverse = kRev;
     static constexpr bool kAccumulates = false;
+    static constexpr bool kSegments = false;
     static constexpr bool kB2 = true;
     using In = TIn;
     using Out = TOut;

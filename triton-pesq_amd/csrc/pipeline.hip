@@ -50,6 +50,8 @@ struct PipeFwdMode {
     static constexpr bool kRamp = true;
     static constexpr bool kReverse = false;
     static constexpr bool kAccumulates = true;
+    static constexpr bool kSegments = true;
+    static constexpr int64_t kSegmentSlots = 3 * 1024;  // by registers and LDS (44 KB per 4)
     static constexpr bool kB2 = false;
     using In = float;
     using Out = float;
@@ -93,6 +95,8 @@ struct PipeBwdMode {
     static constexpr bool kRamp = true;
     static constexpr bool kReverse = true;
     static constexpr bool kAccumulates = false;
+    static constexpr bool kSegments = true;
+    static constexpr int64_t kSegmentSlots = 2 * 1024;  // by LDS (81 KB per 4 wavefronts)
     static constexpr bool kB2 = false;
     using In = float;
     using Out = float;
@@ -177,6 +181,7 @@ struct PipeBwdPowerMode {
     static constexpr bool kRamp = false;
     static constexpr bool kReverse = true;
     static constexpr bool kAccumulates = false;
+    static constexpr bool kSegments = false;
     static constexpr bool kB2 = false;
     using In = float;
     using Out = float;
@@ -1677,6 +1682,7 @@ using StftBwdReal = float;
 // asks about are the ones that run.
 struct PipePlan {
     ScanPlan fwd_scan, bwd_scan;
+    SegmentPlan fwd_seg, bwd_seg;
     bool stft_lean;      // stft_fwd_kernel<.., true>: grids above kWideTiles
     int chain_fwd_waves, chain_bwd_waves;
     int chain_bpl;       // bands per lane: 1 up to 64 bands, 2 up to 128
@@ -1686,6 +1692,10 @@ static PipePlan pipe_plan(const PipeLayout &L) {
     PipePlan P{};
     P.fwd_scan = scan_plan(L.rows, L.nblk);
     P.bwd_scan = scan_plan(L.nrg, L.nblk);
+    if (kPipeWindow) {
+        P.fwd_seg = segment_plan(L.rows, L.nblk, PipeFwdMode::kSegmentSlots);
+        P.bwd_seg = segment_plan(L.nrg, L.nblk, PipeBwdMode::kSegmentSlots);
+    }
     const int64_t grid = L.batch * L.ntile;
     const bool wide = grid > kWideTiles;
     P.stft_lean = wide;
@@ -1728,8 +1738,8 @@ constexpr bool kSplitAggregate = PESQ_SPLIT_AGGREGATE != 0;
 
 // Names of the kernels of one scan pass, in launch order (host_power: the
 // backward scan is its output launch alone).
-static void scan_kernel_names(const ScanPlan &S, const char *mode, std::string &out,
-                              bool host_power = false) {
+static void scan_kernel_names(const ScanPlan &S, const SegmentPlan &seg, const char *mode,
+                              std::string &out, bool host_power = false) {
     const char *lanes = S.lane_states ? "true" : "false";
     const int prefix = kPipeWindow && S.lane_states
                            ? kWindowStarts
@@ -1746,10 +1756,10 @@ static void scan_kernel_names(const ScanPlan &S, const char *mode, std::string &
     } else if (kSplitAggregate && S.lane_states) {
         out += "iir_aggregate_split_kernel<5, 1, " + std::to_string(kSplitWaves) + ", " + mode +
                ">;";
-    } else {
+    } else if (seg.count != 1) {  // (rows of one segment start from zero)
         out += std::string("iir_aggregate_kernel<5, 1, ") + mode + ", " + lanes + ", 0, 6>;";
     }
-    if (prefix == kStoredStarts) out += "iir_prefix_kernel<6>;";
+    if (prefix == kStoredStarts && seg.count != 1) out += "iir_prefix_kernel<6>;";
     out += output + "false>;";
 }
 
@@ -1809,7 +1819,7 @@ extern "C" int pesq_pipeline_kernels(int64_t batch, int64_t len, int grad_mask, 
     const char *bwd_real = std::is_same<StftBwdReal, double>::value ? "double" : "float";
     std::string out;
     if (!backward) {
-        scan_kernel_names(P.fwd_scan, "PipeFwdMode", out);
+        scan_kernel_names(P.fwd_scan, P.fwd_seg, "PipeFwdMode", out);
         out += std::string("stft_fwd_kernel<") + real + ", " + (P.stft_lean ? "true" : "false") +
                ", " + std::to_string(kStftWaves) + ">;";
         if (L.totals) out += "band_totals_kernel<" + std::to_string(kChainSlices) + ", 2>;";
@@ -1822,7 +1832,7 @@ extern "C" int pesq_pipeline_kernels(int64_t batch, int64_t len, int grad_mask, 
         if (L.totals) out += "band_totals_kernel<" + std::to_string(kGradSlices) + ", 1>;";
         out += std::string("stft_bwd_kernel<") + bwd_real + ", " + std::to_string(L.bwd_fpw) +
                ", " + std::to_string(L.bwd_waves) + ">;";
-        scan_kernel_names(P.bwd_scan, "PipeBwdMode", out, L.host_power);
+        scan_kernel_names(P.bwd_scan, P.bwd_seg, "PipeBwdMode", out, L.host_power);
     }
     out.pop_back();  // the last ';'
     if (needed != nullptr) *needed = out.size() + 1;
