@@ -230,14 +230,15 @@ int pesq_iir_workspace(int64_t rows, int64_t len, size_t *bytes);
 int pesq_iir_apply(const float *x, float *y, int64_t rows, int64_t len, const void *iir_table,
                    int sections, int reverse, void *workspace, hipStream_t stream);
 
-/* Workspace of pesq_iir_cascade_apply: the scan workspace plus up to two
- * float64 [rows, len] intermediate signals. */
+/* Workspace of pesq_iir_cascade_apply: covers the block states of two and more
+ * sections and the scan workspace of one (its size is that of a scan per
+ * section with two float64 [rows, len] signals in between). */
 int pesq_iir_cascade_workspace(int64_t rows, int64_t len, int sections, size_t *bytes);
 
 /* y = lfilter(x) through a packed cascade of `sections` biquads (TritonIIR
- * forward / _IIRFunction, iir.py:1232-1258,1451-1482): one scan pass per
- * section with float64 state, float64 signals between the passes; reverse
- * != 0 applies the adjoint (every pass time reversed). */
+ * forward / _IIRFunction, iir.py:1232-1258,1451-1482): all sections in one
+ * pass over blocks of the rows, float64 states and signals in registers;
+ * reverse != 0 applies the adjoint (time reversed). */
 int pesq_iir_cascade_apply(const float *x, float *y, int64_t rows, int64_t len,
                            const void *cascade_tables, int sections, int reverse,
                            void *workspace, hipStream_t stream);

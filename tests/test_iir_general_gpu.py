@@ -237,3 +237,30 @@ def test_cascade_is_deterministic_and_row_independent():
     assert torch.equal(mod(x), mod(x))
     assert torch.equal(mod(x)[3:4], mod(x[3:4]))
     assert torch.equal(mod(x[:, ::2]), mod(x[:, ::2].contiguous()))
+
+
+@pytest.mark.parametrize("sections", [2, 8, 32])
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 4096, 6151, 20481])
+def test_cascade_block_edges_for_any_section_count(sections, n):
+    """The one pass cascade at the edges of its 2048 sample blocks (one block
+    needs no start states), rows at odd offsets, both directions, the fewest
+    and the most sections: well damped biquads against ``sosfilt`` in float64,
+    to the float32 rounding of the output (6e-8 of the peak, 2e-7 allowed)."""
+
+    from scipy.signal import sosfilt
+
+    from torch_pesq.hip_ops import iir as iir_ops
+
+    rng = np.random.default_rng(sections)
+    radius, angle = rng.uniform(0.3, 0.95, sections), rng.uniform(0.2, 2.9, sections)
+    sos = np.ones((sections, 6))
+    sos[:, 1:3] = np.stack([rng.uniform(-0.3, 0.3, sections), rng.uniform(-0.2, 0.2, sections)], 1)
+    sos[:, 4:] = np.stack([-2 * radius * np.cos(angle), radius**2], 1)
+    sos[:, :3] *= ((1 - radius) * 0.9)[:, None]
+    table = iir_ops._pack_cascade(sos).cuda()
+    x = noise(5, n, seed=n)
+    for reverse in (False, True):
+        got = iir_ops._launch(torch.from_numpy(x).float().cuda(), table, "cascade", sections, reverse)
+        x64 = x.astype(np.float32).astype(np.float64)
+        want = sosfilt(sos, x64[:, ::-1] if reverse else x64)
+        assert peak_error(got, want[:, ::-1] if reverse else want) < 2e-7

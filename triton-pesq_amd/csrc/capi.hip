@@ -2,6 +2,7 @@
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
+#include <vector>
 
 #include "tables.hpp"
 
@@ -88,6 +89,40 @@ static int fill_sections(IirTable &t, int first, const pesq_iir_sections &s, dou
     return PESQ_OK;
 }
 
+// T of a cascade (IirTable::cascade): the matrix of one step without input,
+// column by column, squared log2(kSegmentSpan) times in extended precision
+static void cascade_transfer(IirTable *tables, int sections) {
+    const int n = 2 * sections;
+    std::vector<long double> m(size_t(n) * n), sq(size_t(n) * n);
+    for (int j = 0; j < n; ++j) {
+        long double x = 0.0L;
+        for (int k = 0; k < sections; ++k) {
+            const IirTable &t = tables[k];
+            const long double u = j == 2 * k ? 1.0L : 0.0L, v = j == 2 * k + 1 ? 1.0L : 0.0L;
+            const long double w = x - t.a1[0] * u - t.a2[0] * v;
+            m[size_t(2 * k) * n + j] = w;
+            m[size_t(2 * k + 1) * n + j] = u;
+            x = t.b0[0] * w + t.b1[0] * u + t.b2[0] * v;
+        }
+    }
+    for (int span = 1; span < kSegmentSpan; span *= 2) {
+        for (int i = 0; i < n; ++i) {
+            for (int j = 0; j < n; ++j) {
+                long double acc = 0.0L;
+                // (a section's states depend on the sections up to it)
+                for (int l = j / 2 * 2; l <= (i | 1); ++l) acc += m[size_t(i) * n + l] * m[size_t(l) * n + j];
+                sq[size_t(i) * n + j] = acc;
+            }
+        }
+        m.swap(sq);
+    }
+    for (int i = 0; i < n; ++i) {
+        for (int j = 0; j < n; ++j) {
+            tables[i / 2].cascade[i % 2][j] = static_cast<double>(m[size_t(i) * n + j]);
+        }
+    }
+}
+
 static int pack_iir(IirTable &t, const pesq_iir_sections *a, const pesq_iir_sections *b) {
     std::memset(&t, 0, sizeof(t));
     PESQ_CHECK_ARG(a != nullptr, "null filter");
@@ -142,6 +177,7 @@ extern "C" int pesq_iir_cascade_pack(const double *sos, int sections, void *out)
         if (int st = fill_sections(t, 0, one, t.c0a, false)) return st;
         std::memcpy(&tables[k], &t, sizeof(t));
     }
+    cascade_transfer(tables, sections);
     return PESQ_OK;
 }
 

@@ -1,6 +1,6 @@
 // Stand-alone IIR filter (the TritonIIR operator), forward or time reversed:
 // one filter in parallel form (one scan pass), or a cascade of full biquads
-// (one scan pass per section, float64 rows between the passes).
+// (all sections in one pass, iir_cascade_kernel).
 #include "iir.hpp"
 
 namespace pesq {
@@ -60,11 +60,9 @@ static int dispatch(int sections, const float *x, float *y, int64_t rows, int64_
     return PESQ_ERR_ARGUMENT;
 }
 
-// One pass of a cascade: a full biquad (b2 kept) from In to Out.  Passes
-// between the first and the last read and write float64 rows, so that the
-// cascade rounds to float32 only once, at its output.
-template <bool kRev, typename TIn, typename TOut>
-struct CascadeMode {
+// A cascade of one section: a full biquad (b2 kept) through the scan kernels.
+template <bool kRev>
+struct BiquadMode {
     static constexpr int kInputs = 1;
     static constexpr int kOutputs = 1;
     static constexpr bool kRamp = false;
@@ -72,48 +70,270 @@ struct CascadeMode {
     static constexpr bool kAccumulates = false;
     static constexpr bool kSegments = false;
     static constexpr bool kB2 = true;
-    using In = TIn;
-    using Out = TOut;
+    using In = float;
+    using Out = float;
 
-    const TIn *x;
-    TOut *y;
+    const float *x;
+    float *y;
     int64_t len;
 
-    __device__ __forceinline__ const TIn *src(int row, int) const { return x + int64_t(row) * len; }
-    __device__ __forceinline__ TOut *dst(int row, int) const { return y + int64_t(row) * len; }
-    __device__ __forceinline__ void inputs(double, const TIn *in, double &xa, double &xb) const {
+    __device__ __forceinline__ const float *src(int row, int) const { return x + int64_t(row) * len; }
+    __device__ __forceinline__ float *dst(int row, int) const { return y + int64_t(row) * len; }
+    __device__ __forceinline__ void inputs(double, const float *in, double &xa, double &xb) const {
         xa = static_cast<double>(in[0]);
         xb = 0.0;
     }
     __device__ __forceinline__ void setup(int, double *, int) const {}
     __device__ __forceinline__ void compute(double, double ya, double, double &, const double *,
-                                            TOut *out) const {
-        out[0] = static_cast<TOut>(ya);
+                                            float *out) const {
+        out[0] = static_cast<float>(ya);
     }
     __device__ __forceinline__ void finish(int, int, double) const {}
 };
 
-template <bool kRev, typename TIn, typename TOut>
-static int cascade_pass(const TIn *x, TOut *y, int64_t rows, int64_t len, const IirTable *table,
-                        double *aggr, hipStream_t stream) {
-    CascadeMode<kRev, TIn, TOut> m{x, y, len};
-    return launch_scan<1, 0>(m, table, aggr, rows, len, true, true, stream);
+// --------------------------------------------------------------------------
+// Cascades of two and more biquads.
+//
+// A wavefront holds a block of kSegmentSpan samples of a row, 32 per lane as
+// doubles, and runs the sections over it one after the other: each section's
+// chunk end states (2 FMAs per sample), their scan over the lanes and the
+// recursion (5 FMAs per sample), whose outputs are the next section's inputs,
+// so no signal between the sections leaves the registers.  A block's start
+// states (two per section) depend on the row's earlier blocks through all
+// sections before them, so rows of more than one block take three launches:
+// the blocks run from zero states (kOutput false) to their end states, one
+// wavefront per row carries these over the row (s_(b+1) = T s_b + e_b, T the
+// cascade's transfer over a block), and the blocks run again from their true
+// starts.  The blocks of a row do not depend on the other rows: a row's result
+// is the same in any batch.
+//
+// Bound by issue and the sections' serial chains: about 330 VALU instructions
+// per section and 2048 samples, in both block passes.  One scan pass per
+// section, with float64 signals through memory between them, took 445
+// us for 8 sections over 24 rows of 160001 samples, forward and adjoint; this
+// form takes 121 us (states 16, starts 16, output 22 us per direction).
+// --------------------------------------------------------------------------
+struct CascadeArgs {
+    const float *x;
+    float *y;
+    const IirTable *tables;
+    double *states;  // [rows][blocks][2 sections]: end states of the block before, then starts
+    int64_t rows, len;
+    int sections, blocks;
+};
+
+template <bool kRev, bool kOutput>
+__global__ void __launch_bounds__(kSegmentWaves *kWave, 3) iir_cascade_kernel(CascadeArgs a) {
+    extern __shared__ double powers[];  // [section][kCarryPowers][4]: A^(kSegmentChunk m)
+    __shared__ __attribute__((aligned(16))) float stages[kSegmentWaves][kStageFloats];
+    const int wave = wave_index();
+    const int lane = static_cast<int>(threadIdx.x) % kWave;
+    // the states pass has nothing to do for a row's last block
+    const int per_row = kOutput ? a.blocks : a.blocks - 1;
+    const int64_t id = int64_t(blockIdx.x) * kSegmentWaves + wave;
+    const bool live = id < a.rows * per_row;
+    const int64_t row = live ? id / per_row : 0;
+    const int blk = live ? static_cast<int>(id - row * per_row) : 0;
+    const float *src = a.x + row * a.len;
+    const int64_t lo = segment_lo<kRev>(blk, a.len);
+    Vec4 raw[kSegmentChunk / 4];
+    if (segment_full(lo, a.len)) segment_load(src + lo, lane, raw);
+    for (int i = threadIdx.x; i < a.sections * kCarryPowers; i += kSegmentWaves * kWave) {
+        const int k = i / kCarryPowers, power = i - k * kCarryPowers;
+        const IirTable &t = a.tables[k];
+        const double *p = power < kWave / 2 ? t.lane_pw[0][2 * power] : t.pw[kLevelBlock][0];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) powers[4 * i + e] = p[e];
+    }
+    __syncthreads();
+    if (!live) return;  // whole wavefronts; no barrier follows
+    float *stage = stages[wave];
+    float *own = stage + (kRev ? kWave - 1 - lane : lane) * kStageChunk;
+    stage_in(stage, raw, src, lo, a.len, lane);
+    wave_lds_fence();
+    double y[kSegmentChunk];
+#pragma unroll
+    for (int g = 0; g < kSegmentChunk / 4; ++g) {
+        float v[4];
+        chunk_read<kRev>(own, g, v);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[4 * g + i] = static_cast<double>(v[i]);
+    }
+    double *states = a.states + (row * a.blocks + blk) * 2 * a.sections;
+    const double *c5 = powers + 4 * ((lane & 15) + 1);
+    const double *c6 = powers + 4 * (lane >= 32 ? lane - 31 : 0);
+#pragma unroll 1
+    for (int k = 0; k < a.sections; ++k) {
+        const ConstDoubles pw = (ConstDoubles)(&a.tables[k].pw[0][0][0]);
+        Coeffs<0, 1, true> c;
+        {
+            const IirTable &t = a.tables[k];
+            c.b0[0] = *(ConstDoubles)t.b0;
+            c.b1[0] = *(ConstDoubles)t.b1;
+            c.b2[0] = *(ConstDoubles)t.b2;
+            c.a1[0] = *(ConstDoubles)t.a1;
+            c.a2[0] = *(ConstDoubles)t.a2;
+            c.c0 = 0.0;
+        }
+        Bank<1> z;
+        z.zero();
+#pragma unroll
+        for (int i = 0; i < kSegmentChunk; ++i) c.advance(z, y[i]);
+        double pu = 0.0, pv = 0.0;  // the block's start state
+        if constexpr (kOutput) {
+            if (blk > 0) {
+                pu = states[2 * k];
+                pv = states[2 * k + 1];
+            }
+            const ConstDoubles q = scan_powers(pw, 0, 0);
+            const double fu = lane == 0 ? pu : 0.0, fv = lane == 0 ? pv : 0.0;
+            z.u[0] = fma(q[0], fu, fma(q[1], fv, z.u[0]));
+            z.v[0] = fma(q[2], fu, fma(q[3], fv, z.v[0]));
+        }
+        using std::integral_constant;
+        auto level = [&](auto ctrl, int j) {
+            const ConstDoubles q = scan_powers(pw, j, 0);
+            const double ou = dpp_move<decltype(ctrl)::value, 0xF>(z.u[0]);
+            const double ov = dpp_move<decltype(ctrl)::value, 0xF>(z.v[0]);
+            z.u[0] = fma(q[0], ou, fma(q[1], ov, z.u[0]));
+            z.v[0] = fma(q[2], ou, fma(q[3], ov, z.v[0]));
+        };
+        level(integral_constant<int, 0x111>{}, 0);
+        level(integral_constant<int, 0x112>{}, 1);
+        level(integral_constant<int, 0x114>{}, 2);
+        level(integral_constant<int, 0x118>{}, 3);
+        auto carry_level = [&](auto ctrl, auto mask, const double *p) {
+            const double2 q0 = *reinterpret_cast<const double2 *>(p + 4 * kCarryPowers * k);
+            const double2 q1 = *reinterpret_cast<const double2 *>(p + 4 * kCarryPowers * k + 2);
+            const double ou = dpp_move<decltype(ctrl)::value, decltype(mask)::value>(z.u[0]);
+            const double ov = dpp_move<decltype(ctrl)::value, decltype(mask)::value>(z.v[0]);
+            z.u[0] = fma(q0.x, ou, fma(q0.y, ov, z.u[0]));
+            z.v[0] = fma(q1.x, ou, fma(q1.y, ov, z.v[0]));
+        };
+        carry_level(integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{}, c5);
+        carry_level(integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{}, c6);
+        if constexpr (!kOutput) {
+            // the block's end state, where the next block's start will stand
+            if (lane == kWave - 1) {
+                states[2 * a.sections + 2 * k] = z.u[0];
+                states[2 * a.sections + 2 * k + 1] = z.v[0];
+            }
+            if (k + 1 == a.sections) return;
+        }
+        Bank<1> s;
+        const double before_u = dpp_move<0x138, 0xF>(z.u[0]);  // wave_shr:1, all lanes active
+        const double before_v = dpp_move<0x138, 0xF>(z.v[0]);
+        s.u[0] = lane == 0 ? pu : before_u;
+        s.v[0] = lane == 0 ? pv : before_v;
+#pragma unroll
+        for (int i = 0; i < kSegmentChunk; ++i) y[i] = c.section(0, s, y[i], 0.0);
+    }
+    if constexpr (kOutput) {
+#pragma unroll
+        for (int g = 0; g < kSegmentChunk / 4; ++g) {
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = static_cast<float>(y[4 * g + i]);
+            chunk_write<kRev>(own, g, v);
+        }
+        wave_lds_fence();
+        stage_out(a.y + row * a.len, stage, lo, a.len, lane);
+    }
 }
 
-// passes k = 0 .. count - 1: float x -> double rows (alternating buffers) -> float y
+// Start states of a row's blocks from the end states of the blocks before
+// them, in place, one wavefront per row: lane i holds row i of T (kN >= 2
+// sections columns, zero past them) and state i; the current start state is
+// passed through LDS, every lane reading all of it.  The end states of
+// kStartsAhead blocks are loaded while the ones before them are carried (a load
+// per block, one block ahead, waited out the memory latency at each block: 46
+// us instead of 16 for 79 blocks of 8 sections).
+constexpr int kStartsAhead = 8;
+
+template <int kN>
+__global__ void __launch_bounds__(kWave) iir_cascade_starts_kernel(CascadeArgs a) {
+    __shared__ __attribute__((aligned(16))) double state[kN > kWave ? kN : kWave];
+    const int n = 2 * a.sections;
+    const int lane = threadIdx.x;
+    const int mine = lane < n ? lane : 0;
+    double t[kN];
+#pragma unroll
+    for (int j = 0; j < kN; ++j) {
+        const double v = a.tables[mine / 2].cascade[mine % 2][j];
+        t[j] = lane < n && j < n ? v : 0.0;
+    }
+    state[lane] = 0.0;
+    wave_lds_fence();
+    double *row = a.states + int64_t(blockIdx.x) * a.blocks * n + mine;
+    auto load = [&](int b0, double (&e)[kStartsAhead]) {
+#pragma unroll
+        for (int q = 0; q < kStartsAhead; ++q) {
+            const int b = b0 + q < a.blocks ? b0 + q : a.blocks - 1;
+            e[q] = row[int64_t(b) * n];
+        }
+    };
+    double e[kStartsAhead], next[kStartsAhead];
+    load(1, e);
+    for (int b0 = 1; b0 < a.blocks; b0 += kStartsAhead) {
+        load(b0 + kStartsAhead, next);
+#pragma unroll
+        for (int q = 0; q < kStartsAhead; ++q) {
+            if (b0 + q < a.blocks) {  // uniform
+                double acc[4] = {e[q], 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int j = 0; j < kN; j += 2) {
+                    const double2 s = *reinterpret_cast<const double2 *>(state + j);
+                    acc[j % 4] = fma(t[j], s.x, acc[j % 4]);
+                    acc[j % 4 + 1] = fma(t[j + 1], s.y, acc[j % 4 + 1]);
+                }
+                wave_lds_fence();
+                const double v = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+                state[lane] = lane < n ? v : 0.0;
+                wave_lds_fence();
+                if (lane < n) row[int64_t(b0 + q) * n] = v;
+            }
+            e[q] = next[q];
+        }
+    }
+}
+
 template <bool kRev>
 static int cascade(const float *x, float *y, int64_t rows, int64_t len, const IirTable *tables,
-                   int count, double *aggr, double *mid, hipStream_t stream) {
-    if (count == 1) return cascade_pass<kRev>(x, y, rows, len, tables, aggr, stream);
-    double *buf[2] = {mid, mid + rows * len};
-    if (int st = cascade_pass<kRev>(x, buf[0], rows, len, tables, aggr, stream)) return st;
-    for (int k = 1; k < count - 1; ++k) {
-        const int st = cascade_pass<kRev>(static_cast<const double *>(buf[(k - 1) & 1]),
-                                          buf[k & 1], rows, len, tables + k, aggr, stream);
-        if (st) return st;
+                   int count, double *workspace, hipStream_t stream) {
+    if (count == 1) {
+        BiquadMode<kRev> m{x, y, len};
+        return launch_scan<1, 0>(m, tables, workspace, rows, len, true, true, stream);
     }
-    return cascade_pass<kRev>(static_cast<const double *>(buf[(count - 2) & 1]), y, rows, len,
-                              tables + count - 1, aggr, stream);
+    CascadeArgs a{x, y, tables, workspace, rows, len, count,
+                  static_cast<int>(cdiv(len, kSegmentSpan))};
+    const size_t lds = size_t(count) * kCarryPowers * 4 * sizeof(double);
+    const dim3 block(kSegmentWaves * kWave);
+    auto groups = [&](int64_t per_row) {
+        return dim3(static_cast<unsigned>(cdiv(rows * per_row, kSegmentWaves)));
+    };
+    if (a.blocks > 1) {
+        hipLaunchKernelGGL((iir_cascade_kernel<kRev, false>), groups(a.blocks - 1), block, lds,
+                           stream, a);
+        PESQ_CHECK_LAUNCH("iir cascade states");
+        const dim3 grid(static_cast<unsigned>(rows)), wave(kWave);
+        if (count <= 4) {
+            hipLaunchKernelGGL(iir_cascade_starts_kernel<8>, grid, wave, 0, stream, a);
+        } else if (count <= 8) {
+            hipLaunchKernelGGL(iir_cascade_starts_kernel<16>, grid, wave, 0, stream, a);
+        } else {
+            hipLaunchKernelGGL(iir_cascade_starts_kernel<64>, grid, wave, 0, stream, a);
+        }
+        PESQ_CHECK_LAUNCH("iir cascade starts");
+    }
+    hipLaunchKernelGGL((iir_cascade_kernel<kRev, true>), groups(a.blocks), block, lds, stream, a);
+    PESQ_CHECK_LAUNCH("iir cascade output");
+    return PESQ_OK;
+}
+
+// doubles of the workspace that hold the states
+static int64_t cascade_state_doubles(int64_t rows, int64_t len, int sections) {
+    const int64_t blocks = cdiv(len, kSegmentSpan);
+    return sections > 1 && blocks > 1 ? rows * blocks * 2 * sections : 0;
 }
 
 }  // namespace pesq
@@ -128,7 +348,9 @@ extern "C" int pesq_iir_cascade_workspace(int64_t rows, int64_t len, int section
     const int64_t nblk = cdiv(len, kBlockSpan);
     PESQ_CHECK_ARG(rows * nblk < (int64_t(1) << 31), "too many rows x blocks for one launch");
     const int64_t mid = sections == 1 ? 0 : (sections == 2 ? 1 : 2) * rows * len;
-    *bytes = size_t(scan_workspace_doubles(rows, nblk, 1) + mid) * sizeof(double);
+    const int64_t size = scan_workspace_doubles(rows, nblk, 1) + mid;
+    const int64_t states = cascade_state_doubles(rows, len, sections);
+    *bytes = size_t(size > states ? size : states) * sizeof(double);
     return PESQ_OK;
 }
 
@@ -143,10 +365,9 @@ extern "C" int pesq_iir_cascade_apply(const float *x, float *y, int64_t rows, in
     const int64_t nblk = cdiv(len, kBlockSpan);
     PESQ_CHECK_ARG(rows * nblk < (int64_t(1) << 31), "too many rows x blocks for one launch");
     const IirTable *tables = static_cast<const IirTable *>(cascade_tables);
-    double *aggr = static_cast<double *>(workspace);
-    double *mid = aggr + scan_workspace_doubles(rows, nblk, 1);
-    return reverse ? cascade<true>(x, y, rows, len, tables, sections, aggr, mid, stream)
-                   : cascade<false>(x, y, rows, len, tables, sections, aggr, mid, stream);
+    double *ws = static_cast<double *>(workspace);
+    return reverse ? cascade<true>(x, y, rows, len, tables, sections, ws, stream)
+                   : cascade<false>(x, y, rows, len, tables, sections, ws, stream);
 }
 
 extern "C" int pesq_iir_workspace(int64_t rows, int64_t len, size_t *bytes) {

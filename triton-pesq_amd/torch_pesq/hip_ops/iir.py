@@ -16,12 +16,12 @@ itself (``scipy.signal.lfilter`` in float64), the *fidelity*:
     The sections are independent, so all of them run in one scan pass.  It
     does not exist for repeated poles and loses digits for clustered ones.
 ``cascade``
-    the series of biquads of ``scipy.signal.tf2sos``, one scan pass per
-    section with float64 signals between the passes.  It handles repeated
-    poles, zero poles and numerators longer than the denominator.
+    the series of biquads of ``scipy.signal.tf2sos``, run section after section
+    over blocks held in registers as float64.  It handles repeated poles, zero
+    poles and numerators longer than the denominator.
 
-The parallel form is used whenever its fidelity is within 1e-9 (one pass
-instead of one per section), otherwise the realisation with the better
+The parallel form is used whenever its fidelity is within 1e-9 (the blocks
+run once instead of twice), otherwise the realisation with the better
 fidelity.  Order <= 2 filters are a single full biquad.  The score is rated
 with the reference's limits (``iir.py:38-58``, :func:`_state_space`
 ``iir.py:599-666``): above ``1e5 * 2^-24`` the filter is rejected with a
