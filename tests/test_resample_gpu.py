@@ -277,3 +277,37 @@ def test_moved_after_construction():
         mod(x)
     mod = mod.cuda()
     assert _close(mod(x), O.resample(x.double().cpu(), 48000, 16000))
+
+
+@pytest.mark.parametrize("orig,new", [(8000, 16000), (16000, 48000), (16000, 64000), (8000, 48000)])
+@pytest.mark.parametrize("length", [1, 3, 13, 2047, 2048, 2049, 4109])
+def test_integer_upsampling(orig, new, length):
+    """Upsampling by 2, 3, 4 and 6: the register windows of the forward (all
+    phases of 8 input positions per thread, tiles of 2048 positions) and of the
+    adjoint (a decimation over the transposed bank).  The forward is the
+    untiled kernel's sum in the same order, so the same numbers; the adjoint
+    is held to the float64 one."""
+
+    from torch_pesq import _lib
+
+    mod = HipResample(orig, new).cuda()
+    x = torch.randn(3, length, generator=torch.Generator().manual_seed(length)).cuda()
+    leaf = x.clone().requires_grad_(True)
+    got = mod(leaf)
+    want = torch.empty_like(got)
+    lib = _lib.library()
+    _lib.check(
+        lib.pesq_resample_forward(
+            _lib.ptr(x), _lib.ptr(want), 3, length, got.shape[1], _lib.ptr(mod.kernel),
+            _lib.ptr(mod.tap_lo), _lib.ptr(mod.tap_hi), mod.orig_step, mod.new_step, mod.width,
+            mod.kernel.shape[1], _lib.stream_handle(x.device),
+        ),
+        "pesq_resample_forward",
+    )
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    g = torch.randn(got.shape, generator=torch.Generator().manual_seed(1)).cuda()
+    (gx,) = torch.autograd.grad(got, leaf, g)
+    ref = x.double().cpu().requires_grad_(True)
+    (want_gx,) = torch.autograd.grad(O.resample(ref, orig, new), ref, g.double().cpu())
+    assert _close(gx, want_gx)
