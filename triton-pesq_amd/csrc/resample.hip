@@ -495,14 +495,11 @@ constexpr int kWinOut = 8;  // outputs per thread
 __host__ __device__ constexpr int fwd_window_batch4(int orig) { return 2 * orig + 1; }
 constexpr int kMaxWindowLds = 65536;  // bytes of LDS a window kernel may stage
 
-// (T: the taps' type in memory, float for the transposed bank of an integer
-// upsampling, whose adjoint is such a decimation: 24 rows of 84754 gradient
-// samples, 1:2, 20 -> 9.9 us against the tiled kernel.)
-template <int kOrig, typename T = double>
-__global__ void __launch_bounds__(kResampleThreads)
-    resample_fwd_window(InRows x, OutRows y, int64_t n_in,
-                        int64_t n_out, const T *__restrict__ taps64, int ntaps, int off_min,
-                        int span, int64_t blocks_per_row) {
+// (T: the taps' type in memory.)
+template <int kOrig, typename T>
+__device__ __forceinline__ void fwd_window(const InRows &x, const OutRows &y, int64_t n_in,
+                                           int64_t n_out, const T *__restrict__ taps64, int ntaps,
+                                           int off_min, int span, int64_t blocks_per_row) {
     constexpr int kR = kWinOut;
     constexpr int kTile = kResampleThreads * kR;
     constexpr int kStride = kR * kOrig;  // staged samples between the windows of two lanes
@@ -576,6 +573,25 @@ __global__ void __launch_bounds__(kResampleThreads)
             if (m + r < n_out) yr[m + r] = res[r];
         }
     }
+}
+
+template <int kOrig>
+__global__ void __launch_bounds__(kResampleThreads)
+    resample_fwd_window(InRows x, OutRows y, int64_t n_in, int64_t n_out,
+                        const double *__restrict__ taps64, int ntaps, int off_min, int span,
+                        int64_t blocks_per_row) {
+    fwd_window<kOrig>(x, y, n_in, n_out, taps64, ntaps, off_min, span, blocks_per_row);
+}
+
+// The adjoint of an integer upsampling by kNew, such a decimation over the
+// transposed bank, whose taps are floats: 48 rows of 84754 gradient samples, 1:2,
+// 20 -> 9.9 us against the tiled kernel.
+template <int kNew>
+__global__ void __launch_bounds__(kResampleThreads)
+    resample_up_adjoint(InRows gy, OutRows gx, int64_t n_out, int64_t n_in,
+                        const float *__restrict__ adj, int ntaps, int off_min, int span,
+                        int64_t blocks_per_row) {
+    fwd_window<kNew>(gy, gx, n_out, n_in, adj, ntaps, off_min, span, blocks_per_row);
 }
 
 // Integer upsampling (orig_step 1, kNew phases: 8 kHz to 16 kHz is 1:2): thread
@@ -1237,7 +1253,7 @@ static int plan_backward(InRows grad_y, OutRows grad_x, int64_t rows, int64_t n_
             const dim3 wgrid(static_cast<unsigned>(rows * wbpr)), wblock(kResampleThreads);
 #define PESQ_UP_ADJOINT(N)                                                                       \
     case N:                                                                                       \
-        hipLaunchKernelGGL((resample_fwd_window<N, float>), wgrid, wblock, size_t(wbytes), stream, \
+        hipLaunchKernelGGL(resample_up_adjoint<N>, wgrid, wblock, size_t(wbytes), stream,          \
                            grad_y, grad_x, n_out, n_in, adj, r.adj_taps, r.adj_off_min,           \
                            static_cast<int>(wspan), wbpr);                                        \
         PESQ_CHECK_LAUNCH("resample backward (window)");                                          \
