@@ -234,3 +234,26 @@ def test_other_geometry_rejects_too_few_frames():
     x = torch.randn(1, 8000, device="cuda")
     with pytest.raises(ValueError, match="20 frames"):
         model(x, x)
+
+
+@pytest.mark.parametrize("n_fft, hop", [(512, 160), (512, 512), (1024, 256), (1024, 1024), (256, 64)])
+@pytest.mark.parametrize("rows, nsamples", [(1, 1024), (3, 1025), (2, 4099), (40, 70001)])
+def test_transforms_at_odd_frame_counts(n_fft, hop, rows, nsamples):
+    """The radix-4, radix-8 and radix-2 transforms with one to four frames per
+    wavefront (chosen by the grid), last wavefronts partly filled, rows at odd
+    offsets: a row equals the same row alone bit for bit, and the float64
+    operator within the module's budgets (forward 1e-5 relative + 5e-6 of the
+    frame, backward + 1e-5 of the sample scale)."""
+
+    mod, window, scale = _module(n_fft, 49, hop)
+    signal = 1000.0 * torch.randn(rows, nsamples, generator=torch.Generator().manual_seed(nsamples))
+    got, want, g_got, g_want = _both(mod, window, scale, signal.cuda())
+    assert _violation(got, want, ATOL_FWD, _frame_scale(want)) <= 0.0
+    assert _violation(g_got, g_want, ATOL_BWD, _sample_scale(g_want, hop, mod.novertaps)) <= 0.0
+    x = signal.cuda().requires_grad_(True)
+    y = mod(x)
+    (g,) = torch.autograd.grad(y.sum(), x)
+    x1 = signal[-1:].cuda().requires_grad_(True)
+    y1 = mod(x1)
+    (g1,) = torch.autograd.grad(y1.sum(), x1)
+    assert torch.equal(y[-1:], y1) and torch.equal(g[-1:], g1)

@@ -1,241 +1,14 @@
 // Stand-alone STFT + Bark operator for any power-of-two FFT length and any
 // hop (the general TritonStftBark, torch_pesq/triton_ops/spectral.py:584-774):
-// n_fft = 32 .. 1024, hop >= 1, up to kGenMaxBands bands of a binary,
-// contiguous filterbank.  The PESQ geometry (512 / 256 / 49 bands) has its own
-// fused and stand-alone kernels; this file serves every other configuration.
-//
-// Forward, one wavefront per frame: the real frame u (window applied) is
-// folded into the half length complex sequence z_n = u_{2n} + i u_{2n+1},
-// transformed by a radix-2 Stockham FFT in a wave-private LDS buffer
-// (float64, log2(half) passes, the pass's butterflies spread over the lanes),
-// unfolded into X_f, f < half, and |X_f|^2 (DC dropped) summed per band.
-//
-// Backward: the same spectrum per frame, V_f = g_P(f) X_f, the adjoint of the
-// fold and an inverse FFT give the frame's sample gradient, which is written
-// (times the window) to a [rows, frames, n_fft] scratch; a gather kernel then
-// adds, for each sample, the contributions of the frames that cover it in
-// increasing frame order (deterministic, no atomics, any hop including hops
-// longer than n_fft, whose uncovered samples get exactly zero).
+// table packing, argument checks and launches of the kernels of
+// stft_generic.hpp.  The PESQ geometry (512 / 256 / 49 bands) has its own fused
+// and stand-alone kernels; this file serves every other configuration.
 #include <cmath>
 #include <cstring>
 
-#include "common.hpp"
-#include "spectral.hpp"
+#include "stft_generic.hpp"
 
 namespace pesq {
-
-constexpr int kGenMaxHalf = 512;   // n_fft <= 1024
-constexpr int kGenMinHalf = 16;    // n_fft >= 32
-constexpr int kGenMaxBands = 128;
-constexpr int kGenPerLane = kGenMaxHalf / kWave;       // points per lane (<= 8)
-constexpr int kGenBfly = kGenMaxHalf / 2 / kWave;      // butterflies per lane (<= 4)
-constexpr int kGenWaves = 4;                           // frames per workgroup
-
-struct StftTable {
-    int32_t n_fft, half, hop, nbarks;
-    double2 tw[kGenMaxHalf / 2];      // e^{-2 pi i m / half}, m < half / 2
-    double2 fold[kGenMaxHalf];        // e^{-2 pi i f / n_fft}, f < half
-    float window[2 * kGenMaxHalf];    // n_fft taps, centred
-    int32_t band_start[kGenMaxBands];
-    int32_t band_end[kGenMaxBands];
-    int32_t bin_band[kGenMaxHalf];    // band of bin f, -1 for none and for f = 0
-    double corr[kGenMaxBands];
-};
-
-struct GenArgs {
-    const StftTable *tab;
-    const float *x;       // [rows, len]
-    float *bark;          // [rows, frames, nbarks]
-    const float *gbark;   // [rows, frames, nbarks]
-    float *gx;            // [rows, len]
-    float *scratch;       // [rows, frames, n_fft]
-    int64_t rows, len, frames, ftiles;
-    int n_fft, half, hop, nbarks;
-};
-
-using c64g = cplx<double>;
-
-// In place radix-2 Stockham FFT of buf[0 .. half) (natural order in and out),
-// e^{-2 pi i / half} forward, conjugate twiddles for the inverse; unnormalised.
-// Pass s (sub-transform size ns = 2^s): butterfly j takes buf[j] and
-// buf[j + half / 2], k = j mod ns, w = e^{-2 pi i k / (2 ns)}, and writes
-// positions (j / ns) 2 ns + k and that plus ns.  Every lane reads all of its
-// butterflies' inputs before the wave's writes start.
-template <bool kInv>
-__device__ __forceinline__ void gen_fft(c64g *buf, const double2 *tw, int half, int lane) {
-    const int nb = half / 2;
-    for (int ns = 1; ns < half; ns *= 2) {
-        c64g a[kGenBfly], b[kGenBfly];
-#pragma unroll
-        for (int q = 0; q < kGenBfly; ++q) {
-            const int j = lane + kWave * q;
-            if (j < nb) {
-                a[q] = buf[j];
-                b[q] = buf[j + nb];
-            }
-        }
-        wave_lds_fence();
-#pragma unroll
-        for (int q = 0; q < kGenBfly; ++q) {
-            const int j = lane + kWave * q;
-            if (j < nb) {
-                const int k = j & (ns - 1);
-                const double2 w = tw[k * (nb / ns)];
-                const c64g v = cmul(b[q], c64g{w.x, kInv ? -w.y : w.y});
-                const int o = (j / ns) * 2 * ns + k;
-                buf[o] = {a[q].re + v.re, a[q].im + v.im};
-                buf[o + ns] = {a[q].re - v.re, a[q].im - v.im};
-            }
-        }
-        wave_lds_fence();
-    }
-}
-
-// spectrum X_f, f = lane + 64 r < half, of the frame starting at `start`;
-// buf ends up holding Z (the half length transform)
-__device__ __forceinline__ void gen_spectrum(const StftTable &t, const float *x, int64_t start,
-                                             int64_t len, int half, c64g *buf, int lane,
-                                             c64g (&spec)[kGenPerLane]) {
-#pragma unroll
-    for (int r = 0; r < kGenPerLane; ++r) {
-        const int n = lane + kWave * r;
-        if (n < half) {
-            const double u0 = static_cast<double>(load_or_zero(x, start + 2 * n, len)) *
-                              static_cast<double>(t.window[2 * n]);
-            const double u1 = static_cast<double>(load_or_zero(x, start + 2 * n + 1, len)) *
-                              static_cast<double>(t.window[2 * n + 1]);
-            buf[n] = {u0, u1};
-        }
-    }
-    wave_lds_fence();
-    gen_fft<false>(buf, t.tw, half, lane);
-#pragma unroll
-    for (int r = 0; r < kGenPerLane; ++r) {
-        const int f = lane + kWave * r;
-        if (f < half) {
-            const c64g zf = buf[f];
-            const c64g zm = buf[(half - f) & (half - 1)];
-            const c64g e = {(zf.re + zm.re) * 0.5, (zf.im - zm.im) * 0.5};
-            const c64g o = {(zf.im + zm.im) * 0.5, -(zf.re - zm.re) * 0.5};
-            const double2 c = t.fold[f];
-            const c64g v = cmul(c64g{c.x, c.y}, o);
-            spec[r] = {e.re + v.re, e.im + v.im};
-        }
-    }
-    wave_lds_fence();
-}
-
-__global__ void __launch_bounds__(kWave *kGenWaves) stft_gen_fwd_kernel(GenArgs a) {
-    __shared__ c64g bufs[kGenWaves][kGenMaxHalf];
-    const StftTable &t = *a.tab;
-    const int64_t row = blockIdx.x / a.ftiles;
-    const int64_t ft = blockIdx.x - row * a.ftiles;
-    const int wave = threadIdx.x / kWave;
-    const int lane = threadIdx.x % kWave;
-    const int64_t frame = ft * kGenWaves + wave;
-    if (frame >= a.frames) return;  // whole wavefronts; no block barrier follows
-    c64g *buf = bufs[wave];
-    c64g spec[kGenPerLane];
-    gen_spectrum(t, a.x + row * a.len, frame * a.hop, a.len, a.half, buf, lane, spec);
-    double *power = reinterpret_cast<double *>(buf);
-#pragma unroll
-    for (int r = 0; r < kGenPerLane; ++r) {
-        const int f = lane + kWave * r;
-        if (f < a.half) power[f] = f == 0 ? 0.0 : spec[r].re * spec[r].re + spec[r].im * spec[r].im;
-    }
-    wave_lds_fence();
-    float *out = a.bark + (row * a.frames + frame) * a.nbarks;
-    for (int b = lane; b < a.nbarks; b += kWave) {
-        double acc = 0.0;
-        for (int f = t.band_start[b]; f < t.band_end[b]; ++f) acc += power[f];
-        out[b] = static_cast<float>(acc * t.corr[b]);
-    }
-}
-
-// per frame: the frame's windowed sample gradient into the scratch
-__global__ void __launch_bounds__(kWave *kGenWaves) stft_gen_bwd_frames_kernel(GenArgs a) {
-    __shared__ c64g bufs[kGenWaves][kGenMaxHalf];
-    __shared__ float gband[kGenWaves][kGenMaxBands];
-    const StftTable &t = *a.tab;
-    const int64_t row = blockIdx.x / a.ftiles;
-    const int64_t ft = blockIdx.x - row * a.ftiles;
-    const int wave = threadIdx.x / kWave;
-    const int lane = threadIdx.x % kWave;
-    const int64_t frame = ft * kGenWaves + wave;
-    if (frame >= a.frames) return;
-    const int half = a.half;
-    const float *g = a.gbark + (row * a.frames + frame) * a.nbarks;
-    for (int b = lane; b < a.nbarks; b += kWave) {
-        gband[wave][b] = static_cast<float>(static_cast<double>(g[b]) * t.corr[b]);
-    }
-    c64g *buf = bufs[wave];
-    c64g spec[kGenPerLane];
-    gen_spectrum(t, a.x + row * a.len, frame * a.hop, a.len, half, buf, lane, spec);
-    // V_f = g_P(f) X_f (zero at DC and outside the bands), staged for V_{half - f}
-#pragma unroll
-    for (int r = 0; r < kGenPerLane; ++r) {
-        const int f = lane + kWave * r;
-        if (f < half) {
-            const int band = t.bin_band[f];
-            const double gp = band >= 0 ? static_cast<double>(gband[wave][band]) : 0.0;
-            spec[r] = {gp * spec[r].re, gp * spec[r].im};
-            buf[f] = spec[r];
-        }
-    }
-    wave_lds_fence();
-    // Z'_f = (V_f + conj V_{half-f}) + i e^{+2 pi i f / n} (V_f - conj V_{half-f}), V_half = 0
-    c64g zp[kGenPerLane];
-#pragma unroll
-    for (int r = 0; r < kGenPerLane; ++r) {
-        const int f = lane + kWave * r;
-        if (f < half) {
-            const c64g va = spec[r];
-            const c64g vb = f == 0 ? c64g{0.0, 0.0} : buf[half - f];
-            const c64g s = {va.re + vb.re, va.im - vb.im};
-            const c64g d = {va.re - vb.re, va.im + vb.im};
-            const double2 c = t.fold[f];
-            const c64g v = cmul(c64g{c.x, -c.y}, d);
-            zp[r] = {s.re - v.im, s.im + v.re};
-        }
-    }
-    wave_lds_fence();
-#pragma unroll
-    for (int r = 0; r < kGenPerLane; ++r) {
-        const int f = lane + kWave * r;
-        if (f < half) buf[f] = zp[r];
-    }
-    wave_lds_fence();
-    gen_fft<true>(buf, t.tw, half, lane);
-    float *dst = a.scratch + (row * a.frames + frame) * a.n_fft;
-#pragma unroll
-    for (int r = 0; r < kGenPerLane; ++r) {
-        const int n = lane + kWave * r;
-        if (n < half) {
-            const c64g z = buf[n];
-            dst[2 * n] = static_cast<float>(z.re * static_cast<double>(t.window[2 * n]));
-            dst[2 * n + 1] = static_cast<float>(z.im * static_cast<double>(t.window[2 * n + 1]));
-        }
-    }
-}
-
-constexpr int kGatherThreads = 256;
-
-// per sample: sum of the contributions of the frames covering it, in
-// increasing frame order
-__global__ void __launch_bounds__(kGatherThreads) stft_gen_bwd_gather_kernel(GenArgs a) {
-    const int64_t nblk = cdiv(a.len, kGatherThreads);
-    const int64_t row = blockIdx.x / nblk;
-    const int64_t n = (blockIdx.x - row * nblk) * kGatherThreads + threadIdx.x;
-    if (n >= a.len) return;
-    // frames t with t hop <= n < t hop + n_fft, t < frames
-    const int64_t t_lo = n < a.n_fft ? 0 : (n - a.n_fft) / a.hop + 1;
-    int64_t t_hi = n / a.hop;
-    if (t_hi > a.frames - 1) t_hi = a.frames - 1;
-    const float *src = a.scratch + row * a.frames * a.n_fft;
-    double g = 0.0;
-    for (int64_t t = t_lo; t <= t_hi; ++t) g += static_cast<double>(src[t * a.n_fft + (n - t * a.hop)]);
-    a.gx[row * a.len + n] = static_cast<float>(g);
-}
 
 static int check_geometry(int64_t rows, int64_t len, int64_t n_padded, int n_fft, int hop,
                           int nbarks, int64_t &frames) {
@@ -276,7 +49,7 @@ extern "C" int pesq_stft_table_pack(int n_fft, int hop, const float *window, int
     t->hop = hop;
     t->nbarks = nbarks;
     const double two_pi = 6.283185307179586476925286766559;
-    for (int m = 0; m < half / 2; ++m) {
+    for (int m = 0; m < half; ++m) {
         t->tw[m] = make_double2(std::cos(two_pi * m / half), -std::sin(two_pi * m / half));
     }
     for (int f = 0; f < half; ++f) {
@@ -329,13 +102,11 @@ extern "C" int pesq_stft_forward(const float *x, int64_t rows, int64_t len, int6
     a.rows = rows;
     a.len = len;
     a.frames = frames;
-    a.ftiles = cdiv(frames, kGenWaves);
     a.n_fft = n_fft;
     a.half = n_fft / 2;
     a.hop = hop;
     a.nbarks = nbarks;
-    hipLaunchKernelGGL(stft_gen_fwd_kernel, dim3(static_cast<unsigned>(rows * a.ftiles)),
-                       dim3(kWave * kGenWaves), 0, stream, a);
+    launch_gen_fwd(a, stream);
     PESQ_CHECK_LAUNCH("stft forward");
     return PESQ_OK;
 }
@@ -356,17 +127,11 @@ extern "C" int pesq_stft_backward(const float *gbark, const float *x, int64_t ro
     a.rows = rows;
     a.len = len;
     a.frames = frames;
-    a.ftiles = cdiv(frames, kGenWaves);
     a.n_fft = n_fft;
     a.half = n_fft / 2;
     a.hop = hop;
     a.nbarks = nbarks;
-    hipLaunchKernelGGL(stft_gen_bwd_frames_kernel, dim3(static_cast<unsigned>(rows * a.ftiles)),
-                       dim3(kWave * kGenWaves), 0, stream, a);
-    PESQ_CHECK_LAUNCH("stft backward frames");
-    hipLaunchKernelGGL(stft_gen_bwd_gather_kernel,
-                       dim3(static_cast<unsigned>(rows * cdiv(len, kGatherThreads))),
-                       dim3(kGatherThreads), 0, stream, a);
-    PESQ_CHECK_LAUNCH("stft backward gather");
+    launch_gen_bwd(a, stream);
+    PESQ_CHECK_LAUNCH("stft backward");
     return PESQ_OK;
 }

@@ -11,7 +11,8 @@ radix-4 kernels of ``csrc/pipeline.hip``; every other geometry, i.e.
 ``n_fft`` a power of two in [32, 1024], any ``hop_length`` (also longer than
 ``n_fft``, where uncovered samples get a zero gradient), windows shorter than
 ``n_fft`` (centred like ``torch.stft``) and up to 128 bands, runs the general
-radix-2 kernels of ``csrc/stft_generic.hip``.
+kernels of ``csrc/stft_generic.hpp`` (radix 4 at 512, radix 8 at 1024, else
+radix 2).
 """
 
 import ctypes
