@@ -162,6 +162,26 @@ int pesq_pipeline_backward(const float *g_symm, const float *g_asymm, const floa
                            float *g_ref, float *g_deg, const void *fwd_workspace,
                            void *bwd_workspace, hipStream_t stream);
 
+/* The same two passes at another STFT geometry (PesqLossTriton with other
+ * n_fft, win_length, hop_length; torch_pesq/triton_ops/loss.py:75-147): frames
+ * of n_fft samples every hop through the general STFT kernels, whose table
+ * (window, bands, correction) is pesq_stft_table_pack's for 49 bands; the
+ * model table's filters, thresholds, exponents and widths are used, its window
+ * and bands are not. */
+int pesq_pipeline_general_workspace(int64_t batch, int64_t len, int grad_mask, int n_fft,
+                                    int hop, size_t *forward_bytes, size_t *backward_bytes);
+int pesq_pipeline_general_forward(const float *ref, const float *deg, int64_t batch, int64_t len,
+                                  const void *model_table, const void *stft_table, int n_fft,
+                                  int hop, double factor, int grad_mask, float *d_symm,
+                                  float *d_asymm, float *mos, float *loss, void *fwd_workspace,
+                                  hipStream_t stream);
+int pesq_pipeline_general_backward(const float *g_symm, const float *g_asymm, const float *g_mos,
+                                   const float *g_loss, int64_t batch, int64_t len,
+                                   const void *model_table, const void *stft_table, int n_fft,
+                                   int hop, double factor, int grad_mask, float *g_ref,
+                                   float *g_deg, const void *fwd_workspace, void *bwd_workspace,
+                                   hipStream_t stream);
+
 /* The same two passes restricted to a subset of their kernels, for per stage
  * timing.  Forward bits: 1 scan aggregates, 2 scan outputs, 4 STFT/Bark,
  * 8 chain, 16 overlapping sums + epilogue.  Backward bits: 1 chain, 2 STFT,

@@ -257,3 +257,70 @@ def test_transforms_at_odd_frame_counts(n_fft, hop, rows, nsamples):
     y1 = mod(x1)
     (g1,) = torch.autograd.grad(y1.sum(), x1)
     assert torch.equal(y[-1:], y1) and torch.equal(g[-1:], g1)
+
+
+@pytest.mark.parametrize("n_fft, win_length, hop", [(64, 64, 37), (256, 200, 64), (512, 400, 160), (1024, 1024, 300)])
+@pytest.mark.parametrize("rate, nsamples", [(16000, 12001), (8000, 9003), (44100, 36007)])
+def test_loss_runs_the_operators_composed(n_fft, win_length, hop, rate, nsamples):
+    """The whole loss against its stand-alone operators in the reference's order
+    (common peak first), each input alone and both requiring a gradient, over
+    odd lengths, hops that leave ragged frames, and batches whose tiles pass
+    through the band totals (more than 64).  Both hold the transforms and
+    recursions in float64 and store each stage in float32: values within 2e-6
+    relative; gradients within 1e-4 of the row's peak, for a frame whose
+    disturbance lies at its dead zone takes either side."""
+
+    from bench import speech_like_pair
+    from torch_pesq import PesqLossTriton
+    from torch_pesq.hip_ops.elementwise import peak_normalize, pesq_epilogue
+
+    model = PesqLossTriton(0.5, sample_rate=rate, n_fft=n_fft, win_length=win_length,
+                           hop_length=hop).cuda()
+    ref, deg = speech_like_pair(3, nsamples, seed=n_fft, noise=0.1)
+    signals = [torch.from_numpy(x).cuda() for x in (ref, deg)]
+
+    def composed(r, d):
+        x = model.resampler(peak_normalize(r, d, stack=True)) if rate != 16000 else peak_normalize(r, d, stack=True)
+        y = model.preemphasize(model.align_level(x))
+        n = x.shape[1]
+        spectral = HipStftBark(model.to_spec.window, model.fbank.fbank,
+                               model.fbank.pow_dens_correction, n_fft, hop).cuda()
+        bark = spectral(y, n + n % 256)
+        ds, da = model.chain(bark[:3], bark[3:])
+        mos, loss = pesq_epilogue(ds, da, 0.5)
+        return ds, da, mos, loss
+
+    for need in ((True, True), (True, False), (False, True), (False, False)):
+        runs = []
+        for f in (model._run, composed):
+            ins = [x.clone().requires_grad_(n) for x, n in zip(signals, need)]
+            out = f(*ins)
+            want = [x for x in ins if x.requires_grad]
+            grads = torch.autograd.grad(out[2].sum() + out[3].sum(), want) if want else ()
+            runs.append((out, grads))
+        (got, g_got), (want, g_want) = runs
+        for a, b in zip(got, want):
+            torch.testing.assert_close(a.detach(), b.detach(), rtol=2e-6, atol=0.0)
+        for a, b in zip(g_got, g_want):
+            assert float(((a - b).abs().amax(1) / b.abs().amax(1)).max()) < 1e-4
+
+
+@pytest.mark.parametrize("bad", [float("inf"), -float("inf"), float("nan")])
+def test_general_loss_at_infinities(bad):
+    """An infinite sample is the common peak: neither signal of its pair keeps a
+    gradient; a NaN is not, and the other signal keeps its own.  Other pairs
+    are untouched."""
+
+    from torch_pesq import PesqLossTriton
+
+    model = PesqLossTriton(0.5, sample_rate=16000, hop_length=160).cuda()
+    x = torch.randn(2, 2, 9001, generator=torch.Generator().manual_seed(1)).cuda()
+    want = model(x[0], x[1])
+    y = x.clone()
+    y[0, 0, 777] = bad
+    r, d = y[0].requires_grad_(True), y[1].requires_grad_(True)
+    loss = model(r, d)
+    g_ref, g_deg = torch.autograd.grad(loss.sum(), [r, d])
+    assert loss[1] == want[1]
+    assert not g_ref[0].isfinite().any() and g_ref[1].isfinite().all()
+    assert g_deg[0].isfinite().all() == (bad != bad) and g_deg[1].isfinite().all()

@@ -35,6 +35,7 @@
 #include <type_traits>
 
 #include "pipeline_layout.hpp"
+#include "stft_generic.hpp"
 #include "tables.hpp"
 
 namespace pesq {
@@ -1449,6 +1450,20 @@ __global__ void __launch_bounds__(kWave) chain_partials_kernel(PipeArgs a) {
     }
     const float *bref = a.bark_ref + int64_t(item) * L.frames * nb;
     const float *bdeg = a.bark_deg + int64_t(item) * L.frames * nb;
+    // the tile's spectra are requested together (a load per frame, waited for
+    // before the next, took 15 us for 16 items of 25 tiles)
+    float rf[kTile][kBPL], df[kTile][kBPL];
+#pragma unroll
+    for (int local = 0; local < kTile; ++local) {
+        const int64_t frame = t0 + local < L.frames ? t0 + local : L.frames - 1;
+#pragma unroll
+        for (int k = 0; k < kBPL; ++k) {
+            const int64_t o = frame * nb + (live[k] ? lane + kWave * k : 0);
+            rf[local][k] = bref[o];
+            df[local][k] = bdeg[o];
+        }
+    }
+#pragma unroll
     for (int local = 0; local < kTile; ++local) {
         const int64_t frame = t0 + local;
         if (frame >= L.frames) break;
@@ -1456,9 +1471,8 @@ __global__ void __launch_bounds__(kWave) chain_partials_kernel(PipeArgs a) {
         double aud = 0.0;
 #pragma unroll
         for (int k = 0; k < kBPL; ++k) {
-            const int64_t o = frame * nb + lane + kWave * k;
-            rv[k] = live[k] ? static_cast<double>(bref[o]) : 0.0;
-            dv[k] = live[k] ? static_cast<double>(bdeg[o]) : 0.0;
+            rv[k] = live[k] ? static_cast<double>(rf[local][k]) : 0.0;
+            dv[k] = live[k] ? static_cast<double>(df[local][k]) : 0.0;
             const double x = live[k] && rv[k] > th100[k] ? rv[k] : 0.0;
             aud = k == 0 ? x : aud + x;
         }
@@ -1480,6 +1494,45 @@ __global__ void __launch_bounds__(kWave) chain_partials_kernel(PipeArgs a) {
     }
 }
 
+// Gradients of the mean band powers of an item's band (adjoint of the band
+// power ratio and its clamp) from the tile partials: {reference, degraded}.
+// The summation order of stft_bwd_kernel: the partial of each of its
+// wavefronts (tiles w, w + kBwdFrames, ...), then those in order; the loads of
+// all of them in flight together.
+__device__ __forceinline__ double2 mean_power_gradient(const PipeArgs &a, int item, int band) {
+    const PipeLayout &L = a.L;
+    const int nb = L.nb;
+    const double *gp = region<double>(a.bw, L.grpart) + int64_t(item) * L.ntile * nb;
+    const double *ptr[kBwdFrames];
+    int cnt[kBwdFrames];
+#pragma unroll
+    for (int w = 0; w < kBwdFrames; ++w) {
+        ptr[w] = gp + int64_t(w) * nb + band;
+        cnt[w] = L.ntile > w ? static_cast<int>((L.ntile - 1 - w) / kBwdFrames) + 1 : 0;
+    }
+    double parts[kBwdFrames];
+    strided_sums(ptr, cnt, int64_t(kBwdFrames) * nb, parts);
+    double g = 0.0;
+#pragma unroll
+    for (int w = 0; w < kBwdFrames; ++w) g += parts[w];
+    const double frames_f = static_cast<double>(L.frames);
+    const double ratio = band_array(a, kRatio)[item * nb + band];
+    const double mref = band_array(a, kMref)[item * nb + band];
+    const double gr = (ratio >= 0.01 && ratio <= 100.0) ? g : 0.0;
+    const double inv = 1.0 / (mref + 1000.0);
+    return make_double2(-gr * ratio * inv / frames_f, gr * inv / frames_f);
+}
+
+// once per item, for the general STFT's backward frames (49 bands)
+__global__ void __launch_bounds__(kWave) chain_gradmean_kernel(PipeArgs a) {
+    const int item = blockIdx.x, band = threadIdx.x;
+    if (band >= a.L.nb) return;
+    const double2 g = mean_power_gradient(a, item, band);
+    double *dst = region<double>(a.bw, a.L.gmean) + int64_t(item) * 2 * a.L.nb + band;
+    dst[0] = g.x;
+    dst[a.L.nb] = g.y;
+}
+
 template <int kBPL>
 __global__ void __launch_bounds__(kWave) chain_meanpow_kernel(PipeArgs a) {
     const ModelTable &t = *a.tab;
@@ -1489,45 +1542,37 @@ __global__ void __launch_bounds__(kWave) chain_meanpow_kernel(PipeArgs a) {
     const int tile = blockIdx.x - item * L.ntile;
     const int t0 = tile * kTile;
     const int lane = threadIdx.x;
-    const double *gp = region<double>(a.bw, L.grpart) + int64_t(item) * L.ntile * nb;
     const float *keep = region<float>(a.ws, L.keep) + int64_t(item) * L.frames;
-    const double frames_f = static_cast<double>(L.frames);
 #pragma unroll
     for (int k = 0; k < kBPL; ++k) {
         const int band = lane + kWave * k;
         if (band >= nb) continue;
-        // the summation order of stft_bwd_kernel: the partial of each of its
-        // wavefronts (tiles w, w + kBwdFrames, ...), then those in order; the
-        // loads of all of them in flight together
-        const double *ptr[kBwdFrames];
-        int cnt[kBwdFrames];
+        // the tile's spectra, gradients and flags are requested together (22 us
+        // for 16 items of 25 tiles when each frame waited for its own)
+        float rf[kTile], df[kTile], rg[kTile], dg[kTile], kf[kTile];
 #pragma unroll
-        for (int w = 0; w < kBwdFrames; ++w) {
-            ptr[w] = gp + int64_t(w) * nb + band;
-            cnt[w] = L.ntile > w ? static_cast<int>((L.ntile - 1 - w) / kBwdFrames) + 1 : 0;
+        for (int local = 0; local < kTile; ++local) {
+            const int64_t frame = t0 + local < L.frames ? t0 + local : L.frames - 1;
+            const int64_t o = (int64_t(item) * L.frames + frame) * nb + band;
+            kf[local] = keep[frame];
+            rf[local] = a.bark_ref[o];
+            df[local] = a.bark_deg[o];
+            rg[local] = a.gbark_ref[o];
+            dg[local] = a.gbark_deg[o];
         }
-        double parts[kBwdFrames];
-        strided_sums(ptr, cnt, int64_t(kBwdFrames) * nb, parts);
-        double g = 0.0;
-#pragma unroll
-        for (int w = 0; w < kBwdFrames; ++w) g += parts[w];
-        const double ratio = band_array(a, kRatio)[item * nb + band];
-        const double mref = band_array(a, kMref)[item * nb + band];
-        const double gr = (ratio >= 0.01 && ratio <= 100.0) ? g : 0.0;
-        const double inv = 1.0 / (mref + 1000.0);
-        const double gm_ref = -gr * ratio * inv / frames_f;
-        const double gm_deg = gr * inv / frames_f;
+        const double2 gm = mean_power_gradient(a, item, band);
         const double th100 = 100.0 * t.threshs[band];
+#pragma unroll
         for (int local = 0; local < kTile; ++local) {
             const int64_t frame = t0 + local;
             if (frame >= L.frames) break;
-            if (keep[frame] == 0.0f) continue;
+            if (kf[local] == 0.0f) continue;
             const int64_t o = (int64_t(item) * L.frames + frame) * nb + band;
-            if (static_cast<double>(a.bark_ref[o]) > th100) {
-                a.gbark_ref[o] = static_cast<float>(static_cast<double>(a.gbark_ref[o]) + gm_ref);
+            if (static_cast<double>(rf[local]) > th100) {
+                a.gbark_ref[o] = static_cast<float>(static_cast<double>(rg[local]) + gm.x);
             }
-            if (static_cast<double>(a.bark_deg[o]) > th100) {
-                a.gbark_deg[o] = static_cast<float>(static_cast<double>(a.gbark_deg[o]) + gm_deg);
+            if (static_cast<double>(df[local]) > th100) {
+                a.gbark_deg[o] = static_cast<float>(static_cast<double>(dg[local]) + gm.y);
             }
         }
     }
@@ -1844,17 +1889,64 @@ extern "C" int pesq_pipeline_kernels(int64_t batch, int64_t len, int grad_mask, 
     return PESQ_OK;
 }
 
-extern "C" int pesq_pipeline_forward_stages(const float *ref, const float *deg, int64_t batch,
-                                            int64_t len, const void *model_table, double factor,
-                                            int grad_mask, float *d_symm, float *d_asymm,
-                                            float *mos, float *loss, void *fwd_workspace,
-                                            unsigned stages, hipStream_t stream) {
-    PipeArgs a{};
-    a.L.build(batch, len, grad_mask);
-    if (int st = check_sizes(batch, len, a.L)) return st;
+// An STFT geometry other than the pipeline's own: its packed table (device
+// memory), frame length and hop.  Its frames go through the general kernels,
+// with the level alignment's scale and the mean band power gradients applied
+// where these load; the band partials, which the fused STFT forms in passing,
+// take a pass of their own (6 us for 16 pairs of 400 frames).
+struct Geometry {
+    const void *table;
+    int n_fft, hop;
+};
+
+// Workspace layout of a shape at the pipeline's geometry (geo null) or another.
+static int layout_for(PipeLayout &L, int64_t batch, int64_t len, int grad_mask,
+                      const Geometry *geo) {
     PESQ_CHECK_ARG((grad_mask & ~3) == 0, "invalid grad_mask %d", grad_mask);
+    if (geo == nullptr) {
+        L.build(batch, len, grad_mask);
+        return check_sizes(batch, len, L);
+    }
+    PESQ_CHECK_ARG(geo->n_fft >= 2 * kGenMinHalf && geo->n_fft <= 2 * kGenMaxHalf &&
+                       (geo->n_fft & (geo->n_fft - 1)) == 0 && geo->hop >= 1,
+                   "invalid STFT geometry (n_fft %d, hop %d)", geo->n_fft, geo->hop);
+    L.build_general(batch, len, grad_mask, geo->n_fft, geo->hop);
+    if (int st = check_sizes(batch, len, L)) return st;
+    PESQ_CHECK_ARG(2 * batch * cdiv(L.frames, int64_t(kGenWaves)) < (int64_t(1) << 31),
+                   "problem too large for one launch");
+    return PESQ_OK;
+}
+
+// the general STFT kernels' arguments over stacked rows row0 .. row0 + rows - 1
+static GenArgs general_args(const PipeArgs &a, const Geometry &geo, int row0, int64_t rows) {
+    const PipeLayout &L = a.L;
+    const int64_t bands = int64_t(row0) * L.frames * kBands;
+    GenArgs g{};
+    g.tab = static_cast<const StftTable *>(geo.table);
+    g.x = region<float>(a.ws, L.p) + int64_t(row0) * L.len;
+    g.bark = region<float>(a.ws, L.bark) + bands;
+    g.rowconst = region<double>(a.ws, L.rowconst) + int64_t(row0) * 4;
+    g.rows = rows;
+    g.len = L.len;
+    g.frames = L.frames;
+    g.n_fft = L.n_fft;
+    g.half = L.n_fft / 2;
+    g.hop = L.hop;
+    g.nbarks = kBands;
+    g.batch = L.batch;
+    g.row0 = row0;
+    return g;
+}
+
+static int pipeline_forward(const float *ref, const float *deg, int64_t batch, int64_t len,
+                            const void *model_table, const Geometry *geo, double factor,
+                            int grad_mask, float *d_symm, float *d_asymm, float *mos, float *loss,
+                            void *fwd_workspace, unsigned stages, hipStream_t stream) {
+    PipeArgs a{};
+    if (int st = layout_for(a.L, batch, len, grad_mask, geo)) return st;
     if (batch == 0) return PESQ_OK;  // an empty batch has nothing to score
-    PESQ_CHECK_ARG(ref && deg && model_table && fwd_workspace && d_symm && d_asymm && mos && loss,
+    PESQ_CHECK_ARG(ref && deg && model_table && fwd_workspace && d_symm && d_asymm && mos &&
+                       loss && (geo == nullptr || geo->table != nullptr),
                    "null pointer argument");
     a.tab = static_cast<const ModelTable *>(model_table);
     a.ref = ref;
@@ -1891,7 +1983,18 @@ extern "C" int pesq_pipeline_forward_stages(const float *ref, const float *deg, 
             return st;
         }
     }
-    if (stages & 4u) {
+    if ((stages & 4u) && geo != nullptr) {
+        GenArgs g = general_args(a, *geo, 0, L.rows);
+        g.energy = region<double>(a.ws, L.energy);
+        g.nblk = L.nblk;
+        g.ref = ref;
+        g.deg = deg;
+        launch_gen_fwd(g, stream);
+        PESQ_CHECK_LAUNCH("pipeline general stft");
+        hipLaunchKernelGGL(chain_partials_kernel<1>, dim3(static_cast<unsigned>(batch * L.ntile)),
+                           dim3(kWave), 0, stream, a);
+        PESQ_CHECK_LAUNCH("pipeline band partials");
+    } else if (stages & 4u) {
         unsigned grid = static_cast<unsigned>(batch * L.ntile);
         // and the backward's level alignment aggregate blocks, a wavefront each
         if (L.host_power) grid += static_cast<unsigned>(cdiv(L.nrg * L.nblk, kStftWaves));
@@ -1922,29 +2025,60 @@ extern "C" int pesq_pipeline_forward_stages(const float *ref, const float *deg, 
     return PESQ_OK;
 }
 
+extern "C" int pesq_pipeline_forward_stages(const float *ref, const float *deg, int64_t batch,
+                                            int64_t len, const void *model_table, double factor,
+                                            int grad_mask, float *d_symm, float *d_asymm,
+                                            float *mos, float *loss, void *fwd_workspace,
+                                            unsigned stages, hipStream_t stream) {
+    return pipeline_forward(ref, deg, batch, len, model_table, nullptr, factor, grad_mask, d_symm,
+                            d_asymm, mos, loss, fwd_workspace, stages, stream);
+}
+
 extern "C" int pesq_pipeline_forward(const float *ref, const float *deg, int64_t batch,
                                      int64_t len, const void *model_table, double factor,
                                      int grad_mask, float *d_symm, float *d_asymm, float *mos,
                                      float *loss, void *fwd_workspace, hipStream_t stream) {
-    return pesq_pipeline_forward_stages(ref, deg, batch, len, model_table, factor, grad_mask,
-                                        d_symm, d_asymm, mos, loss, fwd_workspace, 0x1Fu, stream);
+    return pipeline_forward(ref, deg, batch, len, model_table, nullptr, factor, grad_mask, d_symm,
+                            d_asymm, mos, loss, fwd_workspace, 0x1Fu, stream);
 }
 
-extern "C" int pesq_pipeline_backward_stages(const float *g_symm, const float *g_asymm,
-                                             const float *g_mos, const float *g_loss,
-                                             int64_t batch, int64_t len, const void *model_table,
-                                             double factor, int grad_mask, float *g_ref,
-                                             float *g_deg, const void *fwd_workspace,
-                                             void *bwd_workspace, unsigned stages,
-                                             hipStream_t stream) {
+extern "C" int pesq_pipeline_general_workspace(int64_t batch, int64_t len, int grad_mask,
+                                               int n_fft, int hop, size_t *forward_bytes,
+                                               size_t *backward_bytes) {
+    PESQ_CHECK_ARG(forward_bytes && backward_bytes, "null argument");
+    const Geometry geo{nullptr, n_fft, hop};
+    PipeLayout L;
+    if (int st = layout_for(L, batch, len, grad_mask, &geo)) return st;
+    *forward_bytes = L.fwd_bytes;
+    *backward_bytes = L.bwd_bytes;
+    return PESQ_OK;
+}
+
+extern "C" int pesq_pipeline_general_forward(const float *ref, const float *deg, int64_t batch,
+                                             int64_t len, const void *model_table,
+                                             const void *stft_table, int n_fft, int hop,
+                                             double factor, int grad_mask, float *d_symm,
+                                             float *d_asymm, float *mos, float *loss,
+                                             void *fwd_workspace, hipStream_t stream) {
+    const Geometry geo{stft_table, n_fft, hop};
+    return pipeline_forward(ref, deg, batch, len, model_table, &geo, factor, grad_mask, d_symm,
+                            d_asymm, mos, loss, fwd_workspace, 0x1Fu, stream);
+}
+
+static int pipeline_backward(const float *g_symm, const float *g_asymm, const float *g_mos,
+                             const float *g_loss, int64_t batch, int64_t len,
+                             const void *model_table, const Geometry *geo, double factor,
+                             int grad_mask, float *g_ref, float *g_deg, const void *fwd_workspace,
+                             void *bwd_workspace, unsigned stages, hipStream_t stream) {
     PipeArgs a{};
-    a.L.build(batch, len, grad_mask);
-    if (int st = check_sizes(batch, len, a.L)) return st;
     PESQ_CHECK_ARG(grad_mask >= 1 && grad_mask <= 3, "backward needs a non-empty grad_mask");
+    if (int st = layout_for(a.L, batch, len, grad_mask, geo)) return st;
     if (batch == 0) return PESQ_OK;
     PESQ_CHECK_ARG(!(grad_mask & PESQ_GRAD_REF) || g_ref, "g_ref is required by grad_mask");
     PESQ_CHECK_ARG(!(grad_mask & PESQ_GRAD_DEG) || g_deg, "g_deg is required by grad_mask");
-    PESQ_CHECK_ARG(model_table && fwd_workspace && bwd_workspace, "null pointer argument");
+    PESQ_CHECK_ARG(model_table && fwd_workspace && bwd_workspace &&
+                       (geo == nullptr || geo->table != nullptr),
+                   "null pointer argument");
     a.tab = static_cast<const ModelTable *>(model_table);
     a.ws = static_cast<unsigned char *>(const_cast<void *>(fwd_workspace));
     a.bw = static_cast<unsigned char *>(bwd_workspace);
@@ -1964,7 +2098,22 @@ extern "C" int pesq_pipeline_backward_stages(const float *g_symm, const float *g
         launch_chain_bwd(a, static_cast<unsigned>(batch * L.ntile), stream);
         PESQ_CHECK_LAUNCH("pipeline chain backward");
     }
-    if (stages & 2u) {
+    if ((stages & 2u) && geo != nullptr) {
+        hipLaunchKernelGGL(chain_gradmean_kernel, dim3(static_cast<unsigned>(batch)), dim3(kWave),
+                           0, stream, a);
+        PESQ_CHECK_LAUNCH("pipeline mean power gradients");
+        GenArgs g = general_args(a, *geo, static_cast<int>(L.row0), L.nrg);
+        g.gbark = region<float>(a.bw, L.gbark) + L.row0 * L.frames * kBands;
+        g.gx = region<float>(a.bw, L.gp);
+        g.scratch = region<float>(a.bw, L.contrib);
+        g.gmean = region<double>(a.bw, L.gmean);
+        g.threshs = a.tab->threshs;
+        g.keep = region<float>(a.ws, L.keep);
+        g.spart = region<double>(a.bw, L.spart);
+        g.nhop = L.nhop;
+        launch_gen_bwd(g, stream);
+        PESQ_CHECK_LAUNCH("pipeline general stft backward");
+    } else if (stages & 2u) {
         if (L.totals) {
             hipLaunchKernelGGL((band_totals_kernel<kGradSlices, 1>),
                                dim3(static_cast<unsigned>(batch)), dim3(kWave * kGradSlices), 0,
@@ -2014,15 +2163,40 @@ extern "C" int pesq_pipeline_backward_stages(const float *g_symm, const float *g
     return PESQ_OK;
 }
 
+extern "C" int pesq_pipeline_backward_stages(const float *g_symm, const float *g_asymm,
+                                             const float *g_mos, const float *g_loss,
+                                             int64_t batch, int64_t len, const void *model_table,
+                                             double factor, int grad_mask, float *g_ref,
+                                             float *g_deg, const void *fwd_workspace,
+                                             void *bwd_workspace, unsigned stages,
+                                             hipStream_t stream) {
+    return pipeline_backward(g_symm, g_asymm, g_mos, g_loss, batch, len, model_table, nullptr,
+                             factor, grad_mask, g_ref, g_deg, fwd_workspace, bwd_workspace,
+                             stages, stream);
+}
+
 extern "C" int pesq_pipeline_backward(const float *g_symm, const float *g_asymm,
                                       const float *g_mos, const float *g_loss, int64_t batch,
                                       int64_t len, const void *model_table, double factor,
                                       int grad_mask, float *g_ref, float *g_deg,
                                       const void *fwd_workspace, void *bwd_workspace,
                                       hipStream_t stream) {
-    return pesq_pipeline_backward_stages(g_symm, g_asymm, g_mos, g_loss, batch, len, model_table,
-                                         factor, grad_mask, g_ref, g_deg, fwd_workspace,
-                                         bwd_workspace, 0xFu, stream);
+    return pipeline_backward(g_symm, g_asymm, g_mos, g_loss, batch, len, model_table, nullptr,
+                             factor, grad_mask, g_ref, g_deg, fwd_workspace, bwd_workspace, 0xFu,
+                             stream);
+}
+
+extern "C" int pesq_pipeline_general_backward(const float *g_symm, const float *g_asymm,
+                                              const float *g_mos, const float *g_loss,
+                                              int64_t batch, int64_t len, const void *model_table,
+                                              const void *stft_table, int n_fft, int hop,
+                                              double factor, int grad_mask, float *g_ref,
+                                              float *g_deg, const void *fwd_workspace,
+                                              void *bwd_workspace, hipStream_t stream) {
+    const Geometry geo{stft_table, n_fft, hop};
+    return pipeline_backward(g_symm, g_asymm, g_mos, g_loss, batch, len, model_table, &geo,
+                             factor, grad_mask, g_ref, g_deg, fwd_workspace, bwd_workspace, 0xFu,
+                             stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -80,12 +80,25 @@ struct PipeLayout {
     // backward workspace
     size_t gbark = 0, grpart = 0, gp = 0, spart = 0, aggr_b = 0, bwd_bytes = 0;
     size_t gradtot = 0;  // [batch, nb] totals of grpart (with `totals`)
+    // STFT geometries other than the pipeline's own (general): frames of n_fft
+    // samples every hop, through the general STFT kernels
+    bool general = false;
+    int n_fft = kNfft, hop = kHop;
+    size_t gmean = 0;    // [batch, 2, nb] mean band power gradients
+    size_t contrib = 0;  // [nrg, frames, n_fft] float frame gradients
 
     static size_t align(size_t v) { return (v + 255) & ~size_t(255); }
 
-    static int64_t frames_for(int64_t len) {
+    static int64_t frames_for(int64_t len, int n_fft = kNfft, int hop = kHop) {
         const int64_t padded = len + len % 256;
-        return padded < kNfft ? 0 : 1 + (padded - kNfft) / kHop;
+        return padded < n_fft ? 0 : 1 + (padded - n_fft) / hop;
+    }
+
+    void build_general(int64_t b, int64_t n, int mask, int fft, int step) {
+        general = true;
+        n_fft = fft;
+        hop = step;
+        build(b, n, mask);
     }
 
     void build(int64_t b, int64_t n, int mask) {
@@ -94,7 +107,7 @@ struct PipeLayout {
         len = n;
         rows = 2 * b;
         grad_mask = mask;
-        frames = frames_for(n);
+        frames = frames_for(n, n_fft, hop);
         nblk = cdiv(n, kBlockSpan);
         ntile = cdiv(frames, kTile);
         // by the rows the STFT backward runs over: with both gradients twice the
@@ -131,7 +144,7 @@ struct PipeLayout {
         take(loud, loud_store ? kChainTermBytes * batch * frames * nb : 0);
         take(bandtot, totals ? size_t(2) * batch * nb * sizeof(double) : 0);
         const ScanPlan bwd_scan = scan_plan(nrg, nblk);
-        host_power = nrg > 0 && bwd_scan.lane_states && bwd_scan.fused_prefix &&
+        host_power = !general && nrg > 0 && bwd_scan.lane_states && bwd_scan.fused_prefix &&
                      b * ntile <= kWideTiles;
         const size_t bwd_scan_bytes =
             size_t(scan_workspace_doubles(nrg, nblk, kPipeSections)) * sizeof(double);
@@ -146,6 +159,8 @@ struct PipeLayout {
         take(spart, size_t(nrg) * nhop * sizeof(double));
         take(aggr_b, host_power ? 0 : bwd_scan_bytes);
         take(gradtot, totals ? size_t(batch) * nb * sizeof(double) : 0);
+        take(gmean, general ? size_t(2) * batch * nb * sizeof(double) : 0);
+        take(contrib, general ? size_t(nrg) * frames * n_fft * sizeof(float) : 0);
         bwd_bytes = off;
         if (host_power) aggr_b = aggr_f;  // an offset into the forward workspace
     }

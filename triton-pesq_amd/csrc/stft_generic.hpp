@@ -67,6 +67,7 @@ struct GenArgs {
     // gmean [items][2][nbarks], added to gbark in the frames that count
     // (keep) where the Bark value exceeds 100 thresholds
     const double *energy;
+    const float *ref, *deg;  // the pipeline's signals [batch, len], rows 0 .. batch - 1 and on
     double *rowconst;     // [rows, 4]: -, E, scale, -
     const double *gmean, *threshs;
     const float *keep;    // [items, frames]
@@ -345,6 +346,19 @@ __device__ __forceinline__ int gen_frames(const GenArgs &a, int64_t &row, int64_
     return left <= 0 ? 0 : static_cast<int>(left < a.per ? left : a.per);
 }
 
+// the energy of a row from its blocks' partials (a whole wavefront's call)
+__device__ __forceinline__ double gen_energy(const GenArgs &a, int64_t row, int lane) {
+    const int mine = lane < a.nblk ? static_cast<int>((a.nblk - 1 - lane) / kWave + 1) : 0;
+    return wave_sum(mine > 0 ? strided_sum(a.energy + row * a.nblk + lane, mine, kWave) : 0.0);
+}
+
+// whether any of x[0 .. len) is infinite
+__device__ __forceinline__ bool gen_has_infinity(const float *x, int64_t len, int lane) {
+    bool found = false;
+    for (int64_t i = lane; i < len; i += kWave) found |= isinf(x[i]);
+    return __any(found);
+}
+
 template <int kH>
 __global__ void __launch_bounds__(kWave *kGenWaves) stft_gen_fwd_kernel(GenArgs a) {
     using F = GenFft<kH>;
@@ -363,9 +377,17 @@ __global__ void __launch_bounds__(kWave *kGenWaves) stft_gen_fwd_kernel(GenArgs 
     if (count == 0) return;  // whole wavefronts; no barrier follows
     double scale2 = 1.0;
     if (a.energy != nullptr) {
-        const double *energy = a.energy + row * a.nblk;
-        const int mine = lane < a.nblk ? static_cast<int>((a.nblk - 1 - lane) / kWave + 1) : 0;
-        const double e = wave_sum(mine > 0 ? strided_sum(energy + lane, mine, kWave) : 0.0);
+        double e = gen_energy(a, row, lane);
+        // Dividing both signals by an infinite common peak leaves neither any
+        // finite energy: an infinity in the other signal makes this one's
+        // energy NaN too (looked for only where the other's is not finite).
+        const bool is_ref = row < a.batch;
+        const double other = gen_energy(a, is_ref ? row + a.batch : row - a.batch, lane);
+        if (!isfinite(other) &&
+            gen_has_infinity(is_ref ? a.deg + row * a.len : a.ref + (row - a.batch) * a.len,
+                             a.len, lane)) {
+            e = other - other;
+        }
         const double power = e / static_cast<double>(a.len + 5120) / 1.04684;
         const double scale = sqrt(1e7 / power);
         scale2 = scale * scale;

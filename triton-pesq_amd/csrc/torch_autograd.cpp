@@ -20,6 +20,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <array>
+#include <limits>
 #include <vector>
 #include <stdexcept>
 #include <string>
@@ -58,27 +59,76 @@ struct OnceDifferentiable : public torch::autograd::Function<OnceDifferentiable>
     }
 };
 
+// An STFT geometry other than the pipeline's own (stft undefined: its own): the
+// packed table, frame length and hop.
+struct Geometry {
+    at::Tensor stft;
+    int64_t n_fft = 0, hop = 0;
+    bool general() const { return stft.defined(); }
+};
+
+size_t forward_workspace(int64_t batch, int64_t len, int mask, const Geometry &geo) {
+    size_t fwd = 0, bwd = 0;
+    if (geo.general()) {
+        check(pesq_pipeline_general_workspace(batch, len, mask, static_cast<int>(geo.n_fft),
+                                              static_cast<int>(geo.hop), &fwd, &bwd),
+              "pesq_pipeline_general_workspace");
+    } else {
+        check(pesq_pipeline_forward_workspace(batch, len, mask, &fwd),
+              "pesq_pipeline_forward_workspace");
+    }
+    return fwd;
+}
+
+size_t backward_workspace(int64_t batch, int64_t len, int mask, const Geometry &geo) {
+    size_t fwd = 0, bwd = 0;
+    if (geo.general()) {
+        check(pesq_pipeline_general_workspace(batch, len, mask, static_cast<int>(geo.n_fft),
+                                              static_cast<int>(geo.hop), &fwd, &bwd),
+              "pesq_pipeline_general_workspace");
+    } else {
+        check(pesq_pipeline_backward_workspace(batch, len, mask, &bwd),
+              "pesq_pipeline_backward_workspace");
+    }
+    return bwd;
+}
+
 struct Pipeline : public torch::autograd::Function<Pipeline> {
     // (ref, deg) [batch, len] float32 at 16 kHz -> (d_symm, d_asymm, mos, loss) [batch]
     // grad_mask (PESQ_GRAD_*) names the inputs the backward will differentiate
     static variable_list forward(AutogradContext *ctx, const at::Tensor &ref, const at::Tensor &deg,
-                                 const at::Tensor &table, double factor, int64_t grad_mask) {
+                                 const at::Tensor &table, double factor, int64_t grad_mask,
+                                 const Geometry &geo) {
         const int mask = static_cast<int>(grad_mask);
         const c10::DeviceGuard guard(ref.device());
         const int64_t batch = ref.size(0), len = ref.size(1);
-        size_t ws_bytes = 0;
-        check(pesq_pipeline_forward_workspace(batch, len, mask, &ws_bytes),
-              "pesq_pipeline_forward_workspace");
+        const size_t ws_bytes = forward_workspace(batch, len, mask, geo);
         at::Tensor ws = at::empty({static_cast<int64_t>(ws_bytes)}, ref.options().dtype(at::kByte));
         std::array<at::Tensor, 4> out;
         for (at::Tensor &o : out) o = at::empty({batch}, ref.options());
-        check(pesq_pipeline_forward(ref.data_ptr<float>(), deg.data_ptr<float>(), batch, len,
-                                    table.data_ptr(), factor, mask, out[0].data_ptr<float>(),
-                                    out[1].data_ptr<float>(), out[2].data_ptr<float>(),
-                                    out[3].data_ptr<float>(), ws.data_ptr(), current_stream(ref)),
-              "pesq_pipeline_forward");
+        if (geo.general()) {
+            check(pesq_pipeline_general_forward(
+                      ref.data_ptr<float>(), deg.data_ptr<float>(), batch, len, table.data_ptr(),
+                      geo.stft.data_ptr(), static_cast<int>(geo.n_fft), static_cast<int>(geo.hop),
+                      factor, mask, out[0].data_ptr<float>(), out[1].data_ptr<float>(),
+                      out[2].data_ptr<float>(), out[3].data_ptr<float>(), ws.data_ptr(),
+                      current_stream(ref)),
+                  "pesq_pipeline_general_forward");
+        } else {
+            check(pesq_pipeline_forward(ref.data_ptr<float>(), deg.data_ptr<float>(), batch, len,
+                                        table.data_ptr(), factor, mask, out[0].data_ptr<float>(),
+                                        out[1].data_ptr<float>(), out[2].data_ptr<float>(),
+                                        out[3].data_ptr<float>(), ws.data_ptr(),
+                                        current_stream(ref)),
+                  "pesq_pipeline_forward");
+        }
         ctx->set_materialize_grads(false);
-        ctx->save_for_backward({ws, table});
+        ctx->save_for_backward(geo.general() ? variable_list{ws, table, geo.stft}
+                                             : variable_list{ws, table});
+        if (geo.general()) {
+            ctx->saved_data["n_fft"] = geo.n_fft;
+            ctx->saved_data["hop"] = geo.hop;
+        }
         ctx->saved_data["batch"] = batch;
         ctx->saved_data["len"] = len;
         ctx->saved_data["mask"] = mask;
@@ -91,7 +141,7 @@ struct Pipeline : public torch::autograd::Function<Pipeline> {
         const int64_t len = ctx->saved_data["len"].toInt();
         const int mask = static_cast<int>(ctx->saved_data["mask"].toInt());
         const double factor = ctx->saved_data["factor"].toDouble();
-        variable_list result(5);  // one per argument of forward: ref, deg, table, factor, mask
+        variable_list result(6);  // one per argument of forward: ref, deg, table, factor, mask, geo
         bool any = false, upstream_requires_grad = false;
         for (const at::Tensor &g : grads) {
             any = any || g.defined();
@@ -102,6 +152,10 @@ struct Pipeline : public torch::autograd::Function<Pipeline> {
         const variable_list saved = ctx->get_saved_variables();
         const at::Tensor &ws = saved[0];
         const at::Tensor &table = saved[1];
+        Geometry geo;
+        if (saved.size() > 2) {
+            geo = {saved[2], ctx->saved_data["n_fft"].toInt(), ctx->saved_data["hop"].toInt()};
+        }
         const c10::DeviceGuard guard(ws.device());
         std::array<at::Tensor, 4> g;
         {
@@ -109,20 +163,29 @@ struct Pipeline : public torch::autograd::Function<Pipeline> {
             for (size_t i = 0; i < 4; ++i)
                 if (grads[i].defined()) g[i] = grads[i].to(at::kFloat).contiguous();
         }
-        size_t bw_bytes = 0;
-        check(pesq_pipeline_backward_workspace(batch, len, mask, &bw_bytes),
-              "pesq_pipeline_backward_workspace");
+        const size_t bw_bytes = backward_workspace(batch, len, mask, geo);
         at::Tensor scratch = at::empty({static_cast<int64_t>(bw_bytes)}, ws.options());
         const auto f32 = ws.options().dtype(at::kFloat);
         at::Tensor g_ref, g_deg;
         if (mask & PESQ_GRAD_REF) g_ref = at::empty({batch, len}, f32);
         if (mask & PESQ_GRAD_DEG) g_deg = at::empty({batch, len}, f32);
-        check(pesq_pipeline_backward(data_or_null<float>(g[0]), data_or_null<float>(g[1]),
-                                     data_or_null<float>(g[2]), data_or_null<float>(g[3]), batch,
-                                     len, table.data_ptr(), factor, mask,
-                                     data_or_null<float>(g_ref), data_or_null<float>(g_deg),
-                                     ws.data_ptr(), scratch.data_ptr(), current_stream(ws)),
-              "pesq_pipeline_backward");
+        if (geo.general()) {
+            check(pesq_pipeline_general_backward(
+                      data_or_null<float>(g[0]), data_or_null<float>(g[1]),
+                      data_or_null<float>(g[2]), data_or_null<float>(g[3]), batch, len,
+                      table.data_ptr(), geo.stft.data_ptr(), static_cast<int>(geo.n_fft),
+                      static_cast<int>(geo.hop), factor, mask, data_or_null<float>(g_ref),
+                      data_or_null<float>(g_deg), ws.data_ptr(), scratch.data_ptr(),
+                      current_stream(ws)),
+                  "pesq_pipeline_general_backward");
+        } else {
+            check(pesq_pipeline_backward(data_or_null<float>(g[0]), data_or_null<float>(g[1]),
+                                         data_or_null<float>(g[2]), data_or_null<float>(g[3]),
+                                         batch, len, table.data_ptr(), factor, mask,
+                                         data_or_null<float>(g_ref), data_or_null<float>(g_deg),
+                                         ws.data_ptr(), scratch.data_ptr(), current_stream(ws)),
+                  "pesq_pipeline_backward");
+        }
         result[0] = g_ref;
         result[1] = g_deg;
         if (torch::autograd::GradMode::is_enabled() && upstream_requires_grad) {
@@ -387,14 +450,20 @@ void check_pipeline_inputs(const at::Tensor &ref, const at::Tensor &deg, const a
                 pesq_model_table_bytes(), " bytes)");
 }
 
-std::vector<at::Tensor> pipeline(const at::Tensor &ref, const at::Tensor &deg,
-                                 const at::Tensor &table, double factor) {
+std::vector<at::Tensor> run_pipeline(const at::Tensor &ref, const at::Tensor &deg,
+                                     const at::Tensor &table, double factor,
+                                     const Geometry &geo) {
     check_pipeline_inputs(ref, deg, table);
     // what Python's ctx.needs_input_grad gives: the inputs autograd will ask for
     const bool grad = torch::autograd::GradMode::is_enabled();
     const int64_t mask = (grad && ref.requires_grad() ? PESQ_GRAD_REF : 0) |
                          (grad && deg.requires_grad() ? PESQ_GRAD_DEG : 0);
-    return Pipeline::apply(ref, deg, table, factor, mask);
+    return Pipeline::apply(ref, deg, table, factor, mask, geo);
+}
+
+std::vector<at::Tensor> pipeline(const at::Tensor &ref, const at::Tensor &deg,
+                                 const at::Tensor &table, double factor) {
+    return run_pipeline(ref, deg, table, factor, Geometry{});
 }
 
 // pipeline() of the two signals resampled to 16 kHz (n_out samples per row):
@@ -403,10 +472,11 @@ std::vector<at::Tensor> pipeline(const at::Tensor &ref, const at::Tensor &deg,
 // and no Python in between.  bank:
 // the resampler's (kernel, tap_lo, tap_hi, phase_lo, phase_hi, plan, info),
 // steps its (orig_step, new_step, width).
-std::vector<at::Tensor> pipeline_resampled(const at::Tensor &ref, const at::Tensor &deg,
-                                           const at::Tensor &table, double factor,
-                                           const std::vector<at::Tensor> &bank,
-                                           const std::vector<int64_t> &steps, int64_t n_out) {
+std::vector<at::Tensor> run_resampled(const at::Tensor &ref, const at::Tensor &deg,
+                                      const at::Tensor &table, double factor,
+                                      const std::vector<at::Tensor> &bank,
+                                      const std::vector<int64_t> &steps, int64_t n_out,
+                                      const Geometry &geo) {
     TORCH_CHECK(bank.size() == 7 && steps.size() == 3,
                 "pipeline_resampled: the resampler bank is 7 tensors and 3 steps");
     TORCH_CHECK(ref.is_cuda() && deg.is_cuda() && ref.scalar_type() == at::kFloat &&
@@ -418,7 +488,37 @@ std::vector<at::Tensor> pipeline_resampled(const at::Tensor &ref, const at::Tens
     const ResampleBank b = make_bank(ref.get_device(), bank[0], bank[1], bank[2], bank[3],
                                      bank[4], bank[5], bank[6], steps[0], steps[1], steps[2]);
     const variable_list r16 = ResamplePair::apply(ref, deg, n_out, b);
-    return pipeline(r16[0], r16[1], table, factor);
+    return run_pipeline(r16[0], r16[1], table, factor, geo);
+}
+
+std::vector<at::Tensor> pipeline_resampled(const at::Tensor &ref, const at::Tensor &deg,
+                                           const at::Tensor &table, double factor,
+                                           const std::vector<at::Tensor> &bank,
+                                           const std::vector<int64_t> &steps, int64_t n_out) {
+    return run_resampled(ref, deg, table, factor, bank, steps, n_out, Geometry{});
+}
+
+// pipeline() (bank empty) or pipeline_resampled() at another STFT geometry:
+// stft is the packed general STFT table of frames of n_fft samples every hop.
+// The stand-alone operators composed in Python nodes were bound by the host:
+// 16 pairs of 4 s with 400 of 512 taps every 160, both gradients, 37 launches
+// and 581 us a step; here 15 launches and 141 us.
+std::vector<at::Tensor> pipeline_general(const at::Tensor &ref, const at::Tensor &deg,
+                                         const at::Tensor &table, double factor,
+                                         const at::Tensor &stft, int64_t n_fft, int64_t hop,
+                                         const std::vector<at::Tensor> &bank,
+                                         const std::vector<int64_t> &steps, int64_t n_out) {
+    TORCH_CHECK(stft.is_cuda() && stft.get_device() == ref.get_device() &&
+                    stft.scalar_type() == at::kByte && stft.is_contiguous() &&
+                    stft.numel() == static_cast<int64_t>(pesq_stft_table_bytes()),
+                "pipeline_general: stft must be the packed STFT table (uint8, ",
+                pesq_stft_table_bytes(), " bytes) on the device of the signals");
+    TORCH_CHECK(n_fft >= 1 && n_fft <= std::numeric_limits<int>::max() && hop >= 1 &&
+                    hop <= std::numeric_limits<int>::max(),
+                "pipeline_general: invalid STFT geometry (n_fft ", n_fft, ", hop ", hop, ")");
+    const Geometry geo{stft, n_fft, hop};
+    if (bank.empty()) return run_pipeline(ref, deg, table, factor, geo);
+    return run_resampled(ref, deg, table, factor, bank, steps, n_out, geo);
 }
 
 // ---------------------------------------------------------------------------
@@ -793,6 +893,13 @@ PYBIND11_MODULE(_pesq_torch, m) {
           "signals resampled to 16 kHz",
           pybind11::arg("ref"), pybind11::arg("deg"), pybind11::arg("table"),
           pybind11::arg("factor"), pybind11::arg("bank"), pybind11::arg("steps"),
+          pybind11::arg("n_out"));
+    m.def("pipeline_general", &pipeline_general,
+          "(ref, deg, table, factor, stft, n_fft, hop, bank, steps, n_out) -> the same at another "
+          "STFT geometry, resampled to n_out samples first unless bank is empty",
+          pybind11::arg("ref"), pybind11::arg("deg"), pybind11::arg("table"),
+          pybind11::arg("factor"), pybind11::arg("stft"), pybind11::arg("n_fft"),
+          pybind11::arg("hop"), pybind11::arg("bank"), pybind11::arg("steps"),
           pybind11::arg("n_out"));
     m.def("resample", &resample,
           "(x, n_out, kernel, tap_lo, tap_hi, phase_lo, phase_hi, plan, info, orig_step, "

@@ -138,6 +138,15 @@ SIGNATURES = {
         _INT,
         [_P, _P, _P, _P, _I64, _I64, _P, ctypes.c_double, _INT, _P, _P, _P, _P, _P],
     ),
+    "pesq_pipeline_general_workspace": (_INT, [_I64, _I64, _INT, _INT, _INT, _SIZE_P, _SIZE_P]),
+    "pesq_pipeline_general_forward": (
+        _INT,
+        [_P, _P, _I64, _I64, _P, _P, _INT, _INT, ctypes.c_double, _INT, _P, _P, _P, _P, _P, _P],
+    ),
+    "pesq_pipeline_general_backward": (
+        _INT,
+        [_P, _P, _P, _P, _I64, _I64, _P, _P, _INT, _INT, ctypes.c_double, _INT, _P, _P, _P, _P, _P],
+    ),
     "pesq_pipeline_forward_stages": (
         _INT,
         [_P, _P, _I64, _I64, _P, ctypes.c_double, _INT, _P, _P, _P, _P, _P, ctypes.c_uint, _P],

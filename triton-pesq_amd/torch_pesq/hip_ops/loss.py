@@ -30,8 +30,8 @@ class PesqLossHip(PesqLoss):
         At the PESQ geometry the graphs are captured by the C++ extension
         (``GraphedLoss``: the forward and backward library calls, and the
         resampler's when the rate is not 16 kHz), whose autograd node replays
-        them with no Python in between.  Other STFT geometries, which run the
-        per stage operators, go through ``torch.cuda.make_graphed_callables``.
+        them with no Python in between.  Other STFT geometries go through
+        ``torch.cuda.make_graphed_callables``.
         """
 
         sample = tuple(t.detach().clone().requires_grad_(t.requires_grad) for t in (ref, deg))
@@ -63,7 +63,7 @@ class PesqLossHip(PesqLoss):
         ``deg`` to write into), ``replay()`` (on the current stream) and
         ``outputs()`` (the static loss and the gradients of ``ref`` and
         ``deg``, ``None`` where not requested), all bit exact with the eager
-        step.  The PESQ geometry only (the fused pipeline).
+        step.  The PESQ geometry only.
         """
 
         if self.general:

@@ -7,12 +7,12 @@ reference ``torch_pesq/loss.py:20-322`` (``raw``, ``mos``, ``forward``,
 the GPU through ``libpesq_hip.so``; CPU tensors are rejected with a
 ``RuntimeError``.
 
-``raw``/``mos``/``forward`` go through the fused pipeline (``csrc/pipeline.hip``)
-at the PESQ geometry (49 bands, ``n_fft = win_length = 512``,
-``hop_length = 256``).  Other STFT geometries (``n_fft``, ``win_length``,
-``hop_length``) run the reference's stage sequence (``triton_ops/loss.py:104-147``)
-on the stand-alone operators, with the general STFT kernels.  ``align_level``
-and ``preemphasize`` are the stand-alone per stage operators.
+``raw``/``mos``/``forward`` go through the fused pipeline (``csrc/pipeline.hip``).
+Its own STFT kernels are those of the PESQ geometry (49 bands, ``n_fft =
+win_length = 512``, ``hop_length = 256``); other geometries (``n_fft``,
+``win_length``, ``hop_length``) take the general STFT kernels in their place,
+with the rest of the pipeline unchanged.  ``align_level`` and ``preemphasize``
+are the stand-alone per stage operators.
 """
 
 import numpy as np
@@ -84,7 +84,7 @@ class PesqLoss(torch.nn.Module):
         from .hip_ops.iir import HipIIR
         from .hip_ops.pipeline import pack_model_table
         from .hip_ops.resample import HipResample
-        from .hip_ops.spectral import HipStftBark
+        from .hip_ops.spectral import HipStftBark, _general_table
 
         self.factor = factor
         self.source_sample_rate = int(sample_rate)
@@ -108,7 +108,8 @@ class PesqLoss(torch.nn.Module):
         self.power_iir = HipIIR(self.power_filter[0], self.power_filter[1])
         self.pre_iir = HipIIR(self.pre_filter[0], self.pre_filter[1])
 
-        # the per stage operators of the general geometry (triton_ops/loss.py:75-92)
+        # the stand-alone spectral and chain operators (triton_ops/loss.py:75-92)
+        self.geometry = (self.to_spec.n_fft, self.to_spec.hop_length)
         self.general = (nbarks, win_length, n_fft, hop_length) != (49, 512, 512, 256)
         self.spectral = HipStftBark(
             self.to_spec.window,
@@ -124,17 +125,28 @@ class PesqLoss(torch.nn.Module):
             float(self.fbank.total_width),
             SL,
         )
+        window, fbank = self.to_spec.window, self.fbank.fbank
         if self.general:
-            self.register_buffer("model_table", self.spectral.table, persistent=False)
-            return
+            # at any other window too: the general STFT's float64 transform
+            self.register_buffer(
+                "stft_table",
+                _general_table(
+                    self.spectral.window, self.spectral.starts, self.spectral.ends,
+                    self.fbank.pow_dens_correction.reshape(-1), self.to_spec.n_fft,
+                    self.to_spec.hop_length,
+                ),
+                persistent=False,
+            )
+            # the model table's own window and bands are not read
+            window, fbank = torch.zeros(512), torch.zeros(49, 256)
 
         table = pack_model_table(
             self.power_filter[0],
             self.power_filter[1],
             self.pre_filter[0],
             self.pre_filter[1],
-            self.to_spec.window,
-            self.fbank.fbank,
+            window,
+            fbank,
             self.fbank.pow_dens_correction,
             self.loudness.threshs,
             self.loudness.exp,
@@ -182,9 +194,6 @@ class PesqLoss(torch.nn.Module):
                 f"{ref.device}; move it with `.to(...)` first."
             )
 
-        if self.general:
-            return self._run_stages(ref, deg)
-
         resampled = self.source_sample_rate != 16000
         if resampled:
             if self.resampler.kernel.device != ref.device:
@@ -197,7 +206,8 @@ class PesqLoss(torch.nn.Module):
         else:
             length = ref.shape[1]
         padded = length + length % 256
-        frames = 1 + (padded - 512) // 256 if padded >= 512 else 0
+        n_fft, hop = self.geometry
+        frames = 1 + (padded - n_fft) // hop if padded >= n_fft else 0
         if length < 15:
             raise RuntimeError(
                 f"The edge ramp needs at least 15 samples at 16 kHz, got {length}."
@@ -212,53 +222,23 @@ class PesqLoss(torch.nn.Module):
                 "The loss treats `factor` as a constant, pass a Python float. A tensor "
                 "that requires a gradient would receive none."
             )
+        bank, steps = self.resampler.bank() if resampled else ([], [])
+        if self.general:
+            if ref.shape[0] == 0 and self.spectral.general:
+                raise RuntimeError("The general STFT kernels need at least one signal.")
+            return tuple(
+                _lib.torch_ext().pipeline_general(
+                    ref, deg, self.model_table, float(self.factor), self.stft_table, n_fft, hop,
+                    bank, steps, length,
+                )
+            )
         if resampled:
-            bank, steps = self.resampler.bank()
             return tuple(
                 _lib.torch_ext().pipeline_resampled(
                     ref, deg, self.model_table, float(self.factor), bank, steps, length
                 )
             )
         return tuple(_lib.torch_ext().pipeline(ref, deg, self.model_table, float(self.factor)))
-
-    def _run_stages(self, ref: torch.Tensor, deg: torch.Tensor):
-        """The stage sequence of ``PesqLossTriton.raw`` (``triton_ops/loss.py:104-147``).
-
-        Both signals share one peak and are stacked into one batch of twice
-        the size; resampling, level alignment, pre-emphasis, the ``N % 256``
-        padding, the STFT / Bark operator, the chain and the epilogue follow.
-        """
-
-        from .hip_ops.elementwise import peak_normalize, pesq_epilogue
-
-        if isinstance(self.factor, torch.Tensor) and self.factor.requires_grad:
-            raise RuntimeError(
-                "The loss treats `factor` as a constant, pass a Python float. A tensor "
-                "that requires a gradient would receive none."
-            )
-        batch = ref.shape[0]
-        signal = peak_normalize(ref, deg, stack=True)
-        if self.source_sample_rate != 16000:
-            signal = self.resampler(signal)
-        length = signal.shape[1]
-        if length < 15:
-            raise RuntimeError(
-                f"The edge ramp needs at least 15 samples at 16 kHz, got {length}."
-            )
-        padded = length + length % 256
-        n_fft, hop = self.to_spec.n_fft, self.to_spec.hop_length
-        frames = 1 + (padded - n_fft) // hop if padded >= n_fft else 0
-        if frames < 20:
-            raise ValueError(
-                "The PESQ chain needs at least 20 frames for the overlapping sums, "
-                f"got {frames}."
-            )
-        signal = self.align_level(signal)
-        signal = self.preemphasize(signal)
-        bark = self.spectral(signal, padded)
-        d_symm, d_asymm = self.chain(bark[:batch], bark[batch:])
-        mos, loss = pesq_epilogue(d_symm, d_asymm, float(self.factor))
-        return d_symm, d_asymm, mos, loss
 
     def raw(self, ref: torch.Tensor, deg: torch.Tensor):
         """Symmetric and asymmetric distances, both ``[batch]``."""
