@@ -608,3 +608,38 @@ def test_resample_plan_transposed_bank_is_the_adjoint(orig, new):
         got[i] = np.dot(adj[:, j][ok], g[m[ok]])
     # the oracle's bank is the float32 bank promoted: the same products
     np.testing.assert_allclose(got, want[0].numpy(), rtol=0, atol=1e-12 * np.abs(g).max())
+
+
+@pytest.mark.parametrize("kind", ["loss", "general loss", "iir", "cascade", "stft", "general stft", "chain"])
+def test_modules_saved_with_other_tables_load(kind):
+    """A pickled module whose packed tables another build laid out (here: cut
+    short) packs its own when it is loaded; one of this build keeps its bytes."""
+
+    import copy
+
+    from torch_pesq import PesqLossTriton
+    from torch_pesq.hip_ops.chain import HipPesqChain
+    from torch_pesq.hip_ops.iir import HipIIR
+    from torch_pesq.hip_ops.spectral import HipStftBark
+
+    loss = PesqLossTriton(0.5, sample_rate=16000, hop_length=160 if "general" in kind else 256)
+    module = {
+        "loss": lambda: loss,
+        "iir": lambda: loss.power_iir,
+        "cascade": lambda: HipIIR(*butter(8, [325, 3250], fs=16000, btype="band")),
+        # (these two keep their constants in float32)
+        "stft": lambda: HipStftBark(loss.to_spec.window, loss.fbank.fbank,
+                                    loss.fbank.pow_dens_correction.float(), *loss.geometry),
+        "chain": lambda: HipPesqChain(loss.chain.threshs, loss.chain.exp, loss.chain.width_bark,
+                                      loss.chain.total_width, loss.chain.sl),
+    }[kind.replace("general stft", "stft").replace("general loss", "loss")]()
+    names = [n for n in ("table", "model_table", "stft_table") if hasattr(module, n)]
+    want = {n: getattr(module, n).clone() for n in names}
+    old = copy.deepcopy(module)
+    assert all(torch.equal(getattr(old, n), want[n]) for n in names)
+    for n in names:
+        setattr(old, n, getattr(old, n)[:-64])
+    if kind == "general loss":
+        del old.stft_table, old.geometry
+    new = copy.deepcopy(old)
+    assert all(torch.equal(getattr(new, n), want[n]) for n in names)

@@ -117,6 +117,13 @@ class HipPesqChain(torch.nn.Module):
         self.register_buffer("table", _pack_chain(threshs, exps, widths, self.total_width,
                                                   self.sl), persistent=False)
 
+    def __setstate__(self, state):
+        # a module saved with another build of the library holds its table
+        super().__setstate__(state)
+        if self.table.numel() != _lib.library().pesq_model_table_bytes():
+            self.table = _pack_chain(self.threshs, self.exp, self.width_bark, self.total_width,
+                                     self.sl).to(self.table.device)
+
     def forward(self, ref_bark: torch.Tensor, deg_bark: torch.Tensor):
         """``(d_symm, d_asymm)``, both ``[batch]``."""
 

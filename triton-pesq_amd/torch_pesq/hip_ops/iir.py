@@ -458,11 +458,19 @@ class HipIIR(torch.nn.Module):
         self.padded = self.states
         self.c0 = real.c0
         self.section_coeffs = real.sections
-        if real.basis == "parallel":
-            table = _pack_table(sections_struct(real.c0, real.sections))
-        else:
-            table = _pack_cascade(real.sections)
-        self.register_buffer("table", table, persistent=False)
+        self.register_buffer("table", self._packed(), persistent=False)
+
+    def _packed(self) -> torch.Tensor:
+        if self.basis == "parallel":
+            return _pack_table(sections_struct(self.c0, self.section_coeffs))
+        return _pack_cascade(self.section_coeffs)
+
+    def __setstate__(self, state):
+        # a module saved with another build of the library holds its tables
+        super().__setstate__(state)
+        size = _lib.library().pesq_iir_table_bytes()
+        if self.table.numel() != size * (1 if self.basis == "parallel" else self.sections):
+            self.table = self._packed().to(self.table.device)
 
     def forward(self, signal: torch.Tensor) -> torch.Tensor:
         """Filter a ``[batch, sample]`` signal along the sample axis."""

@@ -188,15 +188,28 @@ class HipStftBark(torch.nn.Module):
         self.general = (n_fft, hop_length, self.nbarks) != _PESQ_GEOMETRY or bool(
             np.any(self.ends - self.starts > _MAX_BAND_BINS)
         )
-        if self.general:
-            table = _general_table(full, self.starts, self.ends, corr, n_fft, hop_length)
-        else:
-            ones = torch.ones(_lib.NBARKS, dtype=torch.float64)
-            table = pack_model_table(None, None, None, None, full, fbank, corr,
-                                     ones, ones, ones, 1.0, 0.0)
         self.register_buffer("window", full)
         self.register_buffer("correction", corr.detach().clone().float())
-        self.register_buffer("table", table, persistent=False)
+        self.register_buffer("table", self._packed(corr), persistent=False)
+
+    def _packed(self, corr) -> torch.Tensor:
+        if self.general:
+            return _general_table(self.window, self.starts, self.ends, corr, self.n_fft,
+                                  self.hop_length)
+        fbank = torch.zeros(_lib.NBARKS, _lib.NFFT // 2)
+        for band, (start, end) in enumerate(zip(self.starts, self.ends)):
+            fbank[band, start:end] = 1.0
+        ones = torch.ones(_lib.NBARKS, dtype=torch.float64)
+        return pack_model_table(None, None, None, None, self.window, fbank, corr,
+                                ones, ones, ones, 1.0, 0.0)
+
+    def __setstate__(self, state):
+        # a module saved with another build of the library holds its table
+        super().__setstate__(state)
+        lib = _lib.library()
+        size = lib.pesq_stft_table_bytes() if self.general else lib.pesq_model_table_bytes()
+        if self.table.numel() != size:
+            self.table = self._packed(self.correction).to(self.table.device)
 
     def forward(self, signal: torch.Tensor, n_padded: int = None) -> torch.Tensor:
         """Bark scaled power spectrogram ``[batch, frame, bark]`` of ``[batch, sample]``."""

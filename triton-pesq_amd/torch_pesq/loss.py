@@ -82,9 +82,8 @@ class PesqLoss(torch.nn.Module):
 
         from .hip_ops.chain import HipPesqChain
         from .hip_ops.iir import HipIIR
-        from .hip_ops.pipeline import pack_model_table
         from .hip_ops.resample import HipResample
-        from .hip_ops.spectral import HipStftBark, _general_table
+        from .hip_ops.spectral import HipStftBark
 
         self.factor = factor
         self.source_sample_rate = int(sample_rate)
@@ -109,7 +108,6 @@ class PesqLoss(torch.nn.Module):
         self.pre_iir = HipIIR(self.pre_filter[0], self.pre_filter[1])
 
         # the stand-alone spectral and chain operators (triton_ops/loss.py:75-92)
-        self.geometry = (self.to_spec.n_fft, self.to_spec.hop_length)
         self.general = (nbarks, win_length, n_fft, hop_length) != (49, 512, 512, 256)
         self.spectral = HipStftBark(
             self.to_spec.window,
@@ -125,18 +123,21 @@ class PesqLoss(torch.nn.Module):
             float(self.fbank.total_width),
             SL,
         )
+        self._pack_tables(None)
+
+    def _pack_tables(self, device):
+        from .hip_ops.pipeline import pack_model_table
+        from .hip_ops.spectral import _general_table
+
+        self.geometry = (self.to_spec.n_fft, self.to_spec.hop_length)
         window, fbank = self.to_spec.window, self.fbank.fbank
         if self.general:
             # at any other window too: the general STFT's float64 transform
-            self.register_buffer(
-                "stft_table",
-                _general_table(
-                    self.spectral.window, self.spectral.starts, self.spectral.ends,
-                    self.fbank.pow_dens_correction.reshape(-1), self.to_spec.n_fft,
-                    self.to_spec.hop_length,
-                ),
-                persistent=False,
+            stft_table = _general_table(
+                self.spectral.window, self.spectral.starts, self.spectral.ends,
+                self.fbank.pow_dens_correction.reshape(-1), *self.geometry,
             )
+            self.register_buffer("stft_table", stft_table.to(device), persistent=False)
             # the model table's own window and bands are not read
             window, fbank = torch.zeros(512), torch.zeros(49, 256)
 
@@ -154,7 +155,19 @@ class PesqLoss(torch.nn.Module):
             self.fbank.total_width,
             SL,
         )
-        self.register_buffer("model_table", table, persistent=False)
+        self.register_buffer("model_table", table.to(device), persistent=False)
+
+    def __setstate__(self, state):
+        # a module saved with another build of the library holds its tables
+        from . import _lib
+
+        super().__setstate__(state)
+        lib = _lib.library()
+        if self.model_table.numel() != lib.pesq_model_table_bytes() or (
+            self.general
+            and getattr(self, "stft_table", self.model_table).numel() != lib.pesq_stft_table_bytes()
+        ):
+            self._pack_tables(self.model_table.device)
 
     # -- stages -------------------------------------------------------------
 
