@@ -643,3 +643,44 @@ def test_modules_saved_with_other_tables_load(kind):
         del old.stft_table, old.geometry
     new = copy.deepcopy(old)
     assert all(torch.equal(getattr(new, n), want[n]) for n in names)
+
+
+@pytest.mark.parametrize("kind", ["loss", "general loss", "iir", "cascade"])
+def test_tables_of_the_same_size_but_another_layout_are_packed_again(kind):
+    """A module of a build whose tables are laid out otherwise at the very same
+    size: the size says nothing, the layout mark does.  Modules of builds
+    without marks count as such; their losses had no ``geometry``, and the
+    general ones no table of the pipeline."""
+
+    import pickle
+
+    from torch_pesq import PesqLossTriton
+
+    module = {
+        "loss": lambda: PesqLossTriton(0.5, sample_rate=16000),
+        "general loss": lambda: PesqLossTriton(0.5, sample_rate=16000, hop_length=160),
+        "iir": lambda: HipIIR(*butter(5, [325, 3250], fs=16000, btype="band")),
+        "cascade": lambda: HipIIR(*butter(8, [325, 3250], fs=16000, btype="band")),
+    }[kind]()
+    names = [n for n in ("table", "model_table", "stft_table") if hasattr(module, n)]
+    want = {n: getattr(module, n).clone() for n in names}
+    for unmarked in (False, True):
+        old = pickle.loads(pickle.dumps(module))
+        for part in {old, *(m for m in old.modules() if isinstance(m, HipIIR))}:
+            for n in {*names, "table"}:
+                if hasattr(part, n):
+                    setattr(part, n, getattr(part, n) ^ 0x55)
+            part.__dict__.pop("layout", None)
+            if not unmarked:
+                part.layout = "another"
+        if unmarked and "loss" in kind:
+            del old.geometry
+        if unmarked and kind == "general loss":
+            old.model_table = old.spectral.table
+            del old.stft_table
+        new = pickle.loads(pickle.dumps(old))
+        assert all(torch.equal(getattr(new, n), want[n]) for n in names)
+        if "loss" in kind:
+            assert new.geometry == module.geometry
+            assert torch.equal(new.power_iir.table, module.power_iir.table)
+            assert torch.equal(new.pre_iir.table, module.pre_iir.table)

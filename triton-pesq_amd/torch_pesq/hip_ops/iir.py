@@ -51,6 +51,7 @@ from scipy.signal import lfilter as _lfilter64, residuez, sosfilt, tf2sos
 
 from .. import _lib
 from ._common import check_input, require_hip
+from ._tables import table_layout
 
 __all__ = ["HipIIR", "Realisation", "realise", "parallel_sections", "sections_struct"]
 
@@ -458,6 +459,7 @@ class HipIIR(torch.nn.Module):
         self.padded = self.states
         self.c0 = real.c0
         self.section_coeffs = real.sections
+        self.layout = table_layout()
         self.register_buffer("table", self._packed(), persistent=False)
 
     def _packed(self) -> torch.Tensor:
@@ -469,7 +471,11 @@ class HipIIR(torch.nn.Module):
         # a module saved with another build of the library holds its tables
         super().__setstate__(state)
         size = _lib.library().pesq_iir_table_bytes()
-        if self.table.numel() != size * (1 if self.basis == "parallel" else self.sections):
+        if (
+            self.__dict__.get("layout") != table_layout()
+            or self.table.numel() != size * (1 if self.basis == "parallel" else self.sections)
+        ):
+            self.layout = table_layout()
             self.table = self._packed().to(self.table.device)
 
     def forward(self, signal: torch.Tensor) -> torch.Tensor:

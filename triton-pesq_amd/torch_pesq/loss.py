@@ -126,9 +126,11 @@ class PesqLoss(torch.nn.Module):
         self._pack_tables(None)
 
     def _pack_tables(self, device):
+        from .hip_ops._tables import table_layout
         from .hip_ops.pipeline import pack_model_table
         from .hip_ops.spectral import _general_table
 
+        self.layout = table_layout()
         self.geometry = (self.to_spec.n_fft, self.to_spec.hop_length)
         window, fbank = self.to_spec.window, self.fbank.fbank
         if self.general:
@@ -160,12 +162,17 @@ class PesqLoss(torch.nn.Module):
     def __setstate__(self, state):
         # a module saved with another build of the library holds its tables
         from . import _lib
+        from .hip_ops._tables import table_layout
 
         super().__setstate__(state)
         lib = _lib.library()
-        if self.model_table.numel() != lib.pesq_model_table_bytes() or (
-            self.general
-            and getattr(self, "stft_table", self.model_table).numel() != lib.pesq_stft_table_bytes()
+        if (
+            self.__dict__.get("layout") != table_layout()
+            or self.model_table.numel() != lib.pesq_model_table_bytes()
+            or (
+                self.general
+                and getattr(self, "stft_table", self.model_table).numel() != lib.pesq_stft_table_bytes()
+            )
         ):
             self._pack_tables(self.model_table.device)
 
