@@ -684,3 +684,61 @@ def test_tables_of_the_same_size_but_another_layout_are_packed_again(kind):
             assert new.geometry == module.geometry
             assert torch.equal(new.power_iir.table, module.power_iir.table)
             assert torch.equal(new.pre_iir.table, module.pre_iir.table)
+
+
+@pytest.mark.parametrize("kind", ["loss", "general loss", "stft", "general stft", "chain"])
+def test_tables_are_packed_again_from_the_values_of_the_first_time(kind):
+    """Another layout's tables are replaced by the bytes of a module built now:
+    from float64 constants where the module's buffers are float32 copies, and
+    after a cast that changed buffers and parameters."""
+
+    import pickle
+
+    from torch_pesq import PesqLossTriton
+    from torch_pesq.hip_ops.chain import HipPesqChain
+    from torch_pesq.hip_ops.spectral import HipStftBark
+
+    loss = PesqLossTriton(0.5, sample_rate=16000, hop_length=160 if "general" in kind else 256)
+    th, ex, width = loss.loudness.threshs, loss.loudness.exp, loss.fbank.width_bark
+    corr = loss.fbank.pow_dens_correction.detach().clone()
+    build = {
+        "loss": lambda: PesqLossTriton(0.5, sample_rate=16000, hop_length=loss.geometry[1]),
+        "stft": lambda: HipStftBark(torch.hann_window(512), loss.fbank.fbank, corr, *loss.geometry),
+        "chain": lambda: HipPesqChain(th, ex, width, float(loss.fbank.total_width)),
+    }[kind.replace("general ", "")]
+    module = build()
+    names = [n for n in ("table", "model_table", "stft_table") if hasattr(module, n)]
+    want = {n: getattr(module, n).clone() for n in names}
+    assert module.layout
+    for cast in (lambda m: m, lambda m: m.half(), lambda m: m.float()):
+        old = cast(pickle.loads(pickle.dumps(module)))
+        for n in names:
+            setattr(old, n, getattr(old, n) ^ 0x55)
+        old.layout = "another"
+        new = pickle.loads(pickle.dumps(old))
+        assert all(torch.equal(getattr(new, n), want[n]) for n in names)
+
+
+@pytest.mark.parametrize("hop", [160, 256])
+def test_bark_modules_of_builds_without_a_mark_keep_their_constants(hop):
+    """A general module of the first general table layout (twiddles of half the
+    length: 4096 bytes less before the fold's) gets its float64 correction from
+    the end of that table; the other family's table holds as it is."""
+
+    import pickle
+
+    from torch_pesq import PesqLossTriton
+    from torch_pesq.hip_ops.spectral import HipStftBark
+
+    loss = PesqLossTriton(0.5, sample_rate=16000)
+    corr = loss.fbank.pow_dens_correction.detach().clone()
+    module = HipStftBark(torch.hann_window(512), loss.fbank.fbank, corr, 512, hop)
+    want = module.table.clone()
+    old = pickle.loads(pickle.dumps(module))
+    old.__dict__.pop("layout", None)
+    old.__dict__.pop("constants", None)
+    if old.general:
+        head = 16 + 4096
+        old.table = torch.cat([old.table[:head], old.table[head + 4096:]])
+    new = pickle.loads(pickle.dumps(old))
+    assert torch.equal(new.table, want)

@@ -12,6 +12,7 @@ import torch
 
 from .. import _lib
 from ._common import check_input
+from ._tables import table_layout
 
 __all__ = ["HipPesqChain"]
 
@@ -114,15 +115,26 @@ class HipPesqChain(torch.nn.Module):
         self.register_buffer("width_bark", widths.float())
         # float32 buffers like the reference's (chain.py:1060-1076); the kernels
         # evaluate the chain in float64 from the float64 constants
-        self.register_buffer("table", _pack_chain(threshs, exps, widths, self.total_width,
-                                                  self.sl), persistent=False)
+        self.constants = tuple(v.detach().cpu().clone() for v in (threshs, exps, widths))
+        self.layout = table_layout()
+        self.register_buffer("table", self._packed(), persistent=False)
+
+    def _packed(self) -> torch.Tensor:
+        return _pack_chain(*self.constants, self.total_width, self.sl)
 
     def __setstate__(self, state):
         # a module saved with another build of the library holds its table
         super().__setstate__(state)
-        if self.table.numel() != _lib.library().pesq_model_table_bytes():
-            self.table = _pack_chain(self.threshs, self.exp, self.width_bark, self.total_width,
-                                     self.sl).to(self.table.device)
+        same_size = self.table.numel() == _lib.library().pesq_model_table_bytes()
+        if "layout" not in self.__dict__:
+            # builds without a mark kept float32 copies of the constants only; at
+            # this size their tables have the chain's where this build reads them
+            self.constants = tuple(v.detach().cpu().double()
+                                   for v in (self.threshs, self.exp, self.width_bark))
+            self.layout = table_layout() if same_size else None
+        if self.layout != table_layout() or not same_size:
+            self.layout = table_layout()
+            self.table = self._packed().to(self.table.device)
 
     def forward(self, ref_bark: torch.Tensor, deg_bark: torch.Tensor):
         """``(d_symm, d_asymm)``, both ``[batch]``."""

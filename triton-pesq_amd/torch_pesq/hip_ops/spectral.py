@@ -22,6 +22,7 @@ import torch
 
 from .. import _lib
 from ._common import check_input
+from ._tables import table_layout
 from .pipeline import pack_model_table
 
 __all__ = ["HipStftBark", "bark_segments"]
@@ -190,17 +191,21 @@ class HipStftBark(torch.nn.Module):
         )
         self.register_buffer("window", full)
         self.register_buffer("correction", corr.detach().clone().float())
-        self.register_buffer("table", self._packed(corr), persistent=False)
+        # float32 buffers; the tables hold the correction in float64
+        self.constants = (full.clone(), corr.detach().cpu().double().clone())
+        self.layout = table_layout()
+        self.register_buffer("table", self._packed(), persistent=False)
 
-    def _packed(self, corr) -> torch.Tensor:
+    def _packed(self) -> torch.Tensor:
+        window, corr = self.constants
         if self.general:
-            return _general_table(self.window, self.starts, self.ends, corr, self.n_fft,
+            return _general_table(window, self.starts, self.ends, corr, self.n_fft,
                                   self.hop_length)
         fbank = torch.zeros(_lib.NBARKS, _lib.NFFT // 2)
         for band, (start, end) in enumerate(zip(self.starts, self.ends)):
             fbank[band, start:end] = 1.0
         ones = torch.ones(_lib.NBARKS, dtype=torch.float64)
-        return pack_model_table(None, None, None, None, self.window, fbank, corr,
+        return pack_model_table(None, None, None, None, window, fbank, corr,
                                 ones, ones, ones, 1.0, 0.0)
 
     def __setstate__(self, state):
@@ -208,8 +213,21 @@ class HipStftBark(torch.nn.Module):
         super().__setstate__(state)
         lib = _lib.library()
         size = lib.pesq_stft_table_bytes() if self.general else lib.pesq_model_table_bytes()
-        if self.table.numel() != size:
-            self.table = self._packed(self.correction).to(self.table.device)
+        same_size = self.table.numel() == size
+        if "layout" not in self.__dict__:
+            # Builds without a mark kept a float32 copy of the correction only.
+            # Their general tables end with the float64 one; their model tables
+            # have, at this size, window, bands and correction where this build
+            # reads them.
+            corr = self.correction.detach().cpu().double()
+            if self.general:
+                tail = self.table[-8 * _MAX_BANDS :].cpu().numpy().view(np.float64)
+                corr = torch.from_numpy(tail[: self.nbarks].copy())
+            self.constants = (self.window.detach().cpu().float().clone(), corr)
+            self.layout = None if self.general or not same_size else table_layout()
+        if self.layout != table_layout() or not same_size:
+            self.layout = table_layout()
+            self.table = self._packed().to(self.table.device)
 
     def forward(self, signal: torch.Tensor, n_padded: int = None) -> torch.Tensor:
         """Bark scaled power spectrogram ``[batch, frame, bark]`` of ``[batch, sample]``."""

@@ -123,7 +123,28 @@ class PesqLoss(torch.nn.Module):
             float(self.fbank.total_width),
             SL,
         )
+        self.constants = self._table_constants()
         self._pack_tables(None)
+
+    def _table_constants(self):
+        """The values the tables are packed from, apart from the buffers and
+        parameters that hold them: a cast of the module (``half()``, ``float()``)
+        changes those and no table."""
+
+        return {
+            name: value.detach().cpu().clone()
+            for name, value in (
+                ("power", self.power_filter),
+                ("pre", self.pre_filter),
+                ("window", self.to_spec.window),
+                ("fbank", self.fbank.fbank),
+                ("corr", self.fbank.pow_dens_correction),
+                ("threshs", self.loudness.threshs),
+                ("exp", self.loudness.exp),
+                ("width", self.fbank.width_bark),
+                ("total_width", self.fbank.total_width),
+            )
+        }
 
     def _pack_tables(self, device):
         from .hip_ops._tables import table_layout
@@ -132,29 +153,28 @@ class PesqLoss(torch.nn.Module):
 
         self.layout = table_layout()
         self.geometry = (self.to_spec.n_fft, self.to_spec.hop_length)
-        window, fbank = self.to_spec.window, self.fbank.fbank
+        c = self.constants
+        window, fbank = c["window"], c["fbank"]
         if self.general:
             # at any other window too: the general STFT's float64 transform
             stft_table = _general_table(
-                self.spectral.window, self.spectral.starts, self.spectral.ends,
-                self.fbank.pow_dens_correction.reshape(-1), *self.geometry,
+                window, self.spectral.starts, self.spectral.ends, c["corr"].reshape(-1),
+                *self.geometry,
             )
             self.register_buffer("stft_table", stft_table.to(device), persistent=False)
             # the model table's own window and bands are not read
             window, fbank = torch.zeros(512), torch.zeros(49, 256)
 
         table = pack_model_table(
-            self.power_filter[0],
-            self.power_filter[1],
-            self.pre_filter[0],
-            self.pre_filter[1],
+            *c["power"],
+            *c["pre"],
             window,
             fbank,
-            self.fbank.pow_dens_correction,
-            self.loudness.threshs,
-            self.loudness.exp,
-            self.fbank.width_bark,
-            self.fbank.total_width,
+            c["corr"],
+            c["threshs"],
+            c["exp"],
+            c["width"],
+            c["total_width"],
             SL,
         )
         self.register_buffer("model_table", table.to(device), persistent=False)
@@ -174,6 +194,8 @@ class PesqLoss(torch.nn.Module):
                 and getattr(self, "stft_table", self.model_table).numel() != lib.pesq_stft_table_bytes()
             )
         ):
+            if "constants" not in self.__dict__:
+                self.constants = self._table_constants()
             self._pack_tables(self.model_table.device)
 
     # -- stages -------------------------------------------------------------
