@@ -19,6 +19,7 @@ Bounds, peak relative to the float64 output:
 """
 
 import math
+import warnings
 
 import numpy as np
 import pytest
@@ -264,3 +265,34 @@ def test_cascade_block_edges_for_any_section_count(sections, n):
         x64 = x.astype(np.float32).astype(np.float64)
         want = sosfilt(sos, x64[:, ::-1] if reverse else x64)
         assert peak_error(got, want[:, ::-1] if reverse else want) < 2e-7
+
+
+@pytest.mark.parametrize("rows, sections", [(3, 1), (400, 1), (3, 2), (3, 3)])
+@pytest.mark.parametrize("cutoff", [0.1, 0.3, 1.0, 5.0, 100.0])
+def test_high_pass_under_an_offset(rows, sections, cutoff):
+    """High passes far below the sampling rate over a signal with an offset ten
+    times its size, which the poles integrate and the zeros cancel: a second
+    order one alone (the scan kernels, in grids with and without lane states)
+    and followed by milder sections (the cascade), forward and reversed.
+    ``sosfilt`` in extended precision, to the float32 rounding of the output
+    (6e-8 of the peak, 2e-7 allowed; states of the poles alone, or transfer
+    powers squared in double, are 1e-6 to 2e-4 off at 1 Hz and below)."""
+
+    from scipy.signal import sosfilt
+
+    from torch_pesq.hip_ops import iir as iir_ops
+
+    high = butter(2, cutoff, fs=48000, btype="high", output="sos")
+    mild = np.array([[1.0, 0.4, 0.1, 1.0, -0.5, 0.2], [0.8, -0.2, 0.0, 1.0, 0.3, 0.0]])
+    sos = np.concatenate([high, mild])[:sections]
+    table = iir_ops._pack_cascade(sos).cuda()
+    x = torch.from_numpy(0.05 * noise(2, 70001, seed=5) + 0.5).float()
+    x64 = x.numpy().astype(np.longdouble)
+    for reverse in (False, True):
+        got = iir_ops._launch(x.repeat(rows, 1)[:rows].contiguous().cuda(), table, "cascade",
+                              sections, reverse)[-2:]
+        with warnings.catch_warnings():
+            warnings.simplefilter("ignore")  # (scipy means to drop extended precision)
+            want = sosfilt(sos.astype(np.longdouble), x64[:, ::-1] if reverse else x64)
+        want = (want[:, ::-1] if reverse else want).astype(np.float64)
+        assert peak_error(got, want if rows % 2 == 0 else want[::-1]) < 2e-7

@@ -17,75 +17,98 @@ void set_error(const char *fmt, ...) {
     va_end(args);
 }
 
-// A^n for the 2x2 companion block [[-a1, 1], [-a2, 0]], fp64
-static void mat_mul(const double *x, const double *y, double *out) {
-    const double r0 = x[0] * y[0] + x[1] * y[2];
-    const double r1 = x[0] * y[1] + x[1] * y[3];
-    const double r2 = x[2] * y[0] + x[3] * y[2];
-    const double r3 = x[2] * y[1] + x[3] * y[3];
+// out = x y, 2x2 row major
+template <class Real>
+static void mat_mul(const Real *x, const Real *y, Real *out) {
+    const Real r0 = x[0] * y[0] + x[1] * y[2];
+    const Real r1 = x[0] * y[1] + x[1] * y[3];
+    const Real r2 = x[2] * y[0] + x[3] * y[2];
+    const Real r3 = x[2] * y[1] + x[3] * y[3];
     out[0] = r0;
     out[1] = r1;
     out[2] = r2;
     out[3] = r3;
 }
 
-// Sections are stored with b2 = 0: a section with b2 != 0 and a2 != 0 is
-// rewritten as the direct term b2 / a2 plus the section
-// (b0 - b2 / a2) + (b1 - a1 b2 / a2) z^-1 over the same denominator, which is
-// the same transfer function.  `direct` accumulates the direct terms.
-// Section coefficients and scan powers of s into table sections first.. of t.
-// With fold_b2 (parallel form) a section's b2 becomes the direct term b2/a2
-// plus a section without z^-2 in its numerator; otherwise b2 is kept (the
-// full biquads of a cascade).
+static void store(const long double *m, double *out) {
+    for (int i = 0; i < 4; ++i) out[i] = static_cast<double>(m[i]);
+}
+
+// Coefficients, scan powers and chunk weights of s into table sections first..
+// of t, in one of the two forms of iir.hpp; `direct` accumulates the direct terms.
+//   kDirect      b2 = 0: a section with b2 != 0 becomes the direct term b2 / a2
+//                and the section (b0 - b2 / a2) + (b1 - a1 b2 / a2) z^-1 over the
+//                same denominator, which is the same transfer function
+//   kObserver    g1 = b1 - a1 b0 and g2 = b2 - a2 b0, each rounded once (the
+//                differences cancel for zeros near the poles), b0 in `direct`
+// parallel: a term of a parallel form, which has no FIR tail.
+enum class Form { kDirect, kObserver };
 static int fill_sections(IirTable &t, int first, const pesq_iir_sections &s, double &direct,
-                         bool fold_b2 = true) {
+                         Form form, bool parallel = true) {
     PESQ_CHECK_ARG(s.count >= 1 && first + s.count <= kMaxSections,
                    "an IIR filter needs 1..%d sections in total, got %d", kMaxSections,
                    first + s.count);
+    long double sum = direct;
     for (int k = 0; k < s.count; ++k) {
         const int q = first + k;
-        PESQ_CHECK_ARG(std::isfinite(s.b0[k]) && std::isfinite(s.b1[k]) && std::isfinite(s.b2[k]) &&
-                           std::isfinite(s.a1[k]) && std::isfinite(s.a2[k]),
+        const double b0 = s.b0[k], b1 = s.b1[k], b2 = s.b2[k], a1 = s.a1[k], a2 = s.a2[k];
+        PESQ_CHECK_ARG(std::isfinite(b0) && std::isfinite(b1) && std::isfinite(b2) &&
+                           std::isfinite(a1) && std::isfinite(a2),
                        "non finite IIR coefficient in section %d", k);
-        PESQ_CHECK_ARG(!fold_b2 || s.b2[k] == 0.0 || s.a2[k] != 0.0,
+        PESQ_CHECK_ARG(!parallel || b2 == 0.0 || a2 != 0.0,
                        "section %d has b2 != 0 over a first order denominator (an FIR tail)", k);
-        const double d = (!fold_b2 || s.b2[k] == 0.0) ? 0.0 : s.b2[k] / s.a2[k];
-        direct += d;
-        t.b0[q] = s.b0[k] - d;
-        t.b1[q] = s.b1[k] - s.a1[k] * d;
-        t.b2[q] = fold_b2 ? 0.0 : s.b2[k];
-        t.a1[q] = s.a1[k];
-        t.a2[q] = s.a2[k];
+        const bool observer = form == Form::kObserver;
+        if (observer) {
+            sum += b0;
+            t.b0[q] = 0.0;
+            t.b1[q] = std::fma(-a1, b0, b1);
+            t.b2[q] = std::fma(-a2, b0, b2);
+        } else {
+            const double d = b2 == 0.0 ? 0.0 : b2 / a2;
+            sum += d;
+            t.b0[q] = b0 - d;
+            t.b1[q] = b1 - a1 * d;
+            t.b2[q] = 0.0;
+        }
+        t.a1[q] = a1;
+        t.a2[q] = a2;
+        // The powers are formed in extended precision and rounded once: squared
+        // in double, those of poles close to 1 drift by many units (in observer
+        // form, a high pass at 1 Hz of 48 kHz over 70001 samples with an offset
+        // was 7.0e-6 of its peak off, 4.6e-8 now).
+        const long double a[4] = {-a1, observer ? 1.0 : -a2, observer ? -a2 : 1.0, 0.0};
+        const long double one[4] = {1.0L, 0.0L, 0.0L, 1.0L};
         // chunk transfer powers: level 0 = A^kChunk, level j = A^(kChunk 2^j)
-        const double a[4] = {-s.a1[k], -s.a2[k], 1.0, 0.0};
-        double p[4] = {1.0, 0.0, 0.0, 1.0};
-        for (int i = 0; i < kChunk; ++i) mat_mul(a, p, p);
+        long double pw[kLevels][4];
+        std::memcpy(pw[0], one, sizeof(one));
+        for (int i = 0; i < kChunk; ++i) mat_mul(a, pw[0], pw[0]);
         for (int level = 0; level < kLevels; ++level) {
-            std::memcpy(t.pw[level][q], p, sizeof(p));
-            mat_mul(p, p, p);
+            if (level > 0) mat_mul(pw[level - 1], pw[level - 1], pw[level]);
+            store(pw[level], t.pw[level][q]);
         }
-        // chunk end state weights: the impulse response of 1 / (1 + a1 z^-1 + a2 z^-2)
+        // chunk end state weights: z1 of A^m (g1, g2), of A^m (1, 0)
+        long double z[2] = {observer ? t.b1[q] : 1.0, observer ? t.b2[q] : 0.0};
         for (int m = 0; m < kChunk; ++m) {
-            t.fir[q][m] = (m == 0 ? 1.0 : -s.a1[k] * t.fir[q][m - 1]) -
-                          (m >= 2 ? s.a2[k] * t.fir[q][m - 2] : 0.0);
+            t.fir[q][m] = static_cast<double>(z[0]);
+            const long double z1 = a[0] * z[0] + a[1] * z[1];
+            z[1] = a[2] * z[0];
+            z[0] = z1;
         }
+        long double m[4];
         // block pair powers M^(2 i), M = A^kSpan (level kLevelBlock)
-        {
-            double m[4] = {1.0, 0.0, 0.0, 1.0};
-            for (int i = 0; i < kWave; ++i) {
-                std::memcpy(t.blk_pw2[i][q], m, sizeof(m));
-                mat_mul(t.pw[kLevelBlock + 1][q], m, m);
-            }
+        std::memcpy(m, one, sizeof(one));
+        for (int i = 0; i < kWave; ++i) {
+            store(m, t.blk_pw2[i][q]);
+            mat_mul(pw[kLevelBlock + 1], m, m);
         }
-        // lane start powers A^(kChunk lane): product of the levels of the set bits
+        // lane start powers A^(kChunk lane)
+        std::memcpy(m, one, sizeof(one));
         for (int lane = 0; lane < kWave; ++lane) {
-            double m[4] = {1.0, 0.0, 0.0, 1.0};
-            for (int level = 0; level < kLevelBlock; ++level) {
-                if (lane & (1 << level)) mat_mul(t.pw[level][q], m, m);
-            }
-            std::memcpy(t.lane_pw[q][lane], m, sizeof(m));
+            store(m, t.lane_pw[q][lane]);
+            mat_mul(pw[0], m, m);
         }
     }
+    direct = static_cast<double>(sum);
     return PESQ_OK;
 }
 
@@ -99,10 +122,9 @@ static void cascade_transfer(IirTable *tables, int sections) {
         for (int k = 0; k < sections; ++k) {
             const IirTable &t = tables[k];
             const long double u = j == 2 * k ? 1.0L : 0.0L, v = j == 2 * k + 1 ? 1.0L : 0.0L;
-            const long double w = x - t.a1[0] * u - t.a2[0] * v;
-            m[size_t(2 * k) * n + j] = w;
-            m[size_t(2 * k + 1) * n + j] = u;
-            x = t.b0[0] * w + t.b1[0] * u + t.b2[0] * v;
+            m[size_t(2 * k) * n + j] = t.b1[0] * x - t.a1[0] * u + v;
+            m[size_t(2 * k + 1) * n + j] = t.b2[0] * x - t.a2[0] * u;
+            x = t.c0a * x + u;
         }
     }
     for (int span = 1; span < kSegmentSpan; span *= 2) {
@@ -123,16 +145,17 @@ static void cascade_transfer(IirTable *tables, int sections) {
     }
 }
 
-static int pack_iir(IirTable &t, const pesq_iir_sections *a, const pesq_iir_sections *b) {
+static int pack_iir(IirTable &t, const pesq_iir_sections *a, const pesq_iir_sections *b,
+                    Form form) {
     std::memset(&t, 0, sizeof(t));
     PESQ_CHECK_ARG(a != nullptr, "null filter");
     t.na = a->count;
     t.nb = b ? b->count : 0;
     t.c0a = a->c0;
     t.c0b = b ? b->c0 : 0.0;
-    if (int st = fill_sections(t, 0, *a, t.c0a)) return st;
+    if (int st = fill_sections(t, 0, *a, t.c0a, form)) return st;
     if (b) {
-        if (int st = fill_sections(t, a->count, *b, t.c0b)) return st;
+        if (int st = fill_sections(t, a->count, *b, t.c0b, form)) return st;
     }
     return PESQ_OK;
 }
@@ -150,7 +173,7 @@ extern "C" size_t pesq_iir_table_bytes(void) { return sizeof(IirTable); }
 extern "C" int pesq_iir_table_pack(const pesq_iir_sections *filter, void *out) {
     PESQ_CHECK_ARG(out != nullptr, "null output buffer");
     IirTable t;
-    if (int st = pack_iir(t, filter, nullptr)) return st;
+    if (int st = pack_iir(t, filter, nullptr, Form::kObserver)) return st;
     std::memcpy(out, &t, sizeof(t));
     return PESQ_OK;
 }
@@ -174,7 +197,7 @@ extern "C" int pesq_iir_cascade_pack(const double *sos, int sections, void *out)
         IirTable t;
         std::memset(&t, 0, sizeof(t));
         t.na = 1;
-        if (int st = fill_sections(t, 0, one, t.c0a, false)) return st;
+        if (int st = fill_sections(t, 0, one, t.c0a, Form::kObserver, false)) return st;
         std::memcpy(&tables[k], &t, sizeof(t));
     }
     cascade_transfer(tables, sections);
@@ -225,7 +248,7 @@ extern "C" int pesq_model_table_pack(const pesq_model_constants *c, void *out) {
     ModelTable *t = new ModelTable;
     std::memset(t, 0, sizeof(*t));
     if (!no_filters) {
-        const int st = pack_iir(t->iir, &c->power_filter, &c->pre_filter);
+        const int st = pack_iir(t->iir, &c->power_filter, &c->pre_filter, Form::kDirect);
         if (st) {
             delete t;
             return st;

@@ -1,17 +1,36 @@
 // Chunked parallel scan of a bank of parallel second order sections, fp64 state.
 //
-// A filter is realised in parallel form, y = c0 x + sum_k y_k, where section k
-// is a direct form II biquad with b2 = 0 (the form partial fractions give; the
-// table packing folds any b2 into the direct term)
-//     w    = x - a1 z1 - a2 z2
-//     y_k  = b0 w + b1 z1
-//     z1', z2' = w, z1
-// i.e. the state z = (z1, z2) evolves as z' = A_k z + (x, 0) with
-// A_k = [[-a1, -a2], [1, 0]].  Because every A_k is 2x2 and the sections are
-// independent, the chunk transfer matrices are block diagonal (4 numbers per
-// section) and the scan combine costs 4 FMAs per section.  A sample costs 4
-// FMAs per section, of which one (w from z1) is on the serial chain; the
-// transposed form, run before, took 5 operations with two on the chain.
+// A filter is realised in parallel form, y = c0 x + sum_k y_k, or as a cascade
+// of sections.  Section k has the denominator 1 + a1 z^-1 + a2 z^-2 and two
+// states, in one of two forms (Coeffs):
+//   direct form II, the pipeline's two filters (b2 = 0, the form partial
+//   fractions give; the table packing folds any b2 into the direct term):
+//       w    = x - a1 z1 - a2 z2
+//       y_k  = b0 w + b1 z1
+//       z1', z2' = w, z1
+//     i.e. z' = A z + (x, 0), A = [[-a1, -a2], [1, 0]]: 4 FMAs a sample;
+//   observer form, the stand-alone filters (SingleMode, BiquadMode, the
+//   cascade), b1 and b2 holding g1 = b1 - a1 b0 and g2 = b2 - a2 b0:
+//       y_k  = b0 x + z1
+//       z1'  = g1 x - a1 z1 + z2
+//       z2'  = g2 x - a2 z1
+//     i.e. z' = A z + (g1, g2) x, A = [[-a1, 1], [-a2, 0]]: 5 operations a
+//     sample.
+// In both one FMA (from z1) is on the serial chain.  The states of direct form
+// II are those of 1 / (1 + a1 z^-1 + a2 z^-2), which for poles at an angle t
+// of 1 grow with 1 / t^2 of a constant input, and a numerator with zeros at 1
+// cancels them; the observer form's are of the size of the output.  With them
+// and the transfer powers formed in extended precision a second order high pass
+// at 1 Hz of 48 kHz, under an offset ten times the signal, is 4.6e-8 of its
+// peak off (1.8e-6 before, 1.6e-5 in grids without lane states), at 0.1 Hz
+// 4.4e-8 and 1.1e-7 (2.0e-5 and 2.4e-4): the rounding of the float32 output.  8
+// sections over 24 rows of 160001 samples take 56 instead of 52 us a direction
+// for it, 5 parallel ones 29.8 instead of 27.0.  The pipeline's filters, 325 Hz to
+// 3.25 kHz and a pre-emphasis with poles of radius 0.973, keep to 4e-14 in direct
+// form.
+// Because every A_k is 2x2 and the sections are independent, the chunk transfer
+// matrices are block diagonal (4 numbers per section) and the scan combine
+// costs 4 FMAs per section.
 //
 // Geometry.  A lane runs the recursion of all sections over a chunk of kChunk
 // consecutive samples (the sections are independent chains, so the lane has
@@ -78,24 +97,24 @@ constexpr int kOutputWaves = PESQ_OUTPUT_WAVES;
 #define PESQ_SEGMENT_MIN 2
 #endif
 constexpr int kMaxSections = PESQ_IIR_MAX_SECTIONS;
-// power levels: A^(kChunk 2^j); j = 0..5 in-wave, 6 = one block, 6..11 the
-// block level scan over 64 blocks
+// power levels: A^(kChunk 2^j); j = 0..5 in-wave, 6 = one block, 6 and up the
+// block level scan (iir_prefix_kernel: rows of up to 2^18 blocks)
 constexpr int kLevelBlock = 6;
-constexpr int kLevels = 14;
+constexpr int kLevels = 24;
 static_assert(kSpan == kChunk << kLevelBlock, "a block is 2^6 chunks");
 
 struct IirTable {
     int32_t na, nb;      // sections of filter A, then of filter B
-    double c0a, c0b;     // direct feed through of A and B
-    // b2 = 0 in a parallel form table (folded by the packing); kept in the
-    // per section tables of a cascade
+    // direct feed through of A and B; in observer form the sections' b0 too
+    double c0a, c0b;
+    // direct form II: b2 = 0 (folded by the packing); observer form: b0 = 0 (in
+    // c0a), b1 = g1, b2 = g2
     double b0[kMaxSections], b1[kMaxSections], b2[kMaxSections];
     double a1[kMaxSections], a2[kMaxSections];
     double pw[kLevels][kMaxSections][4];     // A_k^(kChunk 2^j), row major 2x2
     double lane_pw[kMaxSections][kWave][4];  // A_k^(kChunk lane), lane start powers
-    // h_m, m < kChunk: the impulse response of 1 / (1 + a1 z^-1 + a2 z^-2),
-    // the weight of the sample m before the last one in z1 after the chunk
-    // from a zero state (z2 is z1 one sample earlier)
+    // h_m, m < kChunk: the weight of the sample m before the last one in z1
+    // after the chunk from a zero state (chunk_end_state)
     double fir[kMaxSections][kChunk];
     // M^(2 i), M = A_k^kSpan the block transfer: the weight of the block pair
     // (M e_j + e_j+1) 2 i + 2 blocks before a block (block_start_reduce)
@@ -225,10 +244,9 @@ struct Bank {
 // after barriers and stores
 using ConstDoubles = const __attribute__((address_space(4))) double *;
 
-// Coefficients of NS sections starting at section S0.  With kB2 the sections
-// are full biquads (z2' = b2 x - a2 y_k, the cascade passes); without it b2 is
-// 0 (the parallel form, whose table packing folds b2 into the direct term).
-template <int S0, int NS, bool kB2 = false>
+// Coefficients of NS sections starting at section S0, in observer form or in
+// direct form II (above).
+template <int S0, int NS, bool kObserver = false>
 struct Coeffs {
     double b0[NS > 0 ? NS : 1], b1[NS > 0 ? NS : 1], b2[NS > 0 ? NS : 1];
     double a1[NS > 0 ? NS : 1], a2[NS > 0 ? NS : 1];
@@ -237,9 +255,9 @@ struct Coeffs {
     __device__ __forceinline__ void load(const IirTable &t, double direct) {
 #pragma unroll
         for (int k = 0; k < NS; ++k) {
-            b0[k] = t.b0[S0 + k];
+            b0[k] = kObserver ? 0.0 : t.b0[S0 + k];
             b1[k] = t.b1[S0 + k];
-            b2[k] = kB2 ? t.b2[S0 + k] : 0.0;
+            b2[k] = kObserver ? t.b2[S0 + k] : 0.0;
             a1[k] = t.a1[S0 + k];
             a2[k] = t.a2[S0 + k];
         }
@@ -248,26 +266,36 @@ struct Coeffs {
 
     __device__ __forceinline__ void load_scalar(const IirTable &t, const double &direct) {
         const ConstDoubles tb0 = (ConstDoubles)t.b0, tb1 = (ConstDoubles)t.b1;
+        const ConstDoubles tb2 = (ConstDoubles)t.b2;
         const ConstDoubles ta1 = (ConstDoubles)t.a1, ta2 = (ConstDoubles)t.a2;
 #pragma unroll
         for (int k = 0; k < NS; ++k) {
-            b0[k] = tb0[S0 + k];
+            b0[k] = kObserver ? 0.0 : tb0[S0 + k];
             b1[k] = tb1[S0 + k];
-            b2[k] = 0.0;
+            b2[k] = kObserver ? tb2[S0 + k] : 0.0;
             a1[k] = ta1[S0 + k];
             a2[k] = ta2[S0 + k];
         }
         c0 = *(ConstDoubles)&direct;
     }
-    // one section's step: its output added to y
+    // the state of section k after x
+    __device__ __forceinline__ void next(int k, Bank<NS> &s, double x) const {
+        const double u = s.u[k];
+        if constexpr (kObserver) {
+            s.u[k] = fma(-a1[k], u, fma(b1[k], x, s.v[k]));
+            s.v[k] = fma(-a2[k], u, b2[k] * x);
+        } else {
+            s.u[k] = fma(-a1[k], u, fma(-a2[k], s.v[k], x));
+            s.v[k] = u;
+        }
+    }
+    // one section's step: its output (in observer form without b0 x, which is
+    // in c0) added to y
     __device__ __forceinline__ double section(int k, Bank<NS> &s, double x, double y) const {
-        const double w = fma(-a1[k], s.u[k], fma(-a2[k], s.v[k], x));
-        double out = fma(b1[k], s.u[k], y);
-        if constexpr (kB2) out = fma(b2[k], s.v[k], out);
-        out = fma(b0[k], w, out);
-        s.v[k] = s.u[k];
-        s.u[k] = w;
-        return out;
+        const double u = s.u[k];
+        next(k, s, x);
+        if constexpr (kObserver) return y + u;
+        return fma(b0[k], s.u[k], fma(b1[k], u, y));
     }
     // one time step: consumes x, advances the state, returns c0 x + sum_k y_k
     __device__ __forceinline__ double step(Bank<NS> &s, double x) const {
@@ -285,11 +313,7 @@ struct Coeffs {
     // the states alone
     __device__ __forceinline__ void advance(Bank<NS> &s, double x) const {
 #pragma unroll
-        for (int k = 0; k < NS; ++k) {
-            const double w = fma(-a1[k], s.u[k], fma(-a2[k], s.v[k], x));
-            s.v[k] = s.u[k];
-            s.u[k] = w;
-        }
+        for (int k = 0; k < NS; ++k) next(k, s, x);
     }
 };
 
@@ -529,7 +553,8 @@ struct BankPair {
 //   Mode::kOutputs                outputs per sample (1 or 2)
 //   Mode::In, Mode::Out           element types of the raw inputs and the
 //                                 outputs in memory (float or double)
-//   Mode::kB2                     full biquad sections (b2 read from the table)
+//   Mode::kObserver               sections in observer form (the table's too),
+//                                 else in direct form II
 //   Mode::kReverse                process the time axis back to front
 //   Mode::kAccumulates            the output pass reduces a per block sum
 //   Mode::kSegments               large grids may run segmented (SegmentPlan),
@@ -660,15 +685,21 @@ __device__ __forceinline__ void element_inputs(const Mode &m,
 
 // state of NS sections from S0 after the chunk, from a zero state, as the
 // weighted sums of the chunk's inputs x[0 .. kChunk - 1]: independent fused
-// multiply-adds instead of the recursion's chain (z2 has the weights of z1 one
-// sample later; the weight of the last sample, h_0, is 1)
-template <int S0, int NS>
+// multiply-adds instead of the recursion's chain.  Direct form II: h is the
+// impulse response of 1 / (1 + a1 z^-1 + a2 z^-2), h_0 = 1, and z2 is z1 one
+// sample earlier.  Observer form: z2 is g2 x of the last sample less a2 times
+// z1 one sample earlier.
+template <int S0, int NS, bool kObserver>
 __device__ __forceinline__ void chunk_end_state(const IirTable &t, const double (&x)[kChunk],
                                                 Bank<NS> &s) {
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
         double u = x[kChunk - 1];
         double v = x[kChunk - 2];
+        if constexpr (kObserver) {
+            u *= t.fir[S0 + k][0];
+            v *= t.fir[S0 + k][0];
+        }
 #pragma unroll
         for (int m = 1; m < kChunk; ++m) {
             const double h = t.fir[S0 + k][m];
@@ -676,7 +707,7 @@ __device__ __forceinline__ void chunk_end_state(const IirTable &t, const double 
             if (m < kChunk - 1) v = fma(h, x[kChunk - 2 - m], v);
         }
         s.u[k] = u;
-        s.v[k] = v;
+        s.v[k] = kObserver ? fma(-t.a2[S0 + k], v, t.b2[S0 + k] * x[kChunk - 1]) : v;
     }
 }
 
@@ -689,8 +720,8 @@ __device__ __forceinline__ void chunk_end_state(const IirTable &t, const double 
 // with the ramp weights and bounds of element_inputs.
 template <bool kGeneral, bool kWeighted, int NA, int NB, class Mode, int kBase = 0>
 __device__ __forceinline__ void zero_run(const Mode &m, const IirTable &t,
-                                         const Coeffs<kBase, NA, Mode::kB2> &ca,
-                                         const Coeffs<kBase + NA, NB, Mode::kB2> &cb,
+                                         const Coeffs<kBase, NA, Mode::kObserver> &ca,
+                                         const Coeffs<kBase + NA, NB, Mode::kObserver> &cb,
                                          const typename Mode::In (&in)[kChunk][Mode::kInputs],
                                          int64_t j0,
                                          int64_t len, BankPair<NA, NB, kBase> &s) {
@@ -709,15 +740,15 @@ __device__ __forceinline__ void zero_run(const Mode &m, const IirTable &t,
             double w;
             element_inputs<false>(m, in[i], j0 + i, len, w, xa[i], xb[i]);
         }
-        if constexpr (NA > 0) chunk_end_state<kBase, NA>(t, xa, s.a);
-        if constexpr (NB > 0) chunk_end_state<kBase + NA, NB>(t, xb, s.b);
+        if constexpr (NA > 0) chunk_end_state<kBase, NA, Mode::kObserver>(t, xa, s.a);
+        if constexpr (NB > 0) chunk_end_state<kBase + NA, NB, Mode::kObserver>(t, xb, s.b);
     }
 }
 
 // run from the true start state s, outputs into out[][i]
 template <bool kGeneral, int NA, int NB, class Mode>
-__device__ __forceinline__ void output_run(const Mode &m, const Coeffs<0, NA, Mode::kB2> &ca,
-                                           const Coeffs<NA, NB, Mode::kB2> &cb,
+__device__ __forceinline__ void output_run(const Mode &m, const Coeffs<0, NA, Mode::kObserver> &ca,
+                                           const Coeffs<NA, NB, Mode::kObserver> &cb,
                                            const typename Mode::In (&in)[kChunk][Mode::kInputs],
                                            int64_t j0, int64_t len, const double *sh,
                                            BankPair<NA, NB> &s,
@@ -783,8 +814,8 @@ __device__ __forceinline__ void aggregate_block(const Mode &m, const IirTable &t
     constexpr int NS = NA + NB;
     static_assert(kBase + NS <= kLayout, "sections inside the layout");
     const int64_t j0 = int64_t(blk) * kSpan + int64_t(lane) * kChunk;
-    Coeffs<kBase, NA, Mode::kB2> ca;
-    Coeffs<kBase + NA, NB, Mode::kB2> cb;
+    Coeffs<kBase, NA, Mode::kObserver> ca;
+    Coeffs<kBase + NA, NB, Mode::kObserver> cb;
     ca.load(t, t.c0a);
     cb.load(t, t.c0b);
 
@@ -840,8 +871,8 @@ __global__ void __launch_bounds__(kWave)
         static_assert(kBase == 0 && kLayout == NA + NB, "all sections without lane states");
         constexpr int NS = NA + NB;
         const int64_t j0 = int64_t(blk) * kSpan + int64_t(lane) * kChunk;
-        Coeffs<0, NA, Mode::kB2> ca;
-        Coeffs<NA, NB, Mode::kB2> cb;
+        Coeffs<0, NA, Mode::kObserver> ca;
+        Coeffs<NA, NB, Mode::kObserver> cb;
         ca.load(t, t.c0a);
         cb.load(t, t.c0b);
         typename Mode::In in[kChunk][Mode::kInputs];
@@ -896,13 +927,16 @@ __global__ void __launch_bounds__(kWaves * kWave)
 // Exclusive scan of the block aggregates, one (row, section) sequence per
 // wavefront; aggr[b] is replaced by the state at the start of block b
 // (s_{b+1} = M s_b + e_b, M = A^1024 the block transfer, e_b the aggregate).
-// Lane l owns the per = ceil(nblk / 64) consecutive blocks l per .. l per +
-// per - 1: it runs them from a zero start (its chunk total), a Kogge-Stone
-// scan over the lanes with the chunk transfer P = M^per and its squares gives
-// every chunk's start state, and the lane runs its blocks again from there,
-// storing each block's start.  The serial depth is 2 per + 6 steps (a scan
-// over groups of 64 blocks with a carry between them waits out a memory round
-// trip per group: 14.4 us per pass at c4, 938 blocks per row).
+// Lane l owns the per (a power of two, at least nblk / 64) consecutive blocks
+// l per .. l per + per - 1: it runs them from a zero start (its chunk total), a
+// Kogge-Stone scan over the lanes with the chunk transfer M^per and its squares
+// gives every chunk's start state, and the lane runs its blocks again from
+// there, storing each block's start.  The powers are the table's levels, formed
+// in extended precision: squared here in double they lost a high pass at 0.3 Hz
+// of 48 kHz, over rows of 69 blocks with an offset, 1.8e-5 of its peak.  The
+// serial depth is 2 per + 6 steps (a scan over groups of 64 blocks with a carry
+// between them waits out a memory round trip per group: 14.4 us per pass at c4,
+// 938 blocks per row).
 constexpr int kPrefixWaves = 4;
 constexpr int kPrefixHeld = 16;  // aggregates a lane keeps in registers
 
@@ -942,8 +976,11 @@ __global__ void __launch_bounds__(kWave *kPrefixWaves)
         }
         return;
     }
-    const int per = (nblk + kWave - 1) / kWave;
-    const int j0 = lane * per;
+    int level = kLevelBlock;  // of M^per
+    while ((int64_t(kWave) << (level - kLevelBlock)) < nblk) ++level;
+    const int per = 1 << (level - kLevelBlock);
+    const int64_t lo = int64_t(lane) * per;
+    const int j0 = lo < nblk ? static_cast<int>(lo) : nblk;
     const int j1 = j0 + per < nblk ? j0 + per : nblk;
     // the chunk's first kPrefixHeld aggregates stay in registers for both
     // runs (one memory round trip for chunks of up to kPrefixHeld blocks)
@@ -972,22 +1009,22 @@ __global__ void __launch_bounds__(kWave *kPrefixWaves)
         tu = u;
         tv = v;
     }
-    // P = M^per, square and multiply
-    Mat2 q{1.0, 0.0, 0.0, 1.0}, sq = m;
-    for (int e = per; e != 0; e >>= 1) {
-        if (e & 1) q = mat2_mul(q, sq);
-        sq = mat2_mul(sq, sq);
-    }
-    // inclusive scan of the chunk ends over the lanes, level j with P^(2^j)
+    // inclusive scan of the chunk ends over the lanes, step j with M^(per 2^j)
+    Mat2 q = m;
 #pragma unroll
     for (int j = 0; j < 6; ++j) {
+        if (level + j < kLevels) {
+            const double *p = t.pw[level + j][k];
+            q = {p[0], p[1], p[2], p[3]};
+        } else {  // (rows past 2^18 blocks)
+            q = mat2_mul(q, q);
+        }
         const int d = 1 << j;
         const double ou = shfl_up(tu, d), ov = shfl_up(tv, d);
         if (lane >= d) {
             tu = fma(q.a, ou, fma(q.b, ov, tu));
             tv = fma(q.c, ou, fma(q.d, ov, tv));
         }
-        q = mat2_mul(q, q);
     }
     // the lane's start state is the end state of the chunks before it
     double su = shfl_up(tu, 1), sv = shfl_up(tv, 1);
@@ -1268,9 +1305,9 @@ __device__ __forceinline__ void output_segment(const Mode &m, const IirTable &t,
                                                const SegmentPlan &seg, int64_t nseg) {
     constexpr int NS = NA + NB;
     constexpr bool kRev = Mode::kReverse;
-    static_assert(!Mode::kB2 && std::is_same<typename Mode::In, float>::value &&
+    static_assert(!Mode::kObserver && std::is_same<typename Mode::In, float>::value &&
                       std::is_same<typename Mode::Out, float>::value,
-                  "float rows, parallel form");
+                  "float rows, direct form II");
     __shared__ __attribute__((aligned(16))) float stages[kSegmentWaves][Mode::kInputs * kStageFloats];
     __shared__ __attribute__((aligned(16))) double carry[kCarryPowers * carry_stride<NS>()];
     const int wave = wave_index();
@@ -1477,8 +1514,8 @@ __global__ void __launch_bounds__(Mode::kSegments && !kLaneStates ? kSegmentWave
         // the previous blocks (weighted sums), v = sum_w M^(w - 1) e_(blk - w)
         // per lane (oldest block first), carried to the block end by
         // A^(kChunk (63 - lane)) and summed over the lanes in LDS
-        Coeffs<NA, 0, Mode::kB2> none;
-        Coeffs<NA, NB, Mode::kB2> wb;
+        Coeffs<NA, 0, Mode::kObserver> none;
+        Coeffs<NA, NB, Mode::kObserver> wb;
         wb.load(t2, t2.c0b);
         const double *mk = t2.pw[kLevelBlock][NA];
         double vu = 0.0, vv = 0.0;
@@ -1517,8 +1554,8 @@ __global__ void __launch_bounds__(Mode::kSegments && !kLaneStates ? kSegmentWave
     }
     if constexpr (!kLaneStates) {
         // the in-block start states again: zero state run, scan, shift by a lane
-        Coeffs<0, NA, Mode::kB2> za;
-        Coeffs<NA, NB, Mode::kB2> zb;
+        Coeffs<0, NA, Mode::kObserver> za;
+        Coeffs<NA, NB, Mode::kObserver> zb;
         za.load(t2, t2.c0a);
         zb.load(t2, t2.c0b);
         s.zero();
@@ -1545,8 +1582,8 @@ __global__ void __launch_bounds__(Mode::kSegments && !kLaneStates ? kSegmentWave
     }
 
     // run from the true start state
-    Coeffs<0, NA, Mode::kB2> ca;
-    Coeffs<NA, NB, Mode::kB2> cb;
+    Coeffs<0, NA, Mode::kObserver> ca;
+    Coeffs<NA, NB, Mode::kObserver> cb;
     ca.load(t2, t2.c0a);
     cb.load(t2, t2.c0b);
     typename Mode::Out out[Mode::kOutputs][kChunk];
@@ -1599,8 +1636,8 @@ struct OutputSplit {
 // kFirst the running sums c0 x + y_lo + ... (yrun), else each A section's
 // output (ya[k]); with B sections B's output (yb, Coeffs::step).
 template <bool kGeneral, bool kFirst, int A0, int NAW, int NBW, class Mode>
-__device__ __forceinline__ void split_run(const Mode &m, const Coeffs<A0, NAW, Mode::kB2> &ca,
-                                          const Coeffs<A0 + NAW, NBW, Mode::kB2> &cb,
+__device__ __forceinline__ void split_run(const Mode &m, const Coeffs<A0, NAW, Mode::kObserver> &ca,
+                                          const Coeffs<A0 + NAW, NBW, Mode::kObserver> &cb,
                                           const typename Mode::In (&in)[kChunk][Mode::kInputs],
                                           int64_t j0, int64_t len, BankPair<NAW, NBW, A0> &s,
                                           double (&yrun)[kChunk],
@@ -1733,8 +1770,8 @@ __device__ __forceinline__ void output_split_wave(const Mode &m, const IirTable 
         // as iir_output_kernel: filter B's chunk end states from zero in the
         // previous blocks, carried to this block's start and summed in LDS,
         // then its in-block lane start states by the aggregate pass's steps
-        Coeffs<A0, 0, Mode::kB2> none;
-        Coeffs<A0, NBW, Mode::kB2> wb;
+        Coeffs<A0, 0, Mode::kObserver> none;
+        Coeffs<A0, NBW, Mode::kObserver> wb;
         wb.load(t, t.c0b);
         const double *mk = t.pw[kLevelBlock][NA];
         double vu = 0.0, vv = 0.0;
@@ -1780,8 +1817,8 @@ __device__ __forceinline__ void output_split_wave(const Mode &m, const IirTable 
     }
 
     // the recursion over this wavefront's sections
-    Coeffs<A0, NAW, Mode::kB2> ca;
-    Coeffs<A0 + NAW, NBW, Mode::kB2> cb;
+    Coeffs<A0, NAW, Mode::kObserver> ca;
+    Coeffs<A0 + NAW, NBW, Mode::kObserver> cb;
     ca.load(t, W == 0 ? t.c0a : 0.0);
     if constexpr (NBW > 0) cb.load(t, t.c0b);
     double yrun[kChunk], ya[NAW > 0 ? NAW : 1][kChunk], yb[kChunk];

@@ -13,7 +13,7 @@ struct SingleMode {
     static constexpr bool kReverse = kRev;
     static constexpr bool kAccumulates = false;
     static constexpr bool kSegments = false;
-    static constexpr bool kB2 = false;
+    static constexpr bool kObserver = true;
     using In = float;
     using Out = float;
 
@@ -60,7 +60,7 @@ static int dispatch(int sections, const float *x, float *y, int64_t rows, int64_
     return PESQ_ERR_ARGUMENT;
 }
 
-// A cascade of one section: a full biquad (b2 kept) through the scan kernels.
+// A cascade of one section: a full biquad through the scan kernels.
 template <bool kRev>
 struct BiquadMode {
     static constexpr int kInputs = 1;
@@ -69,7 +69,7 @@ struct BiquadMode {
     static constexpr bool kReverse = kRev;
     static constexpr bool kAccumulates = false;
     static constexpr bool kSegments = false;
-    static constexpr bool kB2 = true;
+    static constexpr bool kObserver = true;
     using In = float;
     using Out = float;
 
@@ -166,15 +166,7 @@ __global__ void __launch_bounds__(kSegmentWaves *kWave, 3) iir_cascade_kernel(Ca
     for (int k = 0; k < a.sections; ++k) {
         const ConstDoubles pw = (ConstDoubles)(&a.tables[k].pw[0][0][0]);
         Coeffs<0, 1, true> c;
-        {
-            const IirTable &t = a.tables[k];
-            c.b0[0] = *(ConstDoubles)t.b0;
-            c.b1[0] = *(ConstDoubles)t.b1;
-            c.b2[0] = *(ConstDoubles)t.b2;
-            c.a1[0] = *(ConstDoubles)t.a1;
-            c.a2[0] = *(ConstDoubles)t.a2;
-            c.c0 = 0.0;
-        }
+        c.load_scalar(a.tables[k], a.tables[k].c0a);
         Bank<1> z;
         z.zero();
 #pragma unroll
@@ -226,7 +218,7 @@ __global__ void __launch_bounds__(kSegmentWaves *kWave, 3) iir_cascade_kernel(Ca
         s.u[0] = lane == 0 ? pu : before_u;
         s.v[0] = lane == 0 ? pv : before_v;
 #pragma unroll
-        for (int i = 0; i < kSegmentChunk; ++i) y[i] = c.section(0, s, y[i], 0.0);
+        for (int i = 0; i < kSegmentChunk; ++i) y[i] = c.step(s, y[i]);
     }
     if constexpr (kOutput) {
 #pragma unroll

@@ -53,7 +53,7 @@ struct PipeFwdMode {
     static constexpr bool kAccumulates = true;
     static constexpr bool kSegments = true;
     static constexpr int64_t kSegmentSlots = 3 * 1024;  // by registers and LDS (44 KB per 4)
-    static constexpr bool kB2 = false;
+    static constexpr bool kObserver = false;
     using In = float;
     using Out = float;
 
@@ -98,7 +98,7 @@ struct PipeBwdMode {
     static constexpr bool kAccumulates = false;
     static constexpr bool kSegments = true;
     static constexpr int64_t kSegmentSlots = 2 * 1024;  // by LDS (81 KB per 4 wavefronts)
-    static constexpr bool kB2 = false;
+    static constexpr bool kObserver = false;
     using In = float;
     using Out = float;
 
@@ -183,7 +183,7 @@ struct PipeBwdPowerMode {
     static constexpr bool kReverse = true;
     static constexpr bool kAccumulates = false;
     static constexpr bool kSegments = false;
-    static constexpr bool kB2 = false;
+    static constexpr bool kObserver = false;
     using In = float;
     using Out = float;
 

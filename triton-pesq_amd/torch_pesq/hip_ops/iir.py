@@ -2,8 +2,9 @@
 
 Realisations
 ------------
-Every section is a direct form II transposed biquad with a float64 state,
-scanned over the time axis in chunks (``csrc/iir.hpp``).  Two realisations of
+Every section is a biquad in observer form (states of the size of the output)
+with a float64 state, scanned over the time axis in chunks (``csrc/iir.hpp``).
+Two realisations of
 a difference equation ``b / a`` are built on the host and scored by how well
 their float64 impulse response reproduces the one of the difference equation
 itself (``scipy.signal.lfilter`` in float64), the *fidelity*:
