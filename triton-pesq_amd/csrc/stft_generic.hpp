@@ -24,7 +24,13 @@
 // Bound by issue (float64) and LDS.  32 rows of 64123 samples at 1024 / 256:
 // forward 44 -> 27.5 us, backward frames 78 -> 44, gather 11 -> 8.4 against
 // radix-2 passes in LDS for every length; 32 rows of 64000 at 512 / 160, window
-// 400: forward 39 -> 25.6, backward frames (16 rows) 63 -> 41.
+// 400: forward 39 -> 25.6, backward frames (16 rows) 63 -> 41.  The radix-2
+// variant holds two points per lane and a buffer of 128 (63 and 76 registers,
+// eight and six wavefronts per SIMD; with room for 512 points, 168 and 239: three
+// and two).  64000 samples, forward and backward with the gather, against one
+// frame per wavefront of that size: 32 / 16 over 64 rows 200 + 367 -> 114 + 244,
+// 64 / 32 over 64 rows 116 + 217 -> 70 + 151, 128 / 64 over 32 rows 33 + 68 -> 25
+// + 54, 256 / 64 over 32 rows 41 + 89 -> 31 + 73.
 #pragma once
 
 #include "common.hpp"
@@ -35,8 +41,8 @@ namespace pesq {
 constexpr int kGenMaxHalf = 512;   // n_fft <= 1024
 constexpr int kGenMinHalf = 16;    // n_fft >= 32
 constexpr int kGenMaxBands = 128;
-constexpr int kGenPerLane = kGenMaxHalf / kWave;       // points per lane (<= 8)
-constexpr int kGenBfly = kGenMaxHalf / 2 / kWave;      // butterflies per lane (<= 4)
+constexpr int kGenSmallHalf = 128;                     // the radix-2 transform's longest
+constexpr int kGenBfly = kGenSmallHalf / 2 / kWave;    // its butterflies per lane
 constexpr int kGenWaves = 4;                           // frames per workgroup
 
 struct StftTable {
@@ -172,12 +178,12 @@ __device__ __forceinline__ void fft512(c64g (&v)[8], c64g *buf, const double2 *t
 }
 
 // --------------------------------------------------------------------------
-// the transforms by half length: kHalf 256, 512, or 0 for any other
+// the transforms by half length: kHalf 256, 512, or 0 for any up to 128
 // --------------------------------------------------------------------------
 template <int kH>
 struct GenFft {
-    static constexpr int kPoints = kH == 0 ? kGenPerLane : kH / kWave;  // per lane
-    static constexpr int kBuffer = kH == 0 ? kGenMaxHalf : (kH == 512 ? kSlots512 : kH);
+    static constexpr int kPoints = (kH == 0 ? kGenSmallHalf : kH) / kWave;  // per lane
+    static constexpr int kBuffer = kH == 0 ? kGenSmallHalf : (kH == 512 ? kSlots512 : kH);
     // twiddles staged in LDS: the pass twiddles (256: per pass layout), the fold's
     static constexpr int kTw = kH == 512 ? 512 : (kH == 256 ? kPassTwiddles : 1);
     static constexpr int kFold = kH == 0 ? 1 : kH;
