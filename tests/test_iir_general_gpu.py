@@ -296,3 +296,37 @@ def test_high_pass_under_an_offset(rows, sections, cutoff):
             want = sosfilt(sos.astype(np.longdouble), x64[:, ::-1] if reverse else x64)
         want = (want[:, ::-1] if reverse else want).astype(np.float64)
         assert peak_error(got, want if rows % 2 == 0 else want[::-1]) < 2e-7
+
+
+@pytest.mark.parametrize("sections", [2, 4, 5, 8, 9, 32])
+@pytest.mark.parametrize("blocks", [10, 19, 40, 79, 130, 700])
+def test_cascade_start_states_shared_out(sections, blocks):
+    """Rows whose block start states are carried by one wavefront, by several
+    (states handed on with powers of the block transfer, at the edges of their
+    shares) and at every level of powers.  Resonances that keep 0.96 of their
+    state over a block, ringing on through the silence after the row's first
+    third: ``sosfilt`` in extended precision, to 2e-7 of each part's own peak
+    (three roundings to float32)."""
+
+    from scipy.signal import sosfilt
+
+    from torch_pesq.hip_ops import iir as iir_ops
+
+    rng = np.random.default_rng(blocks)
+    radius, angle = 1.0 - 2e-5 * rng.uniform(0.5, 1.5, sections), rng.uniform(0.2, 2.9, sections)
+    sos = np.ones((sections, 6))
+    sos[:, 4:] = np.stack([-2 * radius * np.cos(angle), radius**2], 1)
+    sos[:, 1:3] = sos[:, 4:] * (1 - 1e-4)  # 1 + a resonance
+    table = iir_ops._pack_cascade(sos).cuda()
+    n = 2048 * blocks - 3
+    x = noise(2, n, seed=blocks).astype(np.float32)
+    x[:, n // 3 :] = 0.0
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")  # (scipy means to drop extended precision)
+        want = sosfilt(sos.astype(np.longdouble), x.astype(np.longdouble)).astype(np.float64)
+    for reverse in (False, True):
+        given = torch.from_numpy(x[:, ::-1].copy() if reverse else x).cuda()
+        got = iir_ops._launch(given, table, "cascade", sections, reverse).double().cpu().numpy()
+        got = got[:, ::-1] if reverse else got
+        for part in (slice(0, n // 3), slice(n // 3, n // 2), slice(n // 2, n - 4096), slice(n - 4096, n)):
+            assert peak_error(got[:, part], want[:, part]) < 2e-7

@@ -2,6 +2,7 @@
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
+#include <limits>
 #include <vector>
 
 #include "tables.hpp"
@@ -112,8 +113,10 @@ static int fill_sections(IirTable &t, int first, const pesq_iir_sections &s, dou
     return PESQ_OK;
 }
 
-// T of a cascade (IirTable::cascade): the matrix of one step without input,
-// column by column, squared log2(kSegmentSpan) times in extended precision
+// T^(8^i) of a cascade (IirTable::cascade): the matrix of one step without
+// input, column by column, squared log2(kSegmentSpan) times and three times
+// more per level, in extended precision.  A power that overflows (an unstable
+// cascade) is held at the largest double, so that zero states stay zero.
 static void cascade_transfer(IirTable *tables, int sections) {
     const int n = 2 * sections;
     std::vector<long double> m(size_t(n) * n), sq(size_t(n) * n);
@@ -127,7 +130,7 @@ static void cascade_transfer(IirTable *tables, int sections) {
             x = t.c0a * x + u;
         }
     }
-    for (int span = 1; span < kSegmentSpan; span *= 2) {
+    auto square = [&] {
         for (int i = 0; i < n; ++i) {
             for (int j = 0; j < n; ++j) {
                 long double acc = 0.0L;
@@ -137,10 +140,19 @@ static void cascade_transfer(IirTable *tables, int sections) {
             }
         }
         m.swap(sq);
-    }
-    for (int i = 0; i < n; ++i) {
-        for (int j = 0; j < n; ++j) {
-            tables[i / 2].cascade[i % 2][j] = static_cast<double>(m[size_t(i) * n + j]);
+    };
+    constexpr long double most = std::numeric_limits<double>::max();
+    for (int span = 1; span < kSegmentSpan; span *= 2) square();
+    for (int level = 0; level < kCascadeLevels; ++level) {
+        if (level > 0) {
+            for (int i = 0; i < 3; ++i) square();
+        }
+        for (int i = 0; i < n; ++i) {
+            for (int j = 0; j < n; ++j) {
+                long double v = m[size_t(i) * n + j];
+                if (!(std::fabs(v) <= most)) v = v < 0.0L ? -most : most;
+                tables[i / 2].cascade[level][i % 2][j] = static_cast<double>(v);
+            }
         }
     }
 }

@@ -101,6 +101,7 @@ constexpr int kMaxSections = PESQ_IIR_MAX_SECTIONS;
 // block level scan (iir_prefix_kernel: rows of up to 2^18 blocks)
 constexpr int kLevelBlock = 6;
 constexpr int kLevels = 24;
+constexpr int kCascadeLevels = 4;
 static_assert(kSpan == kChunk << kLevelBlock, "a block is 2^6 chunks");
 
 struct IirTable {
@@ -119,10 +120,10 @@ struct IirTable {
     // M^(2 i), M = A_k^kSpan the block transfer: the weight of the block pair
     // (M e_j + e_j+1) 2 i + 2 blocks before a block (block_start_reduce)
     double blk_pw2[kWave][kMaxSections][4];
-    // rows 2 k and 2 k + 1 of T, k this table's section in a cascade: the
-    // transfer of all the cascade's states (z1, z2 of section 0, of section 1,
-    // ...) over kSegmentSpan samples of zero input
-    double cascade[2][2 * PESQ_IIR_MAX_CASCADE];
+    // rows 2 k and 2 k + 1 of T^(8^i), i < kCascadeLevels, k this table's section
+    // in a cascade: T is the transfer of all the cascade's states (z1, z2 of
+    // section 0, of section 1, ...) over kSegmentSpan samples of zero input
+    double cascade[kCascadeLevels][2][2 * PESQ_IIR_MAX_CASCADE];
 };
 
 // How an output wavefront obtains its block's start state (the kPrefix

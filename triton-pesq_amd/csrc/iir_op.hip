@@ -1,6 +1,8 @@
 // Stand-alone IIR filter (the TritonIIR operator), forward or time reversed:
 // one filter in parallel form (one scan pass), or a cascade of full biquads
 // (all sections in one pass, iir_cascade_kernel).
+#include <utility>
+
 #include "iir.hpp"
 
 namespace pesq {
@@ -101,8 +103,8 @@ struct BiquadMode {
 // so no signal between the sections leaves the registers.  A block's start
 // states (two per section) depend on the row's earlier blocks through all
 // sections before them, so rows of more than one block take three launches:
-// the blocks run from zero states (kOutput false) to their end states, one
-// wavefront per row carries these over the row (s_(b+1) = T s_b + e_b, T the
+// the blocks run from zero states (kOutput false) to their end states, a
+// workgroup per row carries these over the row (s_(b+1) = T s_b + e_(b+1), T the
 // cascade's transfer over a block), and the blocks run again from their true
 // starts.  The blocks of a row do not depend on the other rows: a row's result
 // is the same in any batch.
@@ -111,7 +113,8 @@ struct BiquadMode {
 // per section and 2048 samples, in both block passes.  One scan pass per
 // section, with float64 signals through memory between them, took 445
 // us for 8 sections over 24 rows of 160001 samples, forward and adjoint; this
-// form takes 121 us (states 16, starts 16, output 22 us per direction).
+// form takes 119 us with the host's share (states 16, starts 11, output 24 us per
+// direction).
 // --------------------------------------------------------------------------
 struct CascadeArgs {
     const float *x;
@@ -234,59 +237,145 @@ __global__ void __launch_bounds__(kSegmentWaves *kWave, 3) iir_cascade_kernel(Ca
 }
 
 // Start states of a row's blocks from the end states of the blocks before
-// them, in place, one wavefront per row: lane i holds row i of T (kN >= 2
-// sections columns, zero past them) and state i; the current start state is
-// passed through LDS, every lane reading all of it.  The end states of
-// kStartsAhead blocks are loaded while the ones before them are carried (a load
-// per block, one block ahead, waited out the memory latency at each block: 46
-// us instead of 16 for 79 blocks of 8 sections).
-constexpr int kStartsAhead = 8;
+// them, in place, one workgroup per row: s_(b+1) = T s_b + e_(b+1).  The steps are
+// serial, so a long row is shared out (StartsPlan): a group of lanes carries the
+// blocks of its share from a zero state, the states at the shares' first blocks
+// follow from those ends with T^per = (T^(8^level))^hops, and each group carries
+// its blocks again from its true start.
+//
+// Lane i of a group holds row i of T (kN >= 2 sections columns, zero past them)
+// and state i, which the others take by lane broadcasts: groups of 16 lanes, four
+// shares per wavefront, up to 8 sections, else a wavefront per share.  The end
+// states of kStartsGroup blocks are loaded while the ones before them are
+// carried.  Bound by the issue of the steps on one CU, about 0.1 us each, and 6 us
+// of loads.  1 row of 2880000 samples (1407 blocks), 2 sections: 18.3 us, the
+// filter 38 (170 with one wavefront carrying every block of the row, 48 with a
+// scan per section); 1 row of 960000, 8 sections: 24.6 us, the filter 54 (104,
+// 100).
+constexpr int kStartsGroup = 16;  // blocks carried without a branch; divides per
+
+struct StartsPlan {
+    int shares, per;  // blocks of a share (the last one's may be fewer)
+    int level, hops;  // per = hops 8^level
+};
+
+// The plan of fewest serial steps: a share's blocks twice, and hops for every
+// share before the last.
+static StartsPlan starts_plan(int blocks, int most) {
+    const int count = blocks - 1;
+    StartsPlan best{1, count, 0, count};
+    int cost = count - 8;  // the shared form's barrier and loads of T
+    for (int level = 0, unit = 1; level < kCascadeLevels; ++level, unit *= 8) {
+        const int quantum = unit < kStartsGroup ? kStartsGroup / unit : 1;
+        int hops = (count + most * unit - 1) / (most * unit);
+        hops = (hops + quantum - 1) / quantum * quantum;
+        const int per = hops * unit, shares = (count + per - 1) / per;
+        if (2 * per + (shares - 1) * hops < cost) {
+            cost = 2 * per + (shares - 1) * hops;
+            best = {shares, per, level, hops};
+        }
+    }
+    return best;
+}
+
+// lane j of the lane's group (of 16: DPP row_newbcast, or of the whole wavefront)
+template <int kLanes, int j>
+__device__ __forceinline__ double group_lane(double v) {
+    if constexpr (kLanes == 16) return dpp_move<0x150 + j, 0xF>(v);
+    return read_lane(v, j);
+}
+// e + sum_j t[j] (v of the group's lane j)
+template <int kLanes, int kN, int... j>
+__device__ __forceinline__ double group_product(const double (&t)[kN], double v, double e,
+                                                std::integer_sequence<int, j...>) {
+    double acc[4] = {e, 0.0, 0.0, 0.0};
+    ((acc[j % 4] = fma(t[j], group_lane<kLanes, j>(v), acc[j % 4])), ...);
+    return (acc[0] + acc[1]) + (acc[2] + acc[3]);
+}
 
 template <int kN>
-__global__ void __launch_bounds__(kWave) iir_cascade_starts_kernel(CascadeArgs a) {
-    __shared__ __attribute__((aligned(16))) double state[kN > kWave ? kN : kWave];
+struct Starts {
+    static constexpr int kLanes = kN <= 16 ? 16 : kWave;     // of a share
+    static constexpr int kPerWave = kWave / kLanes;          // shares
+    static constexpr int kWaves = 8;                         // at most, by registers
+};
+
+template <int kN>
+__global__ void __launch_bounds__(kWave *Starts<kN>::kWaves)
+    iir_cascade_starts_kernel(CascadeArgs a, StartsPlan plan) {
+    using S = Starts<kN>;
+    __shared__ double ends[S::kWaves * kWave];
+    static_assert(kN >= 4 && kN <= S::kLanes, "a lane per state");
     const int n = 2 * a.sections;
-    const int lane = threadIdx.x;
-    const int mine = lane < n ? lane : 0;
+    const int lane = static_cast<int>(threadIdx.x) % S::kLanes;
+    const int share = static_cast<int>(threadIdx.x) / S::kLanes;
+    const bool mine = lane < n && share < plan.shares;
+    const int at = lane < n ? lane : 0;
     double t[kN];
+    auto transfer = [&](int level) {
 #pragma unroll
-    for (int j = 0; j < kN; ++j) {
-        const double v = a.tables[mine / 2].cascade[mine % 2][j];
-        t[j] = lane < n && j < n ? v : 0.0;
-    }
-    state[lane] = 0.0;
-    wave_lds_fence();
-    double *row = a.states + int64_t(blockIdx.x) * a.blocks * n + mine;
-    auto load = [&](int b0, double (&e)[kStartsAhead]) {
-#pragma unroll
-        for (int q = 0; q < kStartsAhead; ++q) {
-            const int b = b0 + q < a.blocks ? b0 + q : a.blocks - 1;
-            e[q] = row[int64_t(b) * n];
+        for (int j = 0; j < kN; ++j) {
+            const double v = a.tables[at / 2].cascade[level][at % 2][j];
+            t[j] = lane < n && j < n ? v : 0.0;
         }
     };
-    double e[kStartsAhead], next[kStartsAhead];
-    load(1, e);
-    for (int b0 = 1; b0 < a.blocks; b0 += kStartsAhead) {
-        load(b0 + kStartsAhead, next);
+    // T state + e, state j broadcast to the group
+    auto carry = [&](double state, double e) {
+        return group_product<S::kLanes>(t, state, e, std::make_integer_sequence<int, kN>{});
+    };
+    const int first = 1 + share * plan.per;
+    const int left = a.blocks - first;  // (at most 0 past the shares)
+    const int count = plan.per < left ? plan.per : left;
+    double *row = a.states + int64_t(blockIdx.x) * a.blocks * n + at;
+    auto load = [&](int b0, double (&e)[kStartsGroup]) {
 #pragma unroll
-        for (int q = 0; q < kStartsAhead; ++q) {
-            if (b0 + q < a.blocks) {  // uniform
-                double acc[4] = {e[q], 0.0, 0.0, 0.0};
-#pragma unroll
-                for (int j = 0; j < kN; j += 2) {
-                    const double2 s = *reinterpret_cast<const double2 *>(state + j);
-                    acc[j % 4] = fma(t[j], s.x, acc[j % 4]);
-                    acc[j % 4 + 1] = fma(t[j + 1], s.y, acc[j % 4 + 1]);
-                }
-                wave_lds_fence();
-                const double v = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-                state[lane] = lane < n ? v : 0.0;
-                wave_lds_fence();
-                if (lane < n) row[int64_t(b0 + q) * n] = v;
-            }
-            e[q] = next[q];
+        for (int q = 0; q < kStartsGroup; ++q) {
+            // (past the shares count <= 0: the row's last block)
+            e[q] = row[int64_t(first + (b0 + q < count ? b0 + q : count - 1)) * n];
         }
+    };
+    // a share's blocks from `state`: the state after them (of a whole share)
+    auto run = [&](double state, auto written) {
+        double e[kStartsGroup], next[kStartsGroup];
+        load(0, e);
+        for (int b0 = 0; b0 < plan.per; b0 += kStartsGroup) {
+            load(b0 + kStartsGroup, next);
+#pragma unroll
+            for (int q = 0; q < kStartsGroup; ++q) {
+                state = carry(state, mine ? e[q] : 0.0);
+                if constexpr (decltype(written)::value) {
+                    if (mine && b0 + q < count) row[int64_t(first + b0 + q) * n] = state;
+                }
+                e[q] = next[q];
+            }
+        }
+        return state;
+    };
+    transfer(0);
+    double start = 0.0;
+    if (plan.shares > 1) {  // uniform over the grid
+        ends[threadIdx.x] = run(0.0, std::false_type{});
+        __syncthreads();
+        transfer(plan.level);
+        for (int s = 0; s + 1 < plan.shares; ++s) {
+            const double e = ends[s * S::kLanes + lane];
+            double v = start;
+            for (int h = 1; h < plan.hops; ++h) v = carry(v, 0.0);
+            v = carry(v, e);
+            start = s < share ? v : start;
+        }
+        transfer(0);
     }
+    run(start, std::true_type{});
+}
+
+template <int kN>
+static void launch_starts(const CascadeArgs &a, hipStream_t stream) {
+    using S = Starts<kN>;
+    const StartsPlan plan = starts_plan(a.blocks, S::kWaves * S::kPerWave);
+    const int waves = static_cast<int>(cdiv(plan.shares, int64_t(S::kPerWave)));
+    hipLaunchKernelGGL(iir_cascade_starts_kernel<kN>, dim3(static_cast<unsigned>(a.rows)),
+                       dim3(kWave * waves), 0, stream, a, plan);
 }
 
 template <bool kRev>
@@ -307,13 +396,16 @@ static int cascade(const float *x, float *y, int64_t rows, int64_t len, const Ii
         hipLaunchKernelGGL((iir_cascade_kernel<kRev, false>), groups(a.blocks - 1), block, lds,
                            stream, a);
         PESQ_CHECK_LAUNCH("iir cascade states");
-        const dim3 grid(static_cast<unsigned>(rows)), wave(kWave);
-        if (count <= 4) {
-            hipLaunchKernelGGL(iir_cascade_starts_kernel<8>, grid, wave, 0, stream, a);
+        if (count <= 2) {
+            launch_starts<4>(a, stream);
+        } else if (count <= 4) {
+            launch_starts<8>(a, stream);
         } else if (count <= 8) {
-            hipLaunchKernelGGL(iir_cascade_starts_kernel<16>, grid, wave, 0, stream, a);
+            launch_starts<16>(a, stream);
+        } else if (count <= 16) {
+            launch_starts<32>(a, stream);
         } else {
-            hipLaunchKernelGGL(iir_cascade_starts_kernel<64>, grid, wave, 0, stream, a);
+            launch_starts<64>(a, stream);
         }
         PESQ_CHECK_LAUNCH("iir cascade starts");
     }
