@@ -7,7 +7,9 @@ arguments before touching a GPU.
 
 import ctypes
 import json
+import os
 import re
+import subprocess
 from pathlib import Path
 
 import numpy as np
@@ -486,6 +488,26 @@ def test_pipeline_kernel_variants_per_shape(shape):
     fwd, bwd = VARIANTS[shape]
     assert _lib.pipeline_kernels(*shape, backward=False) == fwd
     assert _lib.pipeline_kernels(*shape, backward=True) == bwd
+
+
+def test_scans_without_windowed_starts_are_not_segmented(tmp_path):
+    """Segments take their start states from the two blocks before them alone,
+    so a build without windowed block starts (``PESQ_WINDOW_STARTS=0``) has no
+    plan for them, and its large grids run the kernels of stored block starts.
+    The host pass over the pipeline, without code generation."""
+
+    src = tmp_path / "plain_starts.hip"
+    src.write_text(
+        "#define PESQ_WINDOW_STARTS 0\n"
+        '#include "pipeline.hip"\n'
+        "static_assert(!pesq::PipeFwdMode::kSegments && !pesq::PipeBwdMode::kSegments);\n"
+    )
+    proc = subprocess.run(
+        [os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--cuda-host-only", "-fsyntax-only",
+         "-std=c++17", "--offload-arch=gfx950", f"-I{ROOT / 'include'}",
+         f"-I{ROOT / 'triton-pesq_amd' / 'csrc'}", str(src)],
+        capture_output=True, text=True)
+    assert proc.returncode == 0, proc.stderr
 
 
 def test_pipeline_kernel_query_edges():

@@ -558,7 +558,7 @@ struct BankPair {
 //                                 else in direct form II
 //   Mode::kReverse                process the time axis back to front
 //   Mode::kAccumulates            the output pass reduces a per block sum
-//   Mode::kSegments               large grids may run segmented (SegmentPlan),
+//   Mode::kSegments               large grids run segmented (SegmentPlan),
 //                                 Mode::kSegmentSlots wavefronts at a time
 //   Mode::kRamp                   the Mode uses the edge ramp weight w of the
 //                                 sample (edge_weight(n, len)); otherwise the
@@ -1909,7 +1909,8 @@ int launch_scan(const Mode &m, const IirTable *table, double *ws, int64_t rows, 
     const bool lane_states = plan.lane_states;
     SegmentPlan seg{0, 0};
     if constexpr (Mode::kSegments) {
-        if (window) seg = segment_plan(rows, nblk, Mode::kSegmentSlots);
+        PESQ_CHECK_ARG(window, "segments need sections that decay within the window");
+        seg = segment_plan(rows, nblk, Mode::kSegmentSlots);
     }
     const bool windowed = window && lane_states;
     const bool fused = !windowed && plan.fused_prefix;

@@ -51,7 +51,7 @@ struct PipeFwdMode {
     static constexpr bool kRamp = true;
     static constexpr bool kReverse = false;
     static constexpr bool kAccumulates = true;
-    static constexpr bool kSegments = true;
+    static constexpr bool kSegments = kPipeWindow;
     static constexpr int64_t kSegmentSlots = 3 * 1024;  // by registers and LDS (44 KB per 4)
     static constexpr bool kObserver = false;
     using In = float;
@@ -96,7 +96,7 @@ struct PipeBwdMode {
     static constexpr bool kRamp = true;
     static constexpr bool kReverse = true;
     static constexpr bool kAccumulates = false;
-    static constexpr bool kSegments = true;
+    static constexpr bool kSegments = kPipeWindow;
     static constexpr int64_t kSegmentSlots = 2 * 1024;  // by LDS (81 KB per 4 wavefronts)
     static constexpr bool kObserver = false;
     using In = float;
