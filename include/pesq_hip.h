@@ -167,7 +167,10 @@ int pesq_pipeline_backward(const float *g_symm, const float *g_asymm, const floa
  * of n_fft samples every hop through the general STFT kernels, whose table
  * (window, bands, correction) is pesq_stft_table_pack's for 49 bands; the
  * model table's filters, thresholds, exponents and widths are used, its window
- * and bands are not. */
+ * and bands are not.  Pairs near the ends of the float32 range (peaks above
+ * 1e38 or below 1e-30) go through pesq_pair_scale_forward first and their
+ * gradients through pesq_pair_scale_backward, or the float32 rows in between
+ * overflow or lose digits. */
 int pesq_pipeline_general_workspace(int64_t batch, int64_t len, int grad_mask, int n_fft,
                                     int hop, size_t *forward_bytes, size_t *backward_bytes);
 int pesq_pipeline_general_forward(const float *ref, const float *deg, int64_t batch, int64_t len,
@@ -445,6 +448,18 @@ int pesq_peak_normalize_forward(const float *ref, const float *deg, int64_t batc
 int pesq_peak_normalize_backward(const float *g_ref, const float *g_deg, const float *peak,
                                  int64_t batch, int64_t len, float *out_ref, float *out_deg,
                                  hipStream_t stream);
+
+/* out = scale x for both signals of a pair, scale[b] = 2^-e (float64) with 2^e
+ * <= peak[b] < 2^(e+1); 0 for an infinite peak, NaN for a zero one.  The workspace
+ * is pesq_elementwise_workspace's for `batch` rows. */
+int pesq_pair_scale_forward(const float *ref, const float *deg, int64_t batch, int64_t len,
+                            float *out_ref, float *out_deg, double *scale, void *workspace,
+                            hipStream_t stream);
+
+/* scale g for the signals whose output is not NULL; the scale is a constant. */
+int pesq_pair_scale_backward(const float *g_ref, const float *g_deg, const double *scale,
+                             int64_t batch, int64_t len, float *out_ref, float *out_deg,
+                             hipStream_t stream);
 
 /* y = (x head) tail with head_k = (k+1)/16 (k < 15), tail_k = (len-k)/16 (last
  * 15); its own adjoint.  Replaces _edge_ramp_kernel (elementwise.py:308-331). */

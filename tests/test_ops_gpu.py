@@ -20,7 +20,7 @@ import pytest
 import torch
 
 from oracle import pesq_oracle as O
-from torch_pesq import PesqLoss
+from torch_pesq import PesqLoss, _lib
 from torch_pesq.hip_ops.chain import HipPesqChain
 from torch_pesq.hip_ops.elementwise import align_scale, edge_ramp, peak_normalize, pesq_epilogue
 from torch_pesq.hip_ops.spectral import HipStftBark
@@ -70,6 +70,52 @@ def test_peak_normalize_errors():
         peak_normalize(torch.randn(2, 0, device="cuda"), torch.randn(2, 0, device="cuda"))
     with pytest.raises(RuntimeError):
         peak_normalize(torch.randn(2, 10), torch.randn(2, 10))
+
+
+# -- common power of two --------------------------------------------------------
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 4095, 4096, 4097, 262145])
+def test_pair_scale_bit_exact(n):
+    """Products by a power of two, rounded once where they are subnormal; the peak
+    at the row's first or last sample, an infinite and a zero pair."""
+
+    lib, device = _lib.library(), torch.device("cuda", torch.cuda.current_device())
+    g = torch.Generator().manual_seed(n)
+    ref, deg = (torch.randn(5, n, generator=g) * 2.0 ** -20 for _ in range(2))
+    ref[0, 0], deg[1, -1], ref[2] = 3e38, 2.0 ** -149, 0.0
+    deg[2, n // 2], ref[3, n // 2] = -1e-44, -float("inf")
+    ref[4], deg[4] = 0.0, 0.0
+    peak = torch.maximum(ref.abs().amax(1), deg.abs().amax(1)).double()
+    want = torch.exp2(-torch.floor(torch.log2(peak)))
+    want[3], want[4] = 0.0, float("nan")
+    ref, deg = ref.to(device), deg.to(device)
+    out = [torch.empty_like(ref) for _ in range(4)]
+    scale = torch.empty(5, dtype=torch.float64, device=device)
+    ws = torch.empty(_lib.size_query(lib.pesq_elementwise_workspace, 5), dtype=torch.uint8,
+                     device=device)
+    stream = _lib.stream_handle(device)
+    p = _lib.ptr
+    _lib.check(lib.pesq_pair_scale_forward(p(ref), p(deg), 5, n, p(out[0]), p(out[1]), p(scale),
+                                           p(ws), stream), "pair scale")
+    assert torch.equal(scale[:4].cpu(), want[:4]) and scale[4].isnan()
+
+    def check(got, x):
+        exact = (x.double() * scale.unsqueeze(1)).float()
+        assert torch.equal(got[:3], exact[:3])
+        assert torch.equal(got.isnan(), exact.isnan()) and not got[exact.isfinite()].isnan().any()
+
+    check(out[0], ref)
+    check(out[1], deg)
+    for wants in ((True, True), (True, False), (False, True)):
+        for o in out[2:]:
+            o.fill_(7.0)
+        args = [p(t if w else None) for t, w in zip((ref, deg), wants)]
+        outs = [p(o if w else None) for o, w in zip(out[2:], wants)]
+        _lib.check(lib.pesq_pair_scale_backward(*args, p(scale), 5, n, *outs, stream), "backward")
+        for o, x, w in zip(out[2:], (ref, deg), wants):
+            check(o, x) if w else None
+            assert w or bool((o == 7.0).all())
 
 
 # -- edge ramp ----------------------------------------------------------------

@@ -324,3 +324,36 @@ def test_general_loss_at_infinities(bad):
     assert loss[1] == want[1]
     assert not g_ref[0].isfinite().any() and g_ref[1].isfinite().all()
     assert g_deg[0].isfinite().all() == (bad != bad) and g_deg[1].isfinite().all()
+
+
+@pytest.mark.parametrize("n_fft, win_length, hop", [(512, 400, 160), (1024, 1024, 256)])
+@pytest.mark.parametrize("rate, nsamples", [(16000, 12001), (8000, 9003), (44100, 36007)])
+def test_general_loss_over_the_whole_float32_range(rate, nsamples, n_fft, win_length, hop):
+    """The loss does not depend on the signals' scale: times a power of two it has
+    the same bits, the gradients times its inverse, rounded once, also where the
+    samples are subnormal (the smallest are 2^-142 here) and where the peak is
+    next to the largest float32."""
+
+    from torch_pesq import PesqLossTriton
+
+    model = PesqLossTriton(0.5, sample_rate=rate, n_fft=n_fft, win_length=win_length,
+                           hop_length=hop).cuda()
+    x = torch.randn(2, 3, nsamples, generator=torch.Generator().manual_seed(7)) * 0.2
+    x[1] = x[0] + 0.3 * x[1]
+    x = ((x.clamp(-0.999, 0.999) * 4096).round() / 4096).double()  # exact at every scale below
+    x[0, :, 100] = 0.999755859375  # 4095 / 4096, the common peak
+
+    def run(power):
+        y = (x * 2.0 ** power).float().cuda()
+        assert torch.equal(y.cpu().double(), x * 2.0 ** power)
+        r, d = y[0].requires_grad_(True), y[1].requires_grad_(True)
+        loss = model(r, d)
+        return (loss.detach(),) + torch.autograd.grad(loss.sum(), [r, d])
+
+    loss, g_ref, g_deg = run(0)
+    assert loss.isfinite().all() and g_ref.isfinite().all() and g_deg.isfinite().all()
+    for power in (-130, -100, -13, 20, 100, 128):
+        got, got_ref, got_deg = run(power)
+        assert torch.equal(got, loss), power
+        for got_g, want_g in ((got_ref, g_ref), (got_deg, g_deg)):
+            assert torch.equal(got_g, (want_g.double() * 2.0 ** -power).float()), power

@@ -174,6 +174,8 @@ SIGNATURES = {
     "pesq_elementwise_workspace": (_INT, [_I64, _SIZE_P]),
     "pesq_peak_normalize_forward": (_INT, [_P, _P, _I64, _I64, _P, _P, _P, _P, _P]),
     "pesq_peak_normalize_backward": (_INT, [_P, _P, _P, _I64, _I64, _P, _P, _P]),
+    "pesq_pair_scale_forward": (_INT, [_P, _P, _I64, _I64, _P, _P, _P, _P, _P]),
+    "pesq_pair_scale_backward": (_INT, [_P, _P, _P, _I64, _I64, _P, _P, _P]),
     "pesq_edge_ramp": (_INT, [_P, _P, _I64, _I64, _P]),
     "pesq_align_scale_forward": (_INT, [_P, _P, _I64, _I64, _I64, _P, _P, _P, _P]),
     "pesq_align_scale_backward": (_INT, [_P, _P, _P, _P, _I64, _I64, _I64, _P, _P, _P, _P]),
