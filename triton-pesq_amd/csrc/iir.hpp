@@ -98,9 +98,9 @@ constexpr int kOutputWaves = PESQ_OUTPUT_WAVES;
 #endif
 constexpr int kMaxSections = PESQ_IIR_MAX_SECTIONS;
 // power levels: A^(kChunk 2^j); j = 0..5 in-wave, 6 = one block, 6 and up the
-// block level scan (iir_prefix_kernel: rows of up to 2^18 blocks)
+// block level scan (iir_prefix_kernel)
 constexpr int kLevelBlock = 6;
-constexpr int kLevels = 24;
+constexpr int kLevels = 32;
 constexpr int kCascadeLevels = 4;
 static_assert(kSpan == kChunk << kLevelBlock, "a block is 2^6 chunks");
 
@@ -978,6 +978,8 @@ __global__ void __launch_bounds__(kWave *kPrefixWaves)
         return;
     }
     int level = kLevelBlock;  // of M^per
+    static_assert((int64_t(kWave) << (kLevels - 1 - kLevelBlock)) >= int64_t(1) << 31,
+                  "M^per of every row that a grid can hold is in the table");
     while ((int64_t(kWave) << (level - kLevelBlock)) < nblk) ++level;
     const int per = 1 << (level - kLevelBlock);
     const int64_t lo = int64_t(lane) * per;
@@ -1017,7 +1019,7 @@ __global__ void __launch_bounds__(kWave *kPrefixWaves)
         if (level + j < kLevels) {
             const double *p = t.pw[level + j][k];
             q = {p[0], p[1], p[2], p[3]};
-        } else {  // (rows past 2^18 blocks)
+        } else {  // (rows past 2^26 blocks)
             q = mat2_mul(q, q);
         }
         const int d = 1 << j;
