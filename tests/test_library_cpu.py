@@ -764,3 +764,24 @@ def test_bark_modules_of_builds_without_a_mark_keep_their_constants(hop):
         old.table = torch.cat([old.table[:head], old.table[head + 4096:]])
     new = pickle.loads(pickle.dumps(old))
     assert torch.equal(new.table, want)
+
+
+def test_the_layout_mark_does_not_depend_on_the_defaults_of_the_caller():
+    """Modules may be built first under another default device (a meta one too,
+    which takes filters, whose tables are packed on the host) or dtype."""
+
+    from torch_pesq.hip_ops._tables import table_layout
+
+    want = table_layout()
+    try:
+        table_layout.cache_clear()
+        with torch.device("meta"):
+            module = HipIIR(torch.tensor([1.0, 0.5], device="cpu"),
+                            torch.tensor([1.0, -0.3], device="cpu"))
+        assert module.layout == want and module.table.device.type == "cpu"
+        table_layout.cache_clear()
+        torch.set_default_dtype(torch.float64)
+        assert table_layout() == want
+    finally:
+        torch.set_default_dtype(torch.float32)
+        table_layout.cache_clear()

@@ -23,8 +23,15 @@ __all__ = ["table_layout"]
 def table_layout() -> str:
     """Digest of tables of every kind that the loaded library packs from fixed
     constants: what the tables hold, and where, decides it, so no number has to
-    be raised by hand when either changes.
+    be raised by hand when either changes.  The same under any default device and
+    dtype of the caller's.
     """
+
+    with torch.device("cpu"):
+        return _digest()
+
+
+def _digest() -> str:
 
     from .chain import _pack_chain
     from .iir import _pack_cascade, _pack_table, sections_struct
@@ -32,8 +39,8 @@ def table_layout() -> str:
     from .spectral import _general_table
 
     bands = torch.arange(1, _lib.NBARKS + 1, dtype=torch.float64)
-    window = torch.linspace(0.25, 0.75, _lib.NFFT)
-    fbank = torch.zeros(_lib.NBARKS, _lib.NFFT // 2)
+    window = torch.linspace(0.25, 0.75, _lib.NFFT, dtype=torch.float32)
+    fbank = torch.zeros(_lib.NBARKS, _lib.NFFT // 2, dtype=torch.float32)
     fbank[torch.arange(_lib.NBARKS), torch.arange(_lib.NBARKS) + 1] = 1.0
     bins = np.arange(1, _lib.NBARKS + 1)
     sos = np.array([[0.5, 0.25, 0.125, 1.0, -0.5, 0.25], [0.75, -0.5, 0.25, 1.0, 0.25, 0.5]])
