@@ -741,29 +741,36 @@ def test_tables_are_packed_again_from_the_values_of_the_first_time(kind):
         assert all(torch.equal(getattr(new, n), want[n]) for n in names)
 
 
-@pytest.mark.parametrize("hop", [160, 256])
-def test_bark_modules_of_builds_without_a_mark_keep_their_constants(hop):
-    """A general module of the first general table layout (twiddles of half the
-    length: 4096 bytes less before the fold's) gets its float64 correction from
-    the end of that table; the other family's table holds as it is."""
+@pytest.mark.parametrize("kind", ["general stft", "stft", "chain"])
+def test_modules_of_builds_without_a_mark_keep_their_constants(kind):
+    """They kept float32 copies of float64 constants, which stand in the tables
+    alone: at the end of a general table (the first had twiddles of half the
+    length: 4096 bytes less before the fold's) and of a model table (whose
+    filters come first and took fewer bytes)."""
 
     import pickle
 
     from torch_pesq import PesqLossTriton
+    from torch_pesq.hip_ops.chain import HipPesqChain
     from torch_pesq.hip_ops.spectral import HipStftBark
 
     loss = PesqLossTriton(0.5, sample_rate=16000)
     corr = loss.fbank.pow_dens_correction.detach().clone()
-    module = HipStftBark(torch.hann_window(512), loss.fbank.fbank, corr, 512, hop)
+    if kind == "chain":
+        module = HipPesqChain(loss.loudness.threshs, loss.loudness.exp, loss.fbank.width_bark,
+                              float(loss.fbank.total_width))
+    else:
+        module = HipStftBark(torch.hann_window(512), loss.fbank.fbank, corr, 512,
+                             160 if kind == "general stft" else 256)
     want = module.table.clone()
-    old = pickle.loads(pickle.dumps(module))
-    old.__dict__.pop("layout", None)
-    old.__dict__.pop("constants", None)
-    if old.general:
-        head = 16 + 4096
-        old.table = torch.cat([old.table[:head], old.table[head + 4096:]])
-    new = pickle.loads(pickle.dumps(old))
-    assert torch.equal(new.table, want)
+    for cut in (0, 4096):
+        old = pickle.loads(pickle.dumps(module))
+        old.__dict__.pop("layout", None)
+        old.__dict__.pop("constants", None)
+        head = 16 + 4096 if kind == "general stft" else 0
+        old.table = torch.cat([old.table[:head], old.table[head + cut:]])
+        new = pickle.loads(pickle.dumps(old))
+        assert torch.equal(new.table, want)
 
 
 def test_the_layout_mark_does_not_depend_on_the_defaults_of_the_caller():

@@ -16,7 +16,7 @@ import torch
 
 from .. import _lib
 
-__all__ = ["table_layout"]
+__all__ = ["model_table_constants", "table_layout"]
 
 
 @functools.lru_cache(maxsize=None)
@@ -56,3 +56,23 @@ def _digest() -> str:
     for table in tables:
         digest.update(table.numpy().tobytes())
     return digest.hexdigest()
+
+
+def model_table_constants(table: torch.Tensor) -> dict:
+    """The float64 constants at the end of a model table of any build so far
+    (``ModelTable`` in ``csrc/tables.hpp``; only what stands before them has
+    changed): the correction of the 49 bands, and the thresholds, exponents and
+    widths of up to 128.
+    """
+
+    end = 16 + 8 + 8  # n_fft, hop, counts; the calibration and the total width
+    column = 8 * 128
+    starts = {"width": end + column, "exp": end + 3 * column, "threshs": end + 4 * column}
+    starts["corr"] = starts["threshs"] + 8 * _lib.NBARKS
+    raw = table.detach().cpu().numpy()
+    values = {}
+    for name, start in starts.items():
+        count = _lib.NBARKS if name == "corr" else 128
+        at = raw.size - start
+        values[name] = torch.from_numpy(raw[at : at + 8 * count].view(np.float64).copy())
+    return values

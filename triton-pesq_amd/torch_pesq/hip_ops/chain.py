@@ -12,7 +12,7 @@ import torch
 
 from .. import _lib
 from ._common import check_input
-from ._tables import table_layout
+from ._tables import model_table_constants, table_layout
 
 __all__ = ["HipPesqChain"]
 
@@ -125,14 +125,14 @@ class HipPesqChain(torch.nn.Module):
     def __setstate__(self, state):
         # a module saved with another build of the library holds its table
         super().__setstate__(state)
-        same_size = self.table.numel() == _lib.library().pesq_model_table_bytes()
         if "layout" not in self.__dict__:
-            # builds without a mark kept float32 copies of the constants only; at
-            # this size their tables have the chain's where this build reads them
-            self.constants = tuple(v.detach().cpu().double()
-                                   for v in (self.threshs, self.exp, self.width_bark))
-            self.layout = table_layout() if same_size else None
-        if self.layout != table_layout() or not same_size:
+            # builds without a mark kept float32 copies of the constants, and the
+            # float64 ones in the table alone
+            saved, bands = model_table_constants(self.table), self.threshs.numel()
+            self.constants = tuple(saved[n][:bands] for n in ("threshs", "exp", "width"))
+            self.layout = None
+        size = _lib.library().pesq_model_table_bytes()
+        if self.layout != table_layout() or self.table.numel() != size:
             self.layout = table_layout()
             self.table = self._packed().to(self.table.device)
 

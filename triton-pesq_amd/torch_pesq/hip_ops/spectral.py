@@ -22,7 +22,7 @@ import torch
 
 from .. import _lib
 from ._common import check_input
-from ._tables import table_layout
+from ._tables import model_table_constants, table_layout
 from .pipeline import pack_model_table
 
 __all__ = ["HipStftBark", "bark_segments"]
@@ -213,19 +213,17 @@ class HipStftBark(torch.nn.Module):
         super().__setstate__(state)
         lib = _lib.library()
         size = lib.pesq_stft_table_bytes() if self.general else lib.pesq_model_table_bytes()
-        same_size = self.table.numel() == size
         if "layout" not in self.__dict__:
-            # Builds without a mark kept a float32 copy of the correction only.
-            # Their general tables end with the float64 one; their model tables
-            # have, at this size, window, bands and correction where this build
-            # reads them.
-            corr = self.correction.detach().cpu().double()
+            # builds without a mark kept a float32 copy of the correction, and the
+            # float64 one at the end of the general table or in the model table
             if self.general:
                 tail = self.table[-8 * _MAX_BANDS :].cpu().numpy().view(np.float64)
                 corr = torch.from_numpy(tail[: self.nbarks].copy())
+            else:
+                corr = model_table_constants(self.table)["corr"]
             self.constants = (self.window.detach().cpu().float().clone(), corr)
-            self.layout = None if self.general or not same_size else table_layout()
-        if self.layout != table_layout() or not same_size:
+            self.layout = None
+        if self.layout != table_layout() or self.table.numel() != size:
             self.layout = table_layout()
             self.table = self._packed().to(self.table.device)
 
