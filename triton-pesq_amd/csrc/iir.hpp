@@ -1410,9 +1410,19 @@ __device__ __forceinline__ void output_segment(const Mode &m, const IirTable &t,
     }
 }
 
+// wavefronts per SIMD of the output kernel: those of the plan where it runs segments
+template <class Mode, bool kLaneStates>
+constexpr int output_occupancy() {
+    if constexpr (Mode::kSegments && !kLaneStates) {
+        return static_cast<int>(Mode::kSegmentSlots / 1024);
+    } else {
+        return 1;
+    }
+}
+
 template <int NA, int NB, class Mode, bool kLaneStates, int kPrefix, bool kWarmB = false>
 __global__ void __launch_bounds__(Mode::kSegments && !kLaneStates ? kSegmentWaves *kWave : kWave,
-                                  Mode::kSegments && !kLaneStates ? 3 : 1)
+                                  (output_occupancy<Mode, kLaneStates>()))
     iir_output_kernel(Mode m, const IirTable *__restrict__ table,
                       const double *__restrict__ aggr, const double *__restrict__ lanes,
                       int64_t len, int nblk, SegmentPlan seg, int64_t rows) {
