@@ -1,8 +1,8 @@
 """The kernel variants chosen for large grids against those of small grids.
 
 The pipeline picks its kernels by grid size (``pesq_pipeline_kernels``): a
-batch of eighteen 30 s items runs the large-grid variants (the scans recompute
-the lane states, the STFT forward takes its lean form, the chain kernels four
+batch of eighteen 30 s items runs the large-grid variants (the scans run
+segments, the STFT forward takes its lean form, the chain kernels four
 frames per wavefront, the STFT backward two frames per wavefront in eight
 wavefronts instead of one in nine), while the same items one at a time run
 the small-grid ones.  Batch items are scored independently; the reference
@@ -13,11 +13,11 @@ Here the losses must be bitwise equal.  The transforms round as written (no
 compiler-chosen contraction) and every sum of the chain and the STFT is taken
 in an order that does not depend on the variant, so those stages give the
 same bits for an item in any batch.  What remains are the scans: the variant
-that stores the lane states runs the zero-state recursion and an in-wave
-scan and takes its block start states from the two previous blocks'
-aggregates, the one that recomputes them uses weighted sums of the chunk's
-inputs and an LDS sum for the block end state, and a prefix kernel.  Both evaluate the same recursion in
-float64 and differ by float64 rounding (the parallel form's sections are
+that stores the lane states runs the zero-state recursion over 16 samples per
+lane and an in-wave scan and takes its block start states from the two previous
+blocks' aggregates, a segment runs 32 samples per lane and carries its state
+from block to block, its first one from such aggregates.  Both evaluate the same
+recursion in float64 and differ by float64 rounding (the parallel form's sections are
 larger than their sum, so that is about 1e-11 of a sample); rounded to the
 float32 signals of the forward, a few samples land on the other side of a
 rounding boundary (one unit in the last place), and the backward filters

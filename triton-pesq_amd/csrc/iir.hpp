@@ -35,8 +35,9 @@
 // Geometry.  A lane runs the recursion of all sections over a chunk of kChunk
 // consecutive samples (the sections are independent chains, so the lane has
 // that much instruction level parallelism); a workgroup is one wavefront and
-// covers one block of kBlockSpan = 64 kChunk samples of one row.  Nothing is
-// shared between wavefronts, so the kernels have no LDS and no barriers.
+// covers one block of kBlockSpan = 64 kChunk samples of one row; the split passes
+// share a block's sections out over a few wavefronts.  (Large grids of the
+// pipeline run segments instead: SegmentPlan.)
 //   aggregate: zero state run per chunk, in-wave Kogge-Stone scan; the block's
 //              end state per section (given a zero state before the block) is
 //              written to `aggr`, laid out [row][section][block][2], and every
@@ -69,11 +70,11 @@ constexpr int kChunk = PESQ_CHUNK;                         // samples per lane
 // Lane states: for grids of up to kLaneStateWaves wavefronts (latency bound)
 // the aggregate pass stores every lane's in-block start state and the output
 // pass reads it; larger grids (bandwidth bound) skip that traffic and the
-// output pass repeats the zero state run and the in-wave scan.  Both compute
-// the same states up to float64 rounding.
-// (8192: grids of up to 7504 wavefronts, such as 8 rows of 60 s, gained 1.5 -
-// 4 us from the stored states; 16128, 256 rows of 4 s, was 6 us faster
-// recomputing)
+// output pass repeats the zero state run and the in-wave scan, in segments where
+// the Mode runs them.  Both compute the same states up to float64 rounding.
+// (8192, measured without segments: grids of up to 7504 wavefronts, such as 8
+// rows of 60 s, gained 1.5 - 4 us from the stored states; 16128, 256 rows of
+// 4 s, was 6 us faster recomputing)
 constexpr int64_t kLaneStateWaves = 8192;
 constexpr int kSpan = kWave * kChunk;                      // samples per block
 constexpr int64_t kBlockSpan = kSpan;
@@ -1077,9 +1078,9 @@ __global__ void __launch_bounds__(kWave *kPrefixWaves)
 // unsegmented passes, aggregate and output, took about 1700), 80 % of the
 // kernel's time forward with three wavefronts per SIMD, 58 % backward with the
 // two that its LDS allows (16 samples per lane and three wavefronts were no
-// faster).  512 rows of 64000 samples: forward scans 173 -> 115 us, backward
-// 117 -> 83 us, the training step at 256 x 4 s, 48 kHz 706 -> 633 us; 74 rows of
-// 116961: 57 -> 51 us.
+// faster).  Kernel trace of 256 x 4 s at 48 kHz (512 rows of 64000 samples forward,
+// 256 backward): forward scans 158 -> 108 us, backward 107 -> 78 us, the training
+// step 706 - 737 -> 631 - 680 us by box; 74 rows of 116961: 57 -> 51 us.
 // --------------------------------------------------------------------------
 constexpr int kSegmentWaves = 4;             // wavefronts (segments) per workgroup
 constexpr int kStageChunk = kSegmentChunk + 4;  // floats between the staged chunks of two lanes

@@ -98,8 +98,8 @@ struct BiquadMode {
 //
 // A wavefront holds a block of kSegmentSpan samples of a row, 32 per lane as
 // doubles, and runs the sections over it one after the other: each section's
-// chunk end states (2 FMAs per sample), their scan over the lanes and the
-// recursion (5 FMAs per sample), whose outputs are the next section's inputs,
+// chunk end states (4 operations per sample), their scan over the lanes and the
+// recursion (5 per sample), whose outputs are the next section's inputs,
 // so no signal between the sections leaves the registers.  A block's start
 // states (two per section) depend on the row's earlier blocks through all
 // sections before them, so rows of more than one block take three launches:
@@ -109,11 +109,11 @@ struct BiquadMode {
 // starts.  The blocks of a row do not depend on the other rows: a row's result
 // is the same in any batch.
 //
-// Bound by issue and the sections' serial chains: about 330 VALU instructions
-// per section and 2048 samples, in both block passes.  One scan pass per
+// Bound by issue and the sections' serial chains: 345 VALU instructions per
+// section and 2048 samples in the states pass, 383 in the output pass.  One scan pass per
 // section, with float64 signals through memory between them, took 445
 // us for 8 sections over 24 rows of 160001 samples, forward and adjoint; this
-// form takes 119 us with the host's share (states 16, starts 11, output 24 us per
+// form takes 119 us with the host's share (states 18, starts 12, output 24 us per
 // direction).
 // --------------------------------------------------------------------------
 struct CascadeArgs {

@@ -4,9 +4,8 @@ Realisations
 ------------
 Every section is a biquad in observer form (states of the size of the output)
 with a float64 state, scanned over the time axis in chunks (``csrc/iir.hpp``).
-Two realisations of
-a difference equation ``b / a`` are built on the host and scored by how well
-their float64 impulse response reproduces the one of the difference equation
+Two realisations of a difference equation ``b / a`` are built on the host and
+scored by how well their float64 impulse response reproduces the one of the difference equation
 itself (``scipy.signal.lfilter`` in float64), the *fidelity*:
 
 ``parallel``
@@ -402,7 +401,8 @@ class HipIIR(torch.nn.Module):
     over the time axis.  Same constructor as ``TritonIIR``
     (``iir.py:1343-1375``); ``chunk_size`` is validated like there and
     ``method`` accepted, but the chunk geometry is fixed by the kernels (16
-    samples per lane, 1024 per wavefront), so results do not depend on them.
+    samples per lane, 1024 per wavefront; cascades of two and more sections 32
+    and 2048), so results do not depend on them.
 
     Attributes
     ----------
