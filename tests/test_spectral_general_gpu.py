@@ -357,3 +357,31 @@ def test_general_loss_over_the_whole_float32_range(rate, nsamples, n_fft, win_le
         assert torch.equal(got, loss), power
         for got_g, want_g in ((got_ref, g_ref), (got_deg, g_deg)):
             assert torch.equal(got_g, (want_g.double() * 2.0 ** -power).float()), power
+
+
+@pytest.mark.parametrize("rate", [16000, 44100])
+def test_general_loss_create_graph_and_double_backward(rate):
+    """``create_graph`` gives the same first derivatives (the signals' common
+    factor is then applied by torch's operators), the second ones raise."""
+
+    from torch_pesq import PesqLossTriton
+
+    model = PesqLossTriton(0.5, sample_rate=rate, hop_length=160).cuda()
+    x = torch.randn(2, 2, rate, generator=torch.Generator().manual_seed(3)) * 0.05
+    ref, deg = x[0].cuda().requires_grad_(True), x[1].cuda().requires_grad_(True)
+    want = torch.autograd.grad(model(ref, deg).sum(), [ref, deg])
+    got = torch.autograd.grad(model(ref, deg).sum(), [ref, deg], create_graph=True)
+    assert all(torch.equal(g, w) and not g.requires_grad for g, w in zip(got, want))
+    upstream = torch.ones(2, device="cuda", requires_grad=True)
+    got = torch.autograd.grad(model(ref, deg), [ref, deg], grad_outputs=upstream, create_graph=True)
+    assert all(torch.equal(g, w) and g.requires_grad for g, w in zip(got, want))
+    with pytest.raises(RuntimeError, match="differentiate twice"):
+        (got[0].sum() + got[1].sum()).backward()
+    # one signal's gradient alone, and one output's
+    d_symm, d_asymm = model.raw(ref.detach(), deg)
+    (g1,) = torch.autograd.grad(d_symm.sum(), deg)
+    d_symm, _ = model.raw(ref, deg.detach())
+    (g2,) = torch.autograd.grad(d_symm.sum(), ref)
+    d_symm, _ = model.raw(ref, deg)
+    both = torch.autograd.grad(d_symm.sum(), [ref, deg])
+    assert torch.equal(g1, both[1]) and torch.equal(g2, both[0])
