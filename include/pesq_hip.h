@@ -167,10 +167,9 @@ int pesq_pipeline_backward(const float *g_symm, const float *g_asymm, const floa
  * of n_fft samples every hop through the general STFT kernels, whose table
  * (window, bands, correction) is pesq_stft_table_pack's for 49 bands; the
  * model table's filters, thresholds, exponents and widths are used, its window
- * and bands are not.  Pairs near the ends of the float32 range (peaks above
- * 1e38 or below 1e-30) go through pesq_pair_scale_forward first and their
- * gradients through pesq_pair_scale_backward, or the float32 rows in between
- * overflow or lose digits. */
+ * and bands are not.  The float32 rows in between hold the pairs times the power
+ * of two that brings their common peak into [1, 2), so the whole float32 range is
+ * taken. */
 int pesq_pipeline_general_workspace(int64_t batch, int64_t len, int grad_mask, int n_fft,
                                     int hop, size_t *forward_bytes, size_t *backward_bytes);
 int pesq_pipeline_general_forward(const float *ref, const float *deg, int64_t batch, int64_t len,
@@ -178,6 +177,14 @@ int pesq_pipeline_general_forward(const float *ref, const float *deg, int64_t ba
                                   int hop, double factor, int grad_mask, float *d_symm,
                                   float *d_asymm, float *mos, float *loss, void *fwd_workspace,
                                   hipStream_t stream);
+/* The forward of pairs that are scaled already (pesq_pair_scale_forward, before a
+ * resampler): it does not look for their peaks.  The same workspace and backward. */
+int pesq_pipeline_general_forward_scaled(const float *ref, const float *deg, int64_t batch,
+                                         int64_t len, const void *model_table,
+                                         const void *stft_table, int n_fft, int hop,
+                                         double factor, int grad_mask, float *d_symm,
+                                         float *d_asymm, float *mos, float *loss,
+                                         void *fwd_workspace, hipStream_t stream);
 int pesq_pipeline_general_backward(const float *g_symm, const float *g_asymm, const float *g_mos,
                                    const float *g_loss, int64_t batch, int64_t len,
                                    const void *model_table, const void *stft_table, int n_fft,

@@ -8,6 +8,7 @@
 #include <cmath>
 
 #include "common.hpp"
+#include "pair_scale.hpp"
 
 namespace pesq {
 
@@ -97,18 +98,10 @@ __global__ void __launch_bounds__(kEwThreads)
 
 // -- common power of two ------------------------------------------------------
 //
-// A pair times 2^-e, 2^e <= peak < 2^(e + 1): every bit of samples that are not
-// far below the peak is kept, and what a scale invariant computation rounds
-// afterwards is rounded as before, only away from the ends of the float32
-// range.  An infinite peak gives 0 (0 for the finite samples, NaN for the
-// infinite ones) and a zero peak NaN, as division by the peak does.  Bound by
-// memory latency at the sizes of a batch: 16 pairs of 64000 samples 5.5 us for the
+// Both signals of each pair times its factor (pair_scale.hpp), for pairs that
+// are resampled before the pipeline at another STFT geometry; of others that
+// pipeline takes the peaks alone and scales its own rows.  Bound by memory latency at the sizes of a batch: 16 pairs of 64000 samples 5.5 us for the
 // peaks, 5.3 for the products, 3.8 for the gradients of both.
-
-__device__ __forceinline__ double pair_factor(float peak) {
-    if (peak == 0.0f) return static_cast<double>(NAN);
-    return isinf(peak) ? 0.0 : ldexp(1.0, -ilogb(static_cast<double>(peak)));
-}
 
 // four samples per thread and signal: enough workgroups to hide the latency
 // (4096 samples per workgroup: 9.0 us for the products)
@@ -149,8 +142,7 @@ __global__ void __launch_bounds__(kEwThreads)
     float r[4], d[4];
     load4(ref + b * n, i, n, r);
     load4(deg + b * n, i, n, d);
-    static_assert(kParts == kWave, "a partial per lane");
-    const double s = pair_factor(wave_max(part[b * kParts + threadIdx.x % kWave]));
+    const double s = pair_factor(part, b, threadIdx.x % kWave);
     if (blk == 0 && threadIdx.x == 0) scale[b] = s;
     store4(oref + b * n, i, n, s, r);
     store4(odeg + b * n, i, n, s, d);
@@ -296,6 +288,20 @@ __global__ void __launch_bounds__(kEwThreads)
 
 }  // namespace pesq
 
+namespace pesq {
+
+int launch_pair_peaks(const float *ref, const float *deg, int64_t batch, int64_t len,
+                      float *peaks, hipStream_t stream) {
+    static_assert(kParts == kPairParts, "the partials of peak_partial_kernel");
+    PESQ_CHECK_ARG(batch * kParts < (int64_t(1) << 31), "too many pairs for one launch");
+    hipLaunchKernelGGL(peak_partial_kernel, dim3(static_cast<unsigned>(batch * kParts)),
+                       dim3(kEwThreads), 0, stream, ref, deg, peaks, len);
+    PESQ_CHECK_LAUNCH("pair peaks");
+    return PESQ_OK;
+}
+
+}  // namespace pesq
+
 using namespace pesq;
 
 static int check_rows(int64_t rows, int64_t n) {
@@ -331,9 +337,7 @@ extern "C" int pesq_peak_normalize_forward(const float *ref, const float *deg, i
     if (batch == 0) return PESQ_OK;
     PESQ_CHECK_ARG(ref && deg && out_ref && out_deg && peak && workspace, "null pointer argument");
     float *part = static_cast<float *>(workspace);
-    hipLaunchKernelGGL(peak_partial_kernel, dim3(static_cast<unsigned>(batch * kParts)),
-                       dim3(kEwThreads), 0, stream, ref, deg, part, len);
-    PESQ_CHECK_LAUNCH("peak partial");
+    if (int st = launch_pair_peaks(ref, deg, batch, len, part, stream)) return st;
     int64_t bpr;
     hipLaunchKernelGGL(peak_apply_kernel, dim3(apply_grid(batch, len, bpr)), dim3(kEwThreads), 0,
                        stream, part, ref, deg, out_ref, out_deg, peak, len, bpr);
@@ -370,9 +374,7 @@ extern "C" int pesq_pair_scale_forward(const float *ref, const float *deg, int64
     if (batch == 0) return PESQ_OK;
     PESQ_CHECK_ARG(ref && deg && out_ref && out_deg && scale && workspace, "null pointer argument");
     float *part = static_cast<float *>(workspace);
-    hipLaunchKernelGGL(peak_partial_kernel, dim3(static_cast<unsigned>(batch * kParts)),
-                       dim3(kEwThreads), 0, stream, ref, deg, part, len);
-    PESQ_CHECK_LAUNCH("pair peak");
+    if (int st = launch_pair_peaks(ref, deg, batch, len, part, stream)) return st;
     const int64_t bpr = cdiv(len, kPairSpan);
     hipLaunchKernelGGL(pair_scale_kernel, dim3(static_cast<unsigned>(batch * bpr)),
                        dim3(kEwThreads), 0, stream, part, ref, deg, out_ref, out_deg, scale, len,

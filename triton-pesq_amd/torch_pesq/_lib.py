@@ -143,6 +143,10 @@ SIGNATURES = {
         _INT,
         [_P, _P, _I64, _I64, _P, _P, _INT, _INT, ctypes.c_double, _INT, _P, _P, _P, _P, _P, _P],
     ),
+    "pesq_pipeline_general_forward_scaled": (
+        _INT,
+        [_P, _P, _I64, _I64, _P, _P, _INT, _INT, ctypes.c_double, _INT, _P, _P, _P, _P, _P, _P],
+    ),
     "pesq_pipeline_general_backward": (
         _INT,
         [_P, _P, _P, _P, _I64, _I64, _P, _P, _INT, _INT, ctypes.c_double, _INT, _P, _P, _P, _P, _P],
