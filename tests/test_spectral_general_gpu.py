@@ -388,3 +388,36 @@ def test_general_loss_create_graph_and_double_backward(rate):
     d_symm, _ = model.raw(ref, deg)
     both = torch.autograd.grad(d_symm.sum(), [ref, deg])
     assert torch.equal(g1, both[1]) and torch.equal(g2, both[0])
+
+
+@pytest.mark.parametrize("batch, nsamples", [(700, 6145), (37, 116961)])
+def test_general_loss_of_large_grids_scales_every_pair(batch, nsamples):
+    """Grids whose scans run segments (rows of one and of several): pairs at any
+    scale among the others give what they give alone, by the lane-state scans
+    (float64 either way, rounded to float32 rows: 1e-6 of the gradient's peak)."""
+
+    from torch_pesq import PesqLossTriton
+
+    assert 2 * batch * -(-nsamples // 1024) > 8192
+    model = PesqLossTriton(0.5, sample_rate=16000, hop_length=160).cuda()
+    gen = torch.Generator(device="cuda").manual_seed(nsamples)
+    x = torch.randn(2, batch, nsamples, generator=gen, device="cuda") * 0.05
+    x[1] = x[0] + 0.4 * x[1]
+    power = torch.zeros(batch, device="cuda", dtype=torch.float64)
+    power[1], power[batch // 2], power[-2] = -110.0, 100.0, 30.0
+    y = (x.double() * torch.exp2(power)[:, None]).float()
+
+    def run(z):
+        r, d = z[0].contiguous().requires_grad_(True), z[1].contiguous().requires_grad_(True)
+        loss = model(r, d)
+        return (loss.detach(),) + torch.autograd.grad(loss.sum(), [r, d])
+
+    loss, *grads = run(y)
+    for first in (0, batch // 2, batch - 3):
+        item = slice(first, first + 3)
+        want_loss, *want = run(x[:, item])
+        assert float(((loss[item] - want_loss).abs() / want_loss).max()) < 1e-6
+        for got, w in zip(grads, want):
+            got = got[item].double() * torch.exp2(power[item])[:, None]
+            peak = w.abs().amax(1, keepdim=True)
+            assert float(((got - w).abs() / peak).max()) < 1e-6

@@ -100,7 +100,8 @@ __global__ void __launch_bounds__(kEwThreads)
 //
 // Both signals of each pair times its factor (pair_scale.hpp), for pairs that
 // are resampled before the pipeline at another STFT geometry; of others that
-// pipeline takes the peaks alone and scales its own rows.  Bound by memory latency at the sizes of a batch: 16 pairs of 64000 samples 5.5 us for the
+// pipeline takes the peaks alone and scales its own rows.  Bound by memory
+// latency at the sizes of a batch: 16 pairs of 64000 samples 5.5 us for the
 // peaks, 5.3 for the products, 3.8 for the gradients of both.
 
 // four samples per thread and signal: enough workgroups to hide the latency
