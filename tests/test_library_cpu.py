@@ -490,18 +490,20 @@ def test_pipeline_kernel_variants_per_shape(shape):
     assert _lib.pipeline_kernels(*shape, backward=True) == bwd
 
 
-def test_scans_without_windowed_starts_are_not_segmented(tmp_path):
+@pytest.mark.parametrize("option, holds", [
+    ("PESQ_WINDOW_STARTS 0", "!pesq::PipeFwdMode::kSegments && !pesq::PipeBwdMode::kSegments"),
+    ("PESQ_CHUNK 8", "pesq::kSegmentSpan == 1024"),
+    ("PESQ_CHUNK 32", "pesq::kSegmentSpan == 4096"),
+])
+def test_build_options_of_the_scans(option, holds, tmp_path):
     """Segments take their start states from the two blocks before them alone,
     so a build without windowed block starts (``PESQ_WINDOW_STARTS=0``) has no
     plan for them, and its large grids run the kernels of stored block starts.
-    The host pass over the pipeline, without code generation."""
+    Segments follow another chunk length (``PESQ_CHUNK``).  The host pass over
+    the pipeline, without code generation."""
 
-    src = tmp_path / "plain_starts.hip"
-    src.write_text(
-        "#define PESQ_WINDOW_STARTS 0\n"
-        '#include "pipeline.hip"\n'
-        "static_assert(!pesq::PipeFwdMode::kSegments && !pesq::PipeBwdMode::kSegments);\n"
-    )
+    src = tmp_path / "option.hip"
+    src.write_text(f'#define {option}\n#include "pipeline.hip"\nstatic_assert({holds});\n')
     proc = subprocess.run(
         [os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--cuda-host-only", "-fsyntax-only",
          "-std=c++17", "--offload-arch=gfx950", f"-I{ROOT / 'include'}",

@@ -194,7 +194,7 @@ struct SegmentPlan {
     int count;   // segments per row (0: the scan is not segmented)
     int blocks;  // segment blocks per segment
 };
-constexpr int kSegmentChunk = 32;                               // samples per lane
+constexpr int kSegmentChunk = 2 * kChunk;                       // samples per lane
 constexpr int kSegmentSpan = kWave * kSegmentChunk;             // samples per segment block
 constexpr int kSegmentRatio = kSegmentSpan / kSpan;             // aggregate blocks in it
 static_assert(kSegmentRatio * kSpan == kSegmentSpan, "whole aggregate blocks");
@@ -1086,6 +1086,7 @@ constexpr int kSegmentWaves = 4;             // wavefronts (segments) per workgr
 constexpr int kStageChunk = kSegmentChunk + 4;  // floats between the staged chunks of two lanes
 constexpr int kStageFloats = kWave * kStageChunk;
 constexpr int kCarryPowers = kWave / 2 + 1;  // A^(kSegmentChunk m), m <= 32
+constexpr int kReach = 2 * kSegmentChunk;    // past a lane's chunk and the ramp after it
 template <int NS>
 constexpr int carry_stride() { return 4 * NS + 2; }  // doubles between two powers m
 
@@ -1165,8 +1166,7 @@ __device__ __forceinline__ void chunk_write(float *own, int g, const float (&y)[
         make_float4(y[kRev ? 3 : 0], y[kRev ? 2 : 1], y[kRev ? 1 : 2], y[kRev ? 0 : 3]);
 }
 
-// A^(kSegmentChunk 2^level)
-static_assert(kSegmentChunk == 2 * kChunk, "one level above the aggregate pass's chunks");
+// A^(kSegmentChunk 2^level): one level above the aggregate pass's chunks
 __device__ __forceinline__ ConstDoubles scan_powers(ConstDoubles pw, int level, int k) {
     return pw + ((level + 1) * kMaxSections + k) * 4;
 }
@@ -1174,7 +1174,7 @@ __device__ __forceinline__ ConstDoubles scan_powers(ConstDoubles pw, int level, 
 // One block of a segment: own[q] the lane's staged chunk of buffer q (raw
 // input q, replaced by output q), p the block's start state (in lane 0),
 // replaced by the next block's.  before / after: samples of the row before
-// the lane's chunk and from its first sample to the row's end, at most 64
+// the lane's chunk and from its first sample to the row's end, at most kReach
 // (ramp weights).  kEdge: the block holds samples with a ramp weight, or the
 // row's end.
 template <bool kEdge, int NA, int NB, class Mode>
@@ -1390,9 +1390,9 @@ __device__ __forceinline__ void output_segment(const Mode &m, const IirTable &t,
         float *out2 = second != nullptr ? second + j0 : nullptr;
         // uniform: ramp weights and row ends only in a row's first and last blocks
         if (blk == 0 || int64_t(blk + 1) * kSegmentSpan + kEdge > len) {
-            const int before = static_cast<int>(j0 < kWave ? j0 : kWave);
+            const int before = static_cast<int>(j0 < kReach ? j0 : kReach);
             const int64_t rest = len - j0;
-            const int after = static_cast<int>(rest < 0 ? 0 : (rest < kWave ? rest : kWave));
+            const int after = static_cast<int>(rest < 0 ? 0 : (rest < kReach ? rest : kReach));
             segment_block<true, NA, NB>(m, pw, ca, cb, carry, own, out2, before, after, sh, lane,
                                         p, acc);
         } else {
